@@ -36,6 +36,7 @@
 #include <type_traits>
 
 #include "nq_common.h"
+#include "nq_gemv_rows.h"
 
 // Phase marks of the fast kernels; empty in the library (a timing build may define them).
 #ifndef NQ_STAMP
@@ -1519,9 +1520,9 @@ __global__ __launch_bounds__(256) void s2b_kernel(const S2bArgs a) {
 // rounding slack. Words: row i of the block at i * (kw + 1).
 //
 // Measured (MI355X, graph-replayed, rotating weights; stage 1 alone, us): n = 11008, r = 1632:
-// batch 16 / 64 / 128: 12.9 / 18.7 / 27.7 against 14.3 / 26.6 / 51.3 for s1m_kernel with one row
-// tile per block (19.0 at 64 rows with two); n = 4096: batch 64 / 128: 11.5 / 15.6 against 8.9 / 13.4
-// for s1m_kernel with two and four row tiles, so it runs on wide rows only. A block
+// batch 16 / 64: 12.9 / 18.7 against 14.3 / 26.6 for s1m_kernel with one row tile per block (19.0 at 64
+// rows with two); n = 4096: batch 64: 11.5 against 8.9 for s1m_kernel with two row tiles, so it runs on
+// wide rows only. A block
 // fetches its slice at 35-45 GB/s (phase stamps), so the plan keeps slices small; the same design
 // for stage 2 (slices of h, partial sums of y) lost to s2t_kernel at every batch and is not used.
 struct SbArgs {
@@ -1566,9 +1567,9 @@ __global__ __launch_bounds__(NW * 64) void sb_kernel(const SbArgs a) {
 
     // 1. DMA: the x slice and s_in, and the rows' words (divisions by a multiply: the issue loops
     //    are VALU work before the first MFMA). V's words come from HBM and the x slice mostly from
-    //    L2: up to 64 batch rows the words go out first, so that part of their longer latency
+    //    L2: the words go out first, so that part of their longer latency
     //    passes while the slice is issued (same-box A/B, down_proj and Llama-3-70B q/o at 16-64
-    //    rows: 1.1-1.9% faster); with 128 rows the larger slice goes first (1.6-1.9% faster so).
+    //    rows: 1.1-1.9% faster).
     auto dma_slice = [&]() {
         const uint32_t xchunks = static_cast<uint32_t>(XCOLS * kw4);
         const uint32_t kend = static_cast<uint32_t>(a.wpr) * 32u;  // elements of k
@@ -1600,13 +1601,8 @@ __global__ __launch_bounds__(NW * 64) void sb_kernel(const SbArgs a) {
             dma4(wbase + min(row, rlast) * static_cast<uint32_t>(a.wpr) + q, wl + l0);
         }
     };
-    if constexpr (CT <= 4) {
-        dma_words();
-        dma_slice();
-    } else {
-        dma_slice();
-        dma_words();
-    }
+    dma_words();
+    dma_slice();
     __builtin_amdgcn_s_waitcnt(0);  // this wave's DMAs have landed (vmcnt, expcnt and lgkmcnt all zero)
     __syncthreads();
     NQ_STAMP(1);
@@ -1813,8 +1809,9 @@ struct SbPlan {
 };
 
 // When the batched stage 1 replaces s1m_kernel (measured crossovers, see sb_kernel): on rows of at
-// least 256 words, from a batch that falls with the row width (sb_min_batch); at most 128 rows (8
-// batch tiles), and an LDS slice of at most 160 KB per block. On narrower rows s1m_kernel with two
+// least 256 words, from a batch that falls with the row width (sb_min_batch) up to where the kernels of
+// nq_gemv_rows.hip take over (rows_stage1_plan: fewer than 64 rows, so four batch tiles), with an LDS
+// slice of at most 160 KB per block. On narrower rows s1m_kernel with two
 // or four row tiles per block is the faster one (n = 4096, r = 1632, 64 / 128 rows: 8.9 / 13.4 us
 // against 11.5 / 15.6).
 constexpr int kSbWideWords = 256;
@@ -1839,7 +1836,7 @@ inline int64_t sb_min_batch(int64_t wpr, int64_t rows) {
     if (wpr >= 320) return 8;
     return rows * wpr < 256 * 1024 ? 8 : 16;
 }
-constexpr int kSbMaxBatch = 128;
+constexpr int kSbMaxBatch = 64;
 constexpr int kSbLdsBytes = 160 * 1024;
 constexpr int kSbMaxBlocks = 256;
 // Rounds of blocks the search may take when no plan fits one round (see sb_plan_any).
@@ -1852,10 +1849,9 @@ constexpr int kSbMaxRounds = 4;
 // ranges, the finishing launch (~4000) plus the per-range sums written and read.
 //
 // Where no plan fits one round (the x slice of 16 * ct + 1 columns crowds the rows' words out of
-// LDS: Llama-3-70B down_proj, n = 28672, from 48 batch rows; n = 11008 at r = 2976 at 128 rows), the
-// search is repeated with up to kSbMaxRounds rounds of blocks, each plan's estimate multiplied by its
-// rounds. The alternative, s1m_kernel, streams all of x through every block of 16 rows of V (n =
-// 28672, r = 3520, stage 1 at 48 / 64 / 128 rows: 102.8 / 136.6 / 237.9 us with s1m_kernel).
+// LDS: long rows at a large rank), the search is repeated with up to kSbMaxRounds rounds of blocks, each
+// plan's estimate multiplied by its rounds. The alternative, s1m_kernel, streams all of x through every
+// block of 16 rows of V (n = 28672, r = 3520, stage 1 at 48 rows: 32.6 against 102.8 us).
 inline bool sb_plan_any(int64_t batch, int64_t rows, int64_t wpr, int64_t kpad, SbPlan& p);
 inline bool sb_plan(int64_t batch, int64_t rows, int64_t wpr, int64_t kpad, SbPlan& p) {
     if (batch > kSbMaxBatch || rows <= 0 || wpr <= 0) return false;
@@ -1871,7 +1867,7 @@ inline bool sb_plan(int64_t batch, int64_t rows, int64_t wpr, int64_t kpad, SbPl
 // (other k ranges) was slower (21.58 -> 22.62), and four blocks per CU were no better.
 inline bool sb_plan_rounds(int64_t batch, int64_t rows, int64_t wpr, int64_t kpad, int max_rounds, SbPlan& p) {
     const int64_t occupancy = batch <= 32 ? 2 : 1;  // blocks per CU a round may count
-    const int ct = static_cast<int>(std::min<int64_t>(8, ceil_div(batch, 16)));
+    const int ct = static_cast<int>(std::min<int64_t>(4, ceil_div(batch, 16)));
     const int passes = static_cast<int>(ceil_div(batch, 16LL * ct));
     const int xcols = 16 * ct + 1;
     double best = -1.0;
@@ -2278,11 +2274,7 @@ int launch_sb_rtw(const SbArgs& s, const SbPlan& p, hipStream_t st) {
         case 1: return launch_sb_cfg<T, RTW, 1>(s, p, st);
         case 2: return launch_sb_cfg<T, RTW, 2>(s, p, st);
         case 3: return launch_sb_cfg<T, RTW, 3>(s, p, st);
-        case 4: return launch_sb_cfg<T, RTW, 4>(s, p, st);
-        case 5: return launch_sb_cfg<T, RTW, 5>(s, p, st);
-        case 6: return launch_sb_cfg<T, RTW, 6>(s, p, st);
-        case 7: return launch_sb_cfg<T, RTW, 7>(s, p, st);
-        default: return launch_sb_cfg<T, RTW, 8>(s, p, st);
+        default: return launch_sb_cfg<T, RTW, 4>(s, p, st);
     }
 }
 
@@ -2324,7 +2316,70 @@ int launch_stage1_sb(const GemvArgs& a, const SbPlan& p) {
 }
 
 template <typename T>
+inline int dtype_code();
+template <>
+inline int dtype_code<F16>() { return NQ_F16; }
+template <>
+inline int dtype_code<BF16>() { return NQ_BF16; }
+
+// Stage 1 of many batch rows (nq_gemv_rows.hip), and the sum of its k ranges where it has several.
+template <typename T>
+int launch_stage1_rows(const GemvArgs& a, const RowsPlan& p) {
+    RowsArgs s{};
+    s.words = a.v_bits;
+    s.x = a.x;
+    s.s_in = a.s_in;
+    s.scale = a.s_mid;
+    s.z_hi = a.z_hi;
+    s.z_lo = a.z_lo;
+    s.part = a.part;
+    s.rows = a.r;
+    s.wpr = a.wn;
+    s.batch = a.batch;
+    s.K = a.n;
+    s.kpad = a.plan.kpad;
+    s.zpitch = a.plan.zpitch;
+    launch_rows_stage1(dtype_code<T>(), s, p, a.stream);
+    if (p.splits > 1) {
+        if (int st = check_launch("nq_gemv stage 1")) return st;
+        SbArgs f{};
+        f.s_mid = a.s_mid;
+        f.z_hi = a.z_hi;
+        f.z_lo = a.z_lo;
+        f.part = a.part;
+        f.M = a.r;
+        f.batch = a.batch;
+        f.kpad = a.plan.kpad;
+        f.zpitch = a.plan.zpitch;
+        const int64_t threads = static_cast<int64_t>(a.batch) * a.plan.zpitch / 4;
+        sb_finish1<T><<<dim3(static_cast<unsigned>(ceil_div(threads, 256))), 256, 0, a.stream>>>(f, p.splits);
+    }
+    return NQ_OK;
+}
+
+template <typename T>
+int launch_stage2_rows(const GemvArgs& a, const RowsPlan& p) {
+    RowsArgs s{};
+    s.words = a.u_bits;
+    s.scale = a.s_out;
+    s.z_hi = a.z_hi;
+    s.z_lo = a.z_lo;
+    s.y = a.y;
+    s.rows = a.m;
+    s.wpr = a.plan.wr;
+    s.batch = a.batch;
+    s.K = 64 * p.split_steps;
+    s.kpad = a.plan.kpad;
+    s.zpitch = a.plan.zpitch;
+    launch_rows_stage2(dtype_code<T>(), s, p, a.stream);
+    return NQ_OK;
+}
+
+template <typename T>
 int launch_stage1(const GemvArgs& a) {
+    RowsPlan rp;
+    if (s1w_applies(a.x, a.s_in, a.n, a.wn, a.r) && rows_stage1_plan(a.batch, a.n, a.r, a.plan.kpad, a.part_bytes, rp))
+        return launch_stage1_rows<T>(a, rp);
     SbPlan sp;
     if (sb1_plan(a, sp)) return launch_stage1_sb<T>(a, sp);
     if (s1w_applies(a.x, a.s_in, a.n, a.wn, a.r)) {
@@ -2521,6 +2576,9 @@ int launch_stage2_batched(const GemvArgs& a) {
 
 template <typename T>
 int launch_stage2(const GemvArgs& a) {
+    RowsPlan rp;
+    if (s2t_applies(a.z_hi, a.z_lo, a.u_bits, a.m, a.plan) && rows_stage2_plan(a.batch, a.m, a.plan.wr, rp))
+        return launch_stage2_rows<T>(a, rp);
     if (s2t_applies(a.z_hi, a.z_lo, a.u_bits, a.m, a.plan) && s2b_chosen(a)) return launch_stage2_batched<T>(a);
     if (s2t_applies(a.z_hi, a.z_lo, a.u_bits, a.m, a.plan)) {
         S2Table tab;
@@ -2564,7 +2622,9 @@ inline size_t gemv_part_bytes(int64_t batch, int64_t n, int64_t r, int64_t m) {
     const Plan pl = plan_of(r);
     size_t bytes = 0;
     SbPlan p;
-    if (n % 32 == 0 && r > 0 && sb_plan(batch, r, ceil_div(n, 32), pl.kpad, p)) bytes = p.part_bytes;
+    RowsPlan rp;
+    if (rows_stage1_plan(batch, n, r, pl.kpad, SIZE_MAX, rp)) bytes = rp.part_bytes;
+    else if (n % 32 == 0 && r > 0 && sb_plan(batch, r, ceil_div(n, 32), pl.kpad, p)) bytes = p.part_bytes;
     return (bytes + 255) / 256 * 256;
 }
 

@@ -1,0 +1,110 @@
+"""The decode GEMV of many batch rows (the kernels that share each decoded sign over 64 batch rows):
+edges of its tiles, k ranges and k groups against the float64 oracle (needs a gfx950 GPU)."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+# An fp16 output is rounded by at most 2^-11 of itself; the intermediate (a bf16 pair, 2^-17) and the fp32
+# sums over r and n of at most 2^13 terms stay below 1e-4 of the largest output. A bf16 output's own
+# rounding is counted apart (half a unit in the last place).
+BAR = 2.0 ** -11 + 1e-4
+
+# (m, n, r, rows, s_mid): narrow inputs run from 129 rows (unless one round of the 16-row MFMA kernel
+# does), 256-511 words from 64, 512 words or more from 33
+CASES = [
+    (300, 8192, 70, 64, True),        # the first batch on 256 words; ragged rank and outputs, k ranges
+    (64, 16384, 1, 33, True),         # the first batch on 512 words; a rank of 1
+    (1000, 8200, 130, 65, False),     # n % 64 == 8: the tail tile's first quarter; a second row tile of one row
+    (129, 8248, 257, 100, True),      # n % 64 == 56; outputs that are not whole 16-byte stores
+    (72, 16416, 96, 127, False),      # n % 64 == 32
+    (4096, 11008, 1632, 96, True),    # several k ranges over k groups
+    (520, 4096, 1632, 630, False),    # four k groups, no k range
+    (11008, 4096, 1632, 300, True),   # 128-feature tiles; stage 2 on these kernels too
+    (8200, 512, 4097, 700, False),    # the shortest rows, several tiles a CU; a large ragged rank, a ragged last tile
+    (2048, 1024, 2240, 2048, True),   # 256-feature tiles on every CU, one range
+]
+
+
+def _words(t, method="half2"):
+    import nanoquant_amd as nq
+    return nq.pack_binary_gemv(t, method=method)
+
+
+@pytest.fixture(scope="module")
+def lib():
+    from nanoquant_amd import _lib
+    return _lib.load()
+
+
+def _run(lib, c, dtype, part=True, offset=0):
+    """nq_gemv on a random-byte workspace, with or without room for the k ranges' sums; ``offset``: elements by
+    which the output is moved off its 16-byte alignment."""
+    from nanoquant_amd import _lib
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    x, s_in, s_out = (t(c[k]).to(dtype) for k in ("x", "s_in", "s_out"))
+    s_mid = None if c["s_mid"] is None else t(c["s_mid"]).to(dtype)
+    V, U = _words(t(c["V"])), _words(t(c["U"]))
+    (batch, n), (m, r) = c["x"].shape, c["U"].shape
+    # the intermediate alone: rows of 32 columns never split
+    nbytes = lib.nq_gemv_workspace_bytes(batch, n if part else 32, r, m)
+    ws = torch.randint(0, 256, (nbytes,), dtype=torch.uint8, device="cuda")
+    y = torch.empty(batch * m + 8, dtype=dtype, device="cuda")[offset:offset + batch * m].view(batch, m)
+    _lib.check(lib.nq_gemv(_lib.dtype_code(dtype), x.data_ptr(), s_in.data_ptr(), V.data_ptr(), _lib.ptr(s_mid),
+                           U.data_ptr(), s_out.data_ptr(), y.data_ptr(), batch, n, r, m, ws.data_ptr(), nbytes,
+                           _lib.stream_of(x.device)), "nq_gemv")
+    torch.cuda.synchronize()
+    return y
+
+
+def _oracle(c, dtype):
+    """The fp64 result for the inputs as ``dtype`` holds them."""
+    q = {k: None if c[k] is None else torch.from_numpy(c[k]).to(dtype).double().numpy() for k in ("x", "s_in", "s_mid", "s_out")}
+    return O.nanoquant_forward_f64(q["x"], q["s_in"], c["V"], q["s_mid"], c["U"], q["s_out"])
+
+
+def _error(y, y64, dtype):
+    diff = np.abs(y.double().cpu().numpy() - y64)
+    if dtype == torch.bfloat16:
+        _, e = np.frexp(np.abs(y64))
+        diff = np.maximum(diff - np.ldexp(1.0, e - 9), 0.0)
+    return diff.max() / np.abs(y64).max()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(str(int(v)) for v in c))
+def test_rows_against_oracle(lib, case, dtype):
+    m, n, r, rows, mid = case
+    print("\n[case] gemv rows", case, dtype, flush=True)
+    c = O.random_case(1000 + m + rows, m, n, r, rows, with_mid=mid)
+    y64 = _oracle(c, dtype)
+    y = _run(lib, c, dtype)
+    assert _error(y, y64, dtype) <= BAR
+    assert torch.equal(y, _run(lib, c, dtype)), "a second call over another workspace's bytes"
+
+
+@pytest.mark.parametrize("offset", [1, 4])
+def test_rows_without_range_sums_and_unaligned_output(lib, offset):
+    """No room for the k ranges' sums (one range runs), and outputs off their 16-byte alignment."""
+    m, n, r, rows = 4096, 11008, 1632, 130
+    print("\n[case] gemv rows, smallest workspace", offset, flush=True)
+    assert lib.nq_gemv_workspace_bytes(rows, n, r, m) > lib.nq_gemv_workspace_bytes(rows, 32, r, m)
+    c = O.random_case(77, m, n, r, rows, with_mid=True)
+    assert _error(_run(lib, c, torch.float16, part=False, offset=offset), _oracle(c, torch.float16), torch.float16) <= BAR
+
+
+def test_rows_take_inputs_off_their_alignment(lib):
+    """x 2 bytes off a 16-byte boundary runs the general kernels, not these: the same result to the bar."""
+    import nanoquant_amd  # noqa: F401
+    m, n, r, rows = 300, 8192, 70, 130
+    print("\n[case] gemv rows, unaligned x", flush=True)
+    c = O.random_case(78, m, n, r, rows, with_mid=False)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    x = torch.empty(rows * n + 1, dtype=torch.float16, device="cuda")[1:].view(rows, n)
+    x.copy_(t(c["x"]))
+    y = torch.ops.binary_kernels.nanoquant_dyn_forward(x, t(c["s_in"]).half(), _words(t(c["V"])), None,
+                                                       _words(t(c["U"])), t(c["s_out"]).half(), 128, 128, 2, 2, 1, 1, 8, 8)
+    assert _error(y, _oracle(c, torch.float16), torch.float16) <= BAR
