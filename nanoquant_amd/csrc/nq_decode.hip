@@ -24,6 +24,7 @@
 #include <algorithm>
 
 #include "nq_common.h"
+#include "nq_dense.h"
 
 namespace nq {
 namespace {
@@ -722,6 +723,10 @@ int nq_dense_gemv(int dtype, const void* w, const void* x, const void* norm_weig
     const int mi = static_cast<int>(m), ni = static_cast<int>(n), bi = static_cast<int>(batch);
     const int li = static_cast<int>(ldy);
     hipStream_t st = as_stream(stream);
+    if (dense_mfma_applies(batch, n)) {
+        launch_dense_mfma(dtype, DenseArgs{wp, xp, gp, y, eps, yf, bi, ni, mi, li}, st);
+        return check_launch(name);
+    }
     if (dtype == NQ_F16) {
         if (gp) launch_dense_gemv<F16, true>(wp, xp, gp, eps, y, yf, mi, ni, bi, li, st);
         else launch_dense_gemv<F16, false>(wp, xp, gp, eps, y, yf, mi, ni, bi, li, st);
