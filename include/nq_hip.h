@@ -182,7 +182,9 @@ typedef enum {
     NQ_EPI_GATED = 2     /* two items (gate, up) of equal m and r: y of item 0 = silu(gate) * up */
 } nq_epilogue;
 
-/* Bytes of workspace the two grouped stages need for these items (0 on bad arguments). */
+/* Bytes of workspace the two grouped stages need for these items (0 on bad arguments). A group of one
+ * item lays its workspace out as nq_gemv does, so nq_gemv_stage1 (with nq_gemv_workspace_bytes) may take
+ * the place of nq_gemv_group_stage1 before nq_gemv_group_stage2. */
 size_t nq_gemv_group_workspace_bytes(int64_t count, const nq_gemv_item* items, int64_t batch);
 
 /* Stage 1 of every item over the shared input x [batch, n]. With rms_eps >= 0 the input is

@@ -1334,9 +1334,11 @@ struct S2bArgs {
     uint16_t* y;
     const uint16_t* z_hi;
     const uint16_t* z_lo;
+    const uint16_t* resid;  // kEpiResidual: laid out as y (may be y itself)
     int m, wr, zpitch, batch, chunks;
+    int ystride;      // elements between batch rows of y and resid
     int u_slots;      // LDS dwords of the U tile (its rows' words and the padding, whole DMAs)
-    int store8;       // y takes 8-byte stores of four rows (m % 4 == 0, y 8-byte aligned)
+    int vec4;         // four rows of y (and resid) as one 8-byte access (ystride % 4 == 0, 8-byte aligned)
 };
 
 template <int RT, int WR, int CTW, int KC>
@@ -1352,7 +1354,10 @@ struct S2bShape {
     static_assert(kSlots % 256 == 0, "whole DMAs per thread");
 };
 
-template <typename T, int RT, int WR, int CTW, int KC>
+// EPI: kEpiStore, kEpiResidual (y = resid + T(sat(s_out acc))) or kEpiGated: the second launch of a
+// gated pair, y holding the gate's output (stored by a kEpiStore launch) on entry and silu(gate) * up,
+// rounded as s2t_kernel rounds it, on exit.
+template <typename T, int RT, int WR, int CTW, int KC, int EPI>
 __global__ __launch_bounds__(256) void s2b_kernel(const S2bArgs a) {
     using S = S2bShape<RT, WR, CTW, KC>;
     constexpr int RTW = S::kRTW;
@@ -1484,8 +1489,31 @@ __global__ __launch_bounds__(256) void s2b_kernel(const S2bArgs a) {
                 out[i] = saturate_to<T>((vv[i] + lo) * T::to_float(so[j][i]), T::SAT);
             }
             if ((c & 1) == 0 && b < a.batch) {
-                uint16_t* yp = a.y + static_cast<size_t>(b) * a.m + row;
-                if (a.store8 && row + 3 < a.m) {
+                const size_t at = static_cast<size_t>(b) * a.ystride + row;
+                uint16_t* yp = a.y + at;
+                const bool vec = a.vec4 && row + 3 < a.m;
+                if (EPI == kEpiResidual || EPI == kEpiGated) {
+                    const uint16_t* src = EPI == kEpiResidual ? a.resid + at : yp;
+                    uint16_t in[4] = {0, 0, 0, 0};
+                    if (vec) {
+                        const uint2 v = *reinterpret_cast<const uint2*>(src);
+                        in[0] = static_cast<uint16_t>(v.x);
+                        in[1] = static_cast<uint16_t>(v.x >> 16);
+                        in[2] = static_cast<uint16_t>(v.y);
+                        in[3] = static_cast<uint16_t>(v.y >> 16);
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            if (row + i < a.m) in[i] = src[i];
+                    }
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float o = T::to_float(out[i]), v = T::to_float(in[i]);
+                        out[i] = EPI == kEpiResidual ? T::from_float(v + o)
+                                                     : T::from_float(T::to_float(T::from_float(silu_of<T>(v))) * o);
+                    }
+                }
+                if (vec) {
                     *reinterpret_cast<uint2*>(yp) = uint2{out[0] | (uint32_t(out[1]) << 16), out[2] | (uint32_t(out[3]) << 16)};
                 } else {
 #pragma unroll
@@ -2501,10 +2529,23 @@ bool launch_s2t_qw(S2Table& tab, int qw, int batch, hipStream_t st) {
     }
 }
 
-// One s2b_kernel shape over the op's arguments: grid (row blocks, batch passes); the U tile is
-// the dynamic LDS. Needs s2t_applies (s2_qw > 0 keeps zpitch >= 32 KC * chunks).
-template <typename T, int RT, int WR, int CTW, int KC>
-int launch_s2b_cfg(const GemvArgs& a) {
+// One batched stage 2: what s2b_kernel takes from its caller.
+struct S2bCall {
+    const uint32_t* u_bits;
+    const uint16_t* s_out;
+    uint16_t* y;
+    const uint16_t* resid;
+    const uint16_t* z_hi;
+    const uint16_t* z_lo;
+    int m, ystride, batch;
+    Plan plan;
+    hipStream_t stream;
+};
+
+// One s2b_kernel shape: grid (row blocks, batch passes); the U tile is the dynamic LDS. Needs
+// s2t_applies (s2_qw > 0 keeps zpitch >= 32 KC * chunks).
+template <typename T, int RT, int WR, int CTW, int KC, int EPI>
+int launch_s2b_cfg(const S2bCall& a) {
     using S = S2bShape<RT, WR, CTW, KC>;
     constexpr int kStatic = 3 * 16 * S::kSlots;
     S2bArgs s;
@@ -2513,21 +2554,23 @@ int launch_s2b_cfg(const GemvArgs& a) {
     s.y = a.y;
     s.z_hi = a.z_hi;
     s.z_lo = a.z_lo;
+    s.resid = a.resid;
     s.m = a.m;
     s.wr = a.plan.wr;
     s.zpitch = a.plan.zpitch;
     s.batch = a.batch;
+    s.ystride = a.ystride;
     s.chunks = static_cast<int>(ceil_div(a.plan.wr, KC));
     s.u_slots = static_cast<int>(ceil_div(static_cast<int64_t>(S::kRows) * a.plan.wr + KC, 64) * 64);
-    s.store8 = a.m % 4 == 0 && aligned(a.y, 8);
+    s.vec4 = a.ystride % 4 == 0 && aligned(a.y, 8) && (EPI != kEpiResidual || aligned(a.resid, 8));
     const size_t dyn = static_cast<size_t>(s.u_slots) * 4;
     if (32LL * KC * s.chunks > a.plan.zpitch || kStatic + dyn > static_cast<size_t>(kSbLdsBytes))
         return fail(NQ_ERR_UNSUPPORTED, "nq_gemv batched stage 2: shape does not fit");
-    static const hipError_t attr = allow_lds_bytes(reinterpret_cast<const void*>(&s2b_kernel<T, RT, WR, CTW, KC>),
+    static const hipError_t attr = allow_lds_bytes(reinterpret_cast<const void*>(&s2b_kernel<T, RT, WR, CTW, KC, EPI>),
                                                    kSbLdsBytes - kStatic);
     if (attr != hipSuccess) return fail(NQ_ERR_HIP, "nq_gemv batched stage 2: LDS limit: %s", hipGetErrorString(attr));
     const dim3 grid(static_cast<unsigned>(ceil_div(a.m, S::kRows)), static_cast<unsigned>(ceil_div(a.batch, S::kBatch)));
-    s2b_kernel<T, RT, WR, CTW, KC><<<grid, 256, dyn, a.stream>>>(s);
+    s2b_kernel<T, RT, WR, CTW, KC, EPI><<<grid, 256, dyn, a.stream>>>(s);
     return NQ_OK;
 }
 
@@ -2553,25 +2596,34 @@ constexpr int kS2bMinBatch = 16;
 // r = 3520 at 8 rows 20.6 -> 12.1).
 constexpr int64_t kS2bMinWordsFewRows = int64_t{1} << 21;
 
-inline bool s2b_chosen(const GemvArgs& a) {
-    if (a.batch >= kS2bMinBatch && static_cast<int64_t>(a.m) * a.batch >= kS2bMinWork) return true;
-    return static_cast<int64_t>(a.m) * a.plan.wr >= kS2bMinWordsFewRows &&
-           ceil_div(a.batch, s2t_rows_per_pass(a.batch, a.plan.s2_qw)) >= 2;
+// `items`: the items a block of s2t_kernel would hold: two for a gated pair, whose alternative is two
+// launches of s2b_kernel, the second one applying silu(gate) * up. s2t_kernel then holds half as many batch
+// rows per pass, so the pair changes over earlier (us, s2t against s2b: m = 11008, r = 1632 at 4 / 8 / 12 / 16 /
+// 32 rows 9.2 / 13, 15.1 / 12.9, 21.3 / 13, 25.6 / 12.9, 47.2 / 14.4; m = 4096, r = 1632 at 16 / 24 rows 10.9 /
+// 13, 15.5 / 13; m = 8192, r = 2240 at 8 rows 19.2 / 16; m = 28672, r = 3520 at 2 / 4 / 16 / 64 rows 21.4 / 25,
+// 39.6 / 25.4, 149 / 28.8, 588 / 67).
+constexpr int kS2bPairBatch = 8;
+constexpr int64_t kS2bPairWork = 4400000;
+inline bool s2b_chosen(int batch, int m, const Plan& plan, int items = 1) {
+    if (batch >= kS2bMinBatch && static_cast<int64_t>(m) * batch >= kS2bMinWork) return true;
+    if (items == 2 && batch >= kS2bPairBatch && static_cast<int64_t>(m) * plan.wr * batch >= kS2bPairWork) return true;
+    return static_cast<int64_t>(m) * plan.wr >= kS2bMinWordsFewRows &&
+           ceil_div(batch, s2t_rows_per_pass(batch, items * plan.s2_qw)) >= 2;
 }
 
-template <typename T>
-int launch_stage2_batched(const GemvArgs& a) {
+template <typename T, int EPI>
+int launch_stage2_batched(const S2bCall& a) {
     const int64_t tiles = ceil_div(a.m, 16);
     if (tiles >= 512) {
         // 640-1023 row tiles (the 11008-row gate/up factors) at 16 rows or fewer: 32-row blocks with
         // four-word chunks (same-box, r = 1632 / 2976: 14.52 / 18.67 -> 13.93 / 17.42 us per GEMV; at
         // 1792 tiles, Llama-3-70B gate/up, they lose 12-25%, at 512 they tie, at 24 rows they lose)
-        if (tiles >= 640 && tiles < 1024 && a.batch <= 16) return launch_s2b_cfg<T, 2, 2, 1, 4>(a);
-        if (a.batch <= 64) return launch_s2b_cfg<T, 4, 4, 2, 2>(a);
-        return launch_s2b_cfg<T, 4, 4, 4, 2>(a);
+        if (tiles >= 640 && tiles < 1024 && a.batch <= 16) return launch_s2b_cfg<T, 2, 2, 1, 4, EPI>(a);
+        if (a.batch <= 64) return launch_s2b_cfg<T, 4, 4, 2, 2, EPI>(a);
+        return launch_s2b_cfg<T, 4, 4, 4, 2, EPI>(a);
     }
-    if (a.batch <= 64) return launch_s2b_cfg<T, 2, 2, 1, 4>(a);
-    return launch_s2b_cfg<T, 2, 2, 2, 2>(a);
+    if (a.batch <= 64) return launch_s2b_cfg<T, 2, 2, 1, 4, EPI>(a);
+    return launch_s2b_cfg<T, 2, 2, 2, 2, EPI>(a);
 }
 
 template <typename T>
@@ -2579,7 +2631,9 @@ int launch_stage2(const GemvArgs& a) {
     RowsPlan rp;
     if (s2t_applies(a.z_hi, a.z_lo, a.u_bits, a.m, a.plan) && rows_stage2_plan(a.batch, a.m, a.plan.wr, rp))
         return launch_stage2_rows<T>(a, rp);
-    if (s2t_applies(a.z_hi, a.z_lo, a.u_bits, a.m, a.plan) && s2b_chosen(a)) return launch_stage2_batched<T>(a);
+    if (s2t_applies(a.z_hi, a.z_lo, a.u_bits, a.m, a.plan) && s2b_chosen(a.batch, a.m, a.plan))
+        return launch_stage2_batched<T, kEpiStore>(S2bCall{a.u_bits, a.s_out, a.y, nullptr, a.z_hi, a.z_lo, a.m, a.m,
+                                                           a.batch, a.plan, a.stream});
     if (s2t_applies(a.z_hi, a.z_lo, a.u_bits, a.m, a.plan)) {
         S2Table tab;
         tab.count = 1;
@@ -3014,6 +3068,14 @@ int nq_gemv_group_stage2_kv(int dtype, const nq_gemv_item* items, int64_t batch,
 namespace nq {
 namespace {
 
+// Item k of a group on the batched stage 2.
+template <typename T>
+int group_batched(const S2bCall& c, int epilogue, int64_t k) {
+    if (epilogue == NQ_EPI_RESIDUAL) return launch_stage2_batched<T, kEpiResidual>(c);
+    if (epilogue == NQ_EPI_GATED && k == 1) return launch_stage2_batched<T, kEpiGated>(c);
+    return launch_stage2_batched<T, kEpiStore>(c);
+}
+
 int group_stage2(const char* name, int dtype, int64_t count, const nq_gemv_item* items, int64_t batch, int epilogue,
                  const RopeArgs* rope, void* workspace, size_t workspace_bytes, nq_stream_t stream) {
     GroupLayout g;
@@ -3054,10 +3116,26 @@ int group_stage2(const char* name, int dtype, int64_t count, const nq_gemv_item*
         it.rope = rope == nullptr ? 0 : rope->kind[k];
         it.cache = rope == nullptr ? nullptr : (it.rope == 2 ? rope->k_cache : it.rope == 3 ? rope->v_cache : nullptr);
     }
-    // one launch per class of items that share the stage-2 word split (equal ranks always do)
     const int b = static_cast<int>(batch);
     hipStream_t st = as_stream(stream);
     bool done[kMaxItems] = {false, false, false, false};
+    if (rope == nullptr) {  // items whose batch the batched kernel serves better: a launch each
+        const int pair = epilogue == NQ_EPI_GATED ? 2 : 1;
+        for (int64_t k = 0; k < count; ++k) {
+            if (!s2b_chosen(b, all[k].m, g.plan[k], pair)) continue;
+            S2bCall c{all[k].u_bits, all[k].s_out, all[k].y, all[k].resid, all[k].z_hi, all[k].z_lo, all[k].m,
+                      all[k].ystride, b, g.plan[k], st};
+            if (pair == 2) {  // the gate into y of item 0, then up against it
+                c.y = all[0].y;
+                c.ystride = all[0].ystride;
+            }
+            const int s = dtype == NQ_F16 ? group_batched<F16>(c, epilogue, k) : group_batched<BF16>(c, epilogue, k);
+            if (s) return s;
+            if (int e = check_launch(name)) return e;
+            done[k] = true;
+        }
+    }
+    // one launch per class of items that share the stage-2 word split (equal ranks always do)
     for (int64_t k0 = 0; k0 < count; ++k0) {
         if (done[k0]) continue;
         const int qw = g.plan[k0].s2_qw;

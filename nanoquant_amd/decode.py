@@ -600,8 +600,10 @@ class FusedDecoder(GraphDecoder):
         self.plans = [self._layer_plan(layer) for layer in model.model.layers]
         need = 0
         for plan in self.plans:
-            for items, count in (plan["qkv"], plan["o"], plan["gu"], plan["down"]):
+            for items, count in (plan["qkv"], plan["gu"]):
                 need = max(need, self.lib.nq_gemv_group_workspace_bytes(count, items, batch))
+            for items, n in ((plan["o"][0], H * D), (plan["down"][0], s.ffn)):  # with the k ranges' sums
+                need = max(need, self.lib.nq_gemv_workspace_bytes(batch, n, items[0].r, items[0].m))
         self.ws = torch.zeros(max(need, 256), dtype=torch.uint8, device=dev)
         self.attn_ws = None
         if attention == "hip":  # the partial results of the 64-position chunks
@@ -669,6 +671,16 @@ class FusedDecoder(GraphDecoder):
     def _check(self, status, what):
         self._lib.check(status, what)
 
+    def _linear_residual(self, plan, x, n, stream, what):
+        """One linear and its residual. It has no norm to fold in, so its stage 1 is the plain GEMV's, which at
+        several batch rows splits wide inputs over the grid (a one-item group has the GEMV's workspace)."""
+        items, count = plan
+        it, B, ws, wsb = items[0], self.batch, self.ws.data_ptr(), self.ws.numel()
+        self._check(self.lib.nq_gemv_stage1(self.dcode, x, it.s_in, it.v_bits, it.s_mid, B, n, it.r, it.m, ws, wsb,
+                                            stream), what + " 1")
+        self._check(self.lib.nq_gemv_group_stage2(self.dcode, count, items, B, self._lib.NQ_EPI_RESIDUAL, ws, wsb,
+                                                  stream), what + " 2")
+
     def _step(self):
         lib, s, B = self.lib, self.model.shape, self.batch
         H, KV, D = s.heads, s.kv_heads, s.head_dim
@@ -719,16 +731,11 @@ class FusedDecoder(GraphDecoder):
                                                 scores=self.scores_all[li])
                 if out.data_ptr() != self.attn.data_ptr():
                     self.attn.copy_(out.view(B, H * D))
-            items, n = plan["o"]
-            self._check(lib.nq_gemv_group_stage1(dt, n, items, attn, B, H * D, -1.0, ws, wsb, st), "o 1")
-            self._check(lib.nq_gemv_group_stage2(dt, n, items, B, self._lib.NQ_EPI_RESIDUAL, ws, wsb, st), "o 2")
+            self._linear_residual(plan["o"], attn, H * D, st, "o")
             items, n = plan["gu"]
             self._check(lib.nq_gemv_group_stage1(dt, n, items, h, B, s.hidden, plan["eps2"], ws, wsb, st), "gu 1")
             self._check(lib.nq_gemv_group_stage2(dt, n, items, B, self._lib.NQ_EPI_GATED, ws, wsb, st), "gu 2")
-            items, n = plan["down"]
-            self._check(lib.nq_gemv_group_stage1(dt, n, items, act, B, s.ffn, -1.0, ws, wsb, st), "down 1")
-            self._check(lib.nq_gemv_group_stage2(dt, n, items, B, self._lib.NQ_EPI_RESIDUAL, ws, wsb, st),
-                        "down 2")
+            self._linear_residual(plan["down"], act, s.ffn, st, "down")
         # the final RMS norm folded into the lm_head launch; float32 logits straight from it (with a
         # bias, the dtype logits, the bias added in dtype, then widened, as the torch head rounds)
         norm = self.model.model.norm
