@@ -299,6 +299,25 @@ int nq_attention_decode(int dtype, const void* q, const void* k, const void* v, 
                         int64_t head_dim, int64_t max_len, float scaling, void* workspace, size_t workspace_bytes,
                         nq_stream_t stream);
 
+/* Attention of a prompt's tokens on a static KV cache, with the rotary embedding and the cache write:
+ *   q, k, v   [batch, tokens] rows of q_stride / k_stride / v_stride elements (multiples of 8); q holds
+ *             heads heads, k and v kv_heads heads, each head_dim wide
+ *   k_cache, v_cache  [batch, kv_heads, max_len, head_dim]; the cache row positions[t] receives token t's
+ *             rotated key and its value
+ *   rope_cos, rope_sin  [tokens, head_dim], row t for token t (the rotate-half convention)
+ *   positions device int64 [tokens], any order (a prompt, or a chunk after a cached context), the same for
+ *             every sequence; a position outside [0, max_len) writes no cache row
+ *   out       [batch, tokens, heads * head_dim]: softmax(q k^T * scaling) v over the cache rows
+ *             0 .. positions[t]
+ * Query head h uses kv head h / (heads / kv_heads). Rotary products and sum rounded to dtype as the torch path
+ * rounds them, scores and softmax in fp32, probabilities rounded to dtype for the value product, which sums
+ * in fp32. Two launches; every tensor 16-byte aligned; head_dim 128, NQ_ERR_UNSUPPORTED otherwise. No
+ * counterpart in the reference, whose prefill runs Hugging Face's attention (kernel/test_decode.py:385-402). */
+int nq_attention_prefill(int dtype, const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
+                         int64_t v_stride, void* k_cache, void* v_cache, const void* rope_cos, const void* rope_sin,
+                         const int64_t* positions, void* out, int64_t batch, int64_t tokens, int64_t heads,
+                         int64_t kv_heads, int64_t head_dim, int64_t max_len, float scaling, nq_stream_t stream);
+
 /* Rotary embedding and KV-cache write of one new token per sequence, with the attention products
  * left to the caller: the first part of nq_attention_decode on its own. qkv [batch, qkv_stride]
  * holds heads query heads, kv_heads key heads and kv_heads value heads of head_dim (even) each;

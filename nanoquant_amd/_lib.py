@@ -76,6 +76,8 @@ SIGNATURES = {
     "nq_attention_decode_workspace_bytes": (_size, [_i64, _i64, _i64, _i64, _i64]),
     "nq_attention_decode": (_int, [_int, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64,
                                    _i64, ctypes.c_float, _vp, _size, _vp]),
+    "nq_attention_prefill": (_int, [_int, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64,
+                                    _i64, _i64, _i64, _i64, ctypes.c_float, _vp]),
     "nq_rope_kv_write": (_int, [_int, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64,
                                  _vp]),
     "nq_dense_gemv": (_int, [_int, _vp, _vp, _vp, ctypes.c_float, _vp, _int, _i64, _i64, _i64, _i64, _vp]),

@@ -28,6 +28,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import _lib
 from .modules.linear import NanoQuantLinear
 
 LINEAR_NAMES = ("q_proj", "k_proj", "v_proj", "o_proj", "gate_proj", "up_proj", "down_proj")
@@ -137,14 +138,63 @@ class StaticKVCache:
         self.key_index = torch.arange(max_len, device=device)
 
 
+def _only_eager(*tensors) -> bool:
+    """Whether a kernel may take the tensors' memory: nothing traces, transforms or differentiates them."""
+    if not all(type(t) in (torch.Tensor, nn.Parameter) for t in tensors) or torch.compiler.is_compiling():
+        return False
+    if torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0:
+        return False
+    if torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0:
+        return False
+    return not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
+
+
+def _prefill_kernel_takes(shape: LlamaShape, q, k, v, cos, sin, positions, k_c, v_c, key_index) -> bool:
+    """Whether ``nq_attention_prefill`` covers this call of ``rotary_attention``; any other (CPU or float32
+    tensors, other head sizes, strides or alignments, autograd, tracing) runs the torch ops."""
+    H, KV, D = shape.heads, shape.kv_heads, shape.head_dim
+    half = (q, k, v, cos, sin, k_c, v_c)
+    if not q.is_cuda or q.dtype not in (torch.float16, torch.bfloat16) or D != 128 or H % KV or q.dim() != 3:
+        return False
+    if not _only_eager(*half, positions):  # before anything asks for an address
+        return False
+    B, T = q.shape[:2]
+    L = k_c.shape[2] if k_c.dim() == 4 else 0
+    if not (T > 1 and B > 0 and L <= 1 << 22 and tuple(q.shape) == (B, T, H * D) and tuple(k.shape) == tuple(v.shape) == (B, T, KV * D)
+            and tuple(cos.shape) == tuple(sin.shape) == (T, D) and tuple(k_c.shape) == tuple(v_c.shape) == (B, KV, L, D)
+            and tuple(positions.shape) == (T,) and positions.dtype == torch.int64 and positions.is_contiguous()
+            and tuple(key_index.shape) == (L,)):
+        return False
+    if not all(t.dtype == q.dtype and t.device == q.device and t.data_ptr() % 16 == 0 for t in half):
+        return False
+    if not all(t.is_contiguous() for t in (cos, sin, k_c, v_c)) or positions.device != q.device:
+        return False
+    return all(t.stride(2) == 1 and t.stride(1) % 8 == 0 and t.stride(1) >= t.shape[2]
+               and (B == 1 or t.stride(0) == T * t.stride(1)) for t in (q, k, v))
+
+
 def rotary_attention(shape: LlamaShape, layer: int, q, k, v, cos, sin, positions, cache: StaticKVCache):
-    """Rotary embedding, KV-cache write at ``positions`` and causal attention over the cache, in
-    torch ops (Hugging Face's Llama attention on a static cache).
+    """Rotary embedding, KV-cache write at ``positions`` and causal attention over the cache
+    (Hugging Face's Llama attention on a static cache).
 
     q [B, T, H*D], k and v [B, T, KV*D] (strided views are fine), cos and sin [T, D];
-    returns [B, T, H*D] in the cache dtype.
+    returns [B, T, H*D] in the cache dtype. Several float16 or bfloat16 tokens on the GPU run
+    ``nq_attention_prefill``, anything else torch ops: the scores of a prompt, which the torch
+    path writes and reads in float32 several times over, then never reach memory.
     """
     H, KV, D = shape.heads, shape.kv_heads, shape.head_dim
+    if _prefill_kernel_takes(shape, q, k, v, cos, sin, positions, cache.k[layer], cache.v[layer], cache.key_index):
+        # torch's own range check of the positions, on the device as index_copy_ makes it
+        torch.empty_like(cache.key_index).index_copy_(0, positions, positions)
+        out = torch.empty_like(q, memory_format=torch.contiguous_format)
+        lib = _lib.load()
+        with torch.cuda.device(q.device):
+            _lib.check(lib.nq_attention_prefill(
+                _lib.dtype_code(q.dtype), q.data_ptr(), q.stride(1), k.data_ptr(), k.stride(1), v.data_ptr(), v.stride(1),
+                cache.k[layer].data_ptr(), cache.v[layer].data_ptr(), cos.data_ptr(), sin.data_ptr(),
+                positions.data_ptr(), out.data_ptr(), q.shape[0], q.shape[1], H, KV, D, cache.k[layer].shape[2],
+                D ** -0.5, _lib.stream_of(q.device)), "rotary_attention")
+        return out
     B, T = q.shape[0], q.shape[1]
     G = H // KV
     q = q.reshape(B, T, H, D).transpose(1, 2)
@@ -532,8 +582,6 @@ class FusedDecoder(GraphDecoder):
     def __init__(self, model: NanoQuantLlama, batch: int, max_len: int, steps_per_graph: int = 1,
                  device="cuda", attention: str = "torch"):
         super().__init__(model, batch, max_len, steps_per_graph, device)
-        from . import _lib
-
         if attention not in ("torch", "rope", "hip"):
             raise ValueError(f"attention must be 'torch', 'rope' or 'hip', got {attention!r}")
         self.attention = attention

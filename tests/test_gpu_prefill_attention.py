@@ -1,0 +1,138 @@
+"""Attention of a prompt on the KV cache (``nq_attention_prefill`` through ``rotary_attention``) against the torch
+ops it replaces and float64 (needs a gfx950 GPU)."""
+import math
+
+import pytest
+import torch
+
+import nanoquant_amd.decode as decode
+from nanoquant_amd.decode import LlamaShape, StaticKVCache, rotary_attention
+
+pytestmark = pytest.mark.gpu
+
+# (heads, kv_heads, batch, tokens, past): fewer rows than a wave's, one row past a block, one key past a tile,
+# groups that do not divide a block, a chunk after a context, several blocks a head
+CASES = [(4, 4, 1, 2, 0), (4, 4, 2, 33, 0), (8, 2, 2, 64, 1), (8, 1, 1, 129, 63), (6, 2, 3, 65, 64), (5, 1, 1, 300, 0),
+         (2, 2, 1, 129, 511), (16, 2, 1, 700, 200)]
+
+
+def _inputs(case, dtype, gap=37):
+    heads, kv, batch, tokens, past = case
+    gen = torch.Generator(device="cuda").manual_seed(tokens + past)
+    draw = lambda *s: torch.randn(*s, device="cuda", generator=gen).to(dtype)  # noqa: E731
+    shape = LlamaShape(hidden=heads * 128, layers=1, heads=heads, kv_heads=kv, ffn=256, vocab=64)
+    cache = StaticKVCache(shape, batch, past + tokens + gap, "cuda", dtype)
+    cache.k[0][:, :, :past].copy_(draw(batch, kv, past, 128))
+    cache.v[0][:, :, :past].copy_(draw(batch, kv, past, 128))
+    q, k, v = draw(batch, tokens, heads * 128), draw(batch, tokens, kv * 128), draw(batch, tokens, kv * 128)
+    positions = torch.arange(past, past + tokens, device="cuda")
+    inv = 1.0 / (10000.0 ** (torch.arange(0, 128, 2, device="cuda").float() / 128))
+    angle = torch.cat((positions.float().view(-1, 1) * inv,) * 2, -1)
+    return shape, q, k, v, angle.cos().to(dtype), angle.sin().to(dtype), positions, cache
+
+
+def _exact(shape, q, k, v, cos, sin, positions, cache):
+    rot = lambda t: torch.cat((-t[..., 64:], t[..., :64]), -1)  # noqa: E731
+    split = lambda t: t.reshape(*t.shape[:2], -1, 128).transpose(1, 2).double()  # noqa: E731
+    Q, K = (split(t) * cos.double() + rot(split(t)) * sin.double() for t in (q, k))
+    kc, vc = cache.k[0].double(), cache.v[0].double()
+    kc[:, :, positions], vc[:, :, positions] = K, split(v)
+    hidden = torch.arange(kc.shape[2], device="cuda") > positions.view(-1, 1)
+    group = shape.heads // shape.kv_heads
+    s = Q.cpu() @ kc.repeat_interleave(group, 1).transpose(2, 3).contiguous().cpu() * 128 ** -0.5
+    p = torch.softmax(s.masked_fill(hidden.cpu(), -math.inf), -1)
+    return (p @ vc.repeat_interleave(group, 1).cpu()).transpose(1, 2).reshape(q.shape).cuda()
+
+
+def _error(y, ref):
+    return ((y.double() - ref).norm() / ref.norm()).item()
+
+
+@pytest.fixture
+def torch_ops(monkeypatch):
+    def run(*args):
+        with monkeypatch.context() as m:
+            m.setattr(decode, "_prefill_kernel_takes", lambda *a: False)
+            return rotary_attention(*args)
+    return run
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c)))
+def test_prefill_attention(case, dtype, torch_ops):
+    """The cache rows equal the torch path's bit for bit (the same roundings). The output rounds once less (its
+    scores stay in float32), so its error against float64 is at most the torch path's, but for chance on few
+    values: 1.1 times."""
+    print("\n[case] prefill attention", case, dtype, flush=True)
+    shape, q, k, v, cos, sin, pos, cache = args = _inputs(case, dtype)
+    ref = _exact(*args)
+    before = cache.k[0].clone(), cache.v[0].clone()
+    assert decode._prefill_kernel_takes(shape, q, k, v, cos, sin, pos, cache.k[0], cache.v[0], cache.key_index)
+    y = rotary_attention(shape, 0, q, k, v, cos, sin, pos, cache)
+    after = cache.k[0].clone(), cache.v[0].clone()
+    cache.k[0].copy_(before[0])
+    cache.v[0].copy_(before[1])
+    want = torch_ops(shape, 0, q, k, v, cos, sin, pos, cache)
+    assert torch.equal(cache.k[0], after[0]) and torch.equal(cache.v[0], after[1])
+    assert y.shape == want.shape and y.dtype == want.dtype and y.is_contiguous()
+    assert _error(y, ref) <= 1.1 * _error(want, ref)
+
+
+def test_prefill_attention_forms(torch_ops):
+    """Forms the kernel takes beside a plain prompt: q, k and v as slices of one projection output, positions in any
+    order, rows of the cache past the last position holding NaN."""
+    shape, q, k, v, cos, sin, pos, cache = _inputs((8, 2, 1, 96, 20), torch.float16)
+    qkv = torch.cat((q, k, v), -1)
+    parts = qkv[..., :1024], qkv[..., 1024:1280], qkv[..., 1280:]
+    order = torch.randperm(96, generator=torch.Generator().manual_seed(3)).cuda()
+    args = (*(p[:, order] for p in (q, k, v)), cos[order], sin[order], pos[order])
+    assert decode._prefill_kernel_takes(shape, *parts, cos, sin, pos, cache.k[0], cache.v[0], cache.key_index)
+    y = rotary_attention(shape, 0, q, k, v, cos, sin, pos, cache)
+    assert torch.equal(rotary_attention(shape, 0, *parts, cos, sin, pos, cache), y)
+    # a row's sums depend on its block's tiles and mask only through its own keys
+    assert torch.equal(rotary_attention(shape, 0, *args, cache), y[:, order])
+    cache.k[0][:, :, 116:] = float("nan")
+    cache.v[0][:, :, 116:] = float("nan")
+    assert torch.equal(rotary_attention(shape, 0, q, k, v, cos, sin, pos, cache), y)
+
+
+def test_prefill_attention_leaves_other_calls_to_torch(torch_ops):
+    """Calls the kernel does not cover keep the torch ops: gradients, other strides and types, one token, a trace."""
+    shape, q, k, v, cos, sin, pos, cache = _inputs((4, 4, 1, 40, 0), torch.float16)
+    takes = lambda *a: decode._prefill_kernel_takes(shape, *a)  # noqa: E731
+    tail = (cos, sin, pos, cache.k[0], cache.v[0], cache.key_index)
+    assert takes(q, k, v, *tail)
+    g = q.clone().requires_grad_()
+    assert not takes(g, k, v, *tail)
+    with torch.no_grad():
+        assert takes(g, k, v, *tail)
+    y = rotary_attention(shape, 0, g, k, v, cos, sin, pos, cache)
+    assert y.requires_grad and torch.equal(y, torch_ops(shape, 0, q, k, v, cos, sin, pos, cache))
+    assert not takes(q.float(), k.float(), v.float(), cos.float(), sin.float(), *tail[2:])
+    assert not takes(q[:, :1], k[:, :1], v[:, :1], cos[:1], sin[:1], pos[:1], *tail[3:])
+    assert not takes(q.transpose(1, 2).contiguous().transpose(1, 2), k, v, *tail)
+    assert not takes(torch.empty(q.numel() + 4, dtype=q.dtype, device="cuda")[4:].view_as(q), k, v, *tail)
+    assert not takes(q, k, v, cos, sin, pos.int(), *tail[3:])
+    seen = []
+    torch.func.vmap(lambda a: seen.append(takes(a, k, v, *tail)) or a)(q[None])
+    with torch.autograd.forward_ad.dual_level():
+        seen.append(takes(q, k, v, *tail))
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode(allow_non_fake_inputs=True):
+        seen.append(takes(q, k, v, *tail))
+    assert seen == [False, False, False]
+
+
+def test_prefill_attention_argument_errors():
+    from nanoquant_amd import _lib
+    lib = _lib.load()
+
+    def call(heads=4, kv=2, dim=128, stride=512, p=16):
+        return lib.nq_attention_prefill(_lib.NQ_F16, p, stride, 16, 256, 16, 256, 16, 16, 16, 16, 16, 16, 1, 8, heads, kv,
+                                        dim, 64, 0.1, None)
+
+    assert call(dim=64) == _lib.NQ_ERR_UNSUPPORTED
+    assert call(heads=3) == _lib.NQ_ERR_UNSUPPORTED
+    assert call(stride=504) == _lib.NQ_ERR_SHAPE
+    assert call(p=None) == _lib.NQ_ERR_INVALID_ARGUMENT
+    assert call(p=24) == _lib.NQ_ERR_ALIGNMENT
