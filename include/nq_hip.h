@@ -333,6 +333,20 @@ int nq_rope_kv_write(int dtype, const void* qkv, int64_t qkv_stride, void* k_cac
                      int64_t q_stride, int64_t batch, int64_t heads, int64_t kv_heads, int64_t head_dim,
                      int64_t max_len, nq_stream_t stream);
 
+/* ---------------------------------------------------------------- norm and activation of many tokens */
+
+/* y[i] = dtype(weight * dtype(x[i] * rsqrt(mean(x[i]^2) + eps))) for each of `rows` contiguous rows of n
+ * elements (mean and product in fp32): a Llama decoder's RMSNorm in one launch. n a multiple of 8, at most
+ * 16384; x, weight and y 16-byte aligned, y may be x. No counterpart in the reference, which runs Hugging
+ * Face's LlamaRMSNorm (kernel/test_decode.py:385-402). */
+int nq_rms_norm(int dtype, const void* x, const void* weight, void* y, int64_t rows, int64_t n, float eps,
+                nq_stream_t stream);
+
+/* y = dtype(dtype(silu(gate)) * up) over `count` elements (silu in fp32): the activation of a gated MLP in one
+ * launch. count a multiple of 8; 16-byte aligned; y may be gate or up. No counterpart in the reference, which
+ * runs Hugging Face's LlamaMLP (kernel/test_decode.py:385-402). */
+int nq_silu_mul(int dtype, const void* gate, const void* up, void* y, int64_t count, nq_stream_t stream);
+
 /* ---------------------------------------------------------------- dense GEMV */
 
 /* y[b, j] = dtype(sum_k w[j, k] xn[b, k]) for b < batch, j < m: a dense linear of a few rows, the

@@ -80,6 +80,8 @@ SIGNATURES = {
                                     _i64, _i64, _i64, _i64, ctypes.c_float, _vp]),
     "nq_rope_kv_write": (_int, [_int, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64,
                                  _vp]),
+    "nq_rms_norm": (_int, [_int, _vp, _vp, _vp, _i64, _i64, ctypes.c_float, _vp]),
+    "nq_silu_mul": (_int, [_int, _vp, _vp, _vp, _i64, _vp]),
     "nq_dense_gemv": (_int, [_int, _vp, _vp, _vp, ctypes.c_float, _vp, _int, _i64, _i64, _i64, _i64, _vp]),
     "nq_argmax_rows": (_int, [_vp, _i64, _i64, _i64, _vp, _vp]),
     "nq_gemm_onebit_workspace_bytes": (_size, [_i64, _i64, _i64]),

@@ -102,6 +102,36 @@ def random_nanoquant_linear(in_features: int, out_features: int, rank: int, gene
     return lin
 
 
+def _only_eager(*tensors) -> bool:
+    """Whether a kernel may take the tensors' memory: nothing traces, transforms or differentiates them."""
+    if not all(type(t) in (torch.Tensor, nn.Parameter) for t in tensors) or torch.compiler.is_compiling():
+        return False
+    if torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0:
+        return False
+    if torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0:
+        return False
+    return not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
+
+
+def _pointwise_kernel_takes(x, other) -> bool:
+    """Whether a row-wise HIP kernel may run on x and a second operand of its last dimension or shape."""
+    return (x.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and other.dtype == x.dtype
+            and other.device == x.device and x.numel() > 0 and x.shape[-1] % 8 == 0 and x.is_contiguous()
+            and other.is_contiguous() and _only_eager(x, other) and x.data_ptr() % 16 == 0 and other.data_ptr() % 16 == 0)
+
+
+def silu_mul(gate, up):
+    """silu(gate) * up, rounded after the silu and after the product: one launch of the HIP library for
+    contiguous float16 or bfloat16 tensors on the GPU, torch ops otherwise."""
+    if gate.shape == up.shape and gate.dim() > 0 and _pointwise_kernel_takes(gate, up):
+        y = torch.empty_like(gate)
+        with torch.cuda.device(gate.device):
+            _lib.check(_lib.load().nq_silu_mul(_lib.dtype_code(gate.dtype), gate.data_ptr(), up.data_ptr(), y.data_ptr(),
+                                               gate.numel(), _lib.stream_of(gate.device)), "silu_mul")
+        return y
+    return F.silu(gate) * up
+
+
 class RMSNorm(nn.Module):
     """Hugging Face LlamaRMSNorm: normalise in fp32, cast back, then scale."""
 
@@ -111,8 +141,16 @@ class RMSNorm(nn.Module):
         self.eps = eps
 
     def forward(self, x):
-        # x * rsqrt(mean(x^2) + eps) in fp32 (torch's fused RMS norm: one launch instead of five on
-        # the GPU, the same values), cast back, then the weight
+        # x * rsqrt(mean(x^2) + eps) in fp32, cast back, then the weight: one launch for contiguous
+        # float16 or bfloat16 rows on the GPU
+        w = self.weight
+        if x.dim() > 0 and w.dim() == 1 and w.shape[0] == x.shape[-1] <= self.MAX_KERNEL_DIM and _pointwise_kernel_takes(x, w):
+            y = torch.empty_like(x)
+            with torch.cuda.device(x.device):
+                _lib.check(_lib.load().nq_rms_norm(_lib.dtype_code(x.dtype), x.data_ptr(), w.data_ptr(), y.data_ptr(),
+                                                   x.numel() // w.shape[0], w.shape[0], self.eps,
+                                                   _lib.stream_of(x.device)), "RMSNorm")
+            return y
         xf = F.rms_norm(x.float(), (x.shape[-1],), eps=self.eps)
         return self.weight * xf.to(x.dtype)
 
@@ -136,17 +174,6 @@ class StaticKVCache:
         self.k = [torch.zeros(batch, kv, max_len, d, device=device, dtype=dtype) for _ in range(shape.layers)]
         self.v = [torch.zeros(batch, kv, max_len, d, device=device, dtype=dtype) for _ in range(shape.layers)]
         self.key_index = torch.arange(max_len, device=device)
-
-
-def _only_eager(*tensors) -> bool:
-    """Whether a kernel may take the tensors' memory: nothing traces, transforms or differentiates them."""
-    if not all(type(t) in (torch.Tensor, nn.Parameter) for t in tensors) or torch.compiler.is_compiling():
-        return False
-    if torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0:
-        return False
-    if torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0:
-        return False
-    return not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
 
 
 def _prefill_kernel_takes(shape: LlamaShape, q, k, v, cos, sin, positions, k_c, v_c, key_index) -> bool:
@@ -355,7 +382,7 @@ class LlamaAttention(nn.Module):
 
 class LlamaMLP(nn.Module):
     def forward(self, x):
-        return self.down_proj(F.silu(self.gate_proj(x)) * self.up_proj(x))
+        return self.down_proj(silu_mul(self.gate_proj(x), self.up_proj(x)))
 
 
 class LlamaDecoderLayer(nn.Module):

@@ -1,0 +1,67 @@
+"""The RMS norm and silu(gate) * up launches of a decoder layer against the torch ops they replace (needs a gfx950
+GPU)."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+import nanoquant_amd.decode as decode
+from nanoquant_amd.decode import RMSNorm, silu_mul
+
+pytestmark = pytest.mark.gpu
+DTYPES = pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+
+
+def _ulps(a, b, dtype):
+    """The largest difference in units in the last place of the larger value's binade."""
+    a, b = a.double(), b.double()
+    bits = 10 if dtype == torch.float16 else 7
+    unit = torch.exp2(torch.floor(torch.log2(torch.maximum(a.abs(), b.abs()).clamp_min(2.0 ** -14))) - bits)
+    return ((a - b).abs() / unit).max().item()
+
+
+@DTYPES
+@pytest.mark.parametrize("shape", [(1, 8), (3, 2040), (5, 2048), (2, 7, 2056), (1, 4096), (300, 8192), (2, 16384)])
+def test_rms_norm(shape, dtype):
+    """The mean's summation order can move each of the two roundings to its neighbour: two units in the last place."""
+    print("\n[case] rms norm", shape, dtype, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(shape[-1])
+    x = (torch.randn(shape, device="cuda", generator=gen) * 3).to(dtype)
+    norm = RMSNorm(shape[-1], 1e-5, "cuda", dtype)
+    norm.weight.data.copy_(torch.rand(shape[-1], device="cuda", generator=gen) + 0.5)
+    assert decode._pointwise_kernel_takes(x, norm.weight)
+    y = norm(x)
+    want = norm.weight * F.rms_norm(x.float(), (shape[-1],), eps=1e-5).to(dtype)
+    assert y.shape == want.shape and y.dtype == dtype and _ulps(y, want, dtype) <= 2.0
+    x[0, ..., 3] = float("nan")
+    assert norm(x)[0].isnan().any() and torch.equal(norm(x)[1:], y[1:])
+
+
+@DTYPES
+@pytest.mark.parametrize("shape", [(8,), (3, 264), (2, 5, 11008)])
+def test_silu_mul(shape, dtype):
+    """exp's last bit can move silu's rounding to its neighbour, and the product follows it: two units in the last
+    place. Infinities and NaN as torch's."""
+    print("\n[case] silu mul", shape, dtype, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(shape[-1])
+    gate, up = ((torch.randn(shape, device="cuda", generator=gen) * 4).to(dtype) for _ in range(2))
+    assert decode._pointwise_kernel_takes(gate, up)
+    assert _ulps(silu_mul(gate, up), F.silu(gate) * up, dtype) <= 2.0
+    gate.view(-1)[:5] = torch.tensor([float("inf"), float("-inf"), float("nan"), -200.0, 60000.0], device="cuda")
+    torch.testing.assert_close(silu_mul(gate, up).view(-1)[:5], (F.silu(gate) * up).view(-1)[:5], rtol=0, atol=0,
+                               equal_nan=True)
+
+
+def test_other_forms_keep_torch_ops():
+    x = torch.randn(4, 64, device="cuda").half()
+    norm = RMSNorm(64, 1e-5, "cuda", torch.float16)
+    for form in (x.float(), x.t().contiguous().t(), torch.randn(4, 63, device="cuda").half(), x[:0],
+                 torch.empty(260, device="cuda").half()[1:257].view(4, 64), x.clone().requires_grad_()):
+        assert not decode._pointwise_kernel_takes(form, form)
+    wide = RMSNorm(16392, 1e-5, "cuda", torch.float16)
+    assert wide(torch.ones(2, 16392, device="cuda").half()).shape == (2, 16392)
+    g = x.clone().requires_grad_()
+    assert norm(g).requires_grad and silu_mul(g, x).requires_grad
+    assert torch.equal(norm(x.t().contiguous().t()), norm.weight * F.rms_norm(x.float(), (64,), eps=1e-5).half())
+    out = torch.func.vmap(lambda a: silu_mul(a, a))(x)
+    assert torch.equal(out, F.silu(x) * x)
+    assert silu_mul(x[:, :1], x).shape == (4, 64)  # torch's broadcasting
