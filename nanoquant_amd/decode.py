@@ -135,6 +135,8 @@ def silu_mul(gate, up):
 class RMSNorm(nn.Module):
     """Hugging Face LlamaRMSNorm: normalise in fp32, cast back, then scale."""
 
+    MAX_KERNEL_DIM = 16384
+
     def __init__(self, dim: int, eps: float, device=None, dtype=torch.float32):
         super().__init__()
         self.weight = nn.Parameter(torch.ones(dim, device=device, dtype=dtype), requires_grad=False)
@@ -439,13 +441,17 @@ class NanoQuantLlama(nn.Module):
         emb = torch.cat((freqs, freqs), dim=-1)
         return emb.cos().to(dtype), emb.sin().to(dtype)
 
-    def forward(self, ids, positions, cache: StaticKVCache):
+    def forward(self, ids, positions, cache: StaticKVCache, head=None):
+        """fp32 logits of every position, or ``head(x)`` of the last layer's hidden states x [B, T, hidden] (a
+        caller that needs the logits of a few positions only)."""
         x = self.model.embed_tokens(ids)
         cos, sin = self.rope(positions, x.dtype)
         consts = (self.step_eye, self.step_rot, self.step_mask_values)
         tables = rotary_step_tables(cos, sin, positions, cache, x.dtype, consts=consts) if ids.shape[1] == 1 else None
         for layer in self.model.layers:
             x = layer(x, cos, sin, positions, cache, tables)
+        if head is not None:
+            return head(x)
         x = self.model.norm(x)
         return self.lm_head(x).float()
 
@@ -558,11 +564,14 @@ class GraphDecoder:
         if B != self.batch or T + 1 > self.max_len:
             raise ValueError(f"prompt {tuple(prompt.shape)} does not fit batch {self.batch}, max_len {self.max_len}")
         self.ids[:, :T].copy_(prompt)
-        positions = torch.arange(T, device=self.device)
-        logits = self.model(self.ids[:, :T], positions, self.cache)[:, -1]
+        logits = self._prompt_logits(self.ids[:, :T], torch.arange(T, device=self.device))
         self.ids[:, T] = logits.argmax(dim=-1)
         self.pos.fill_(T)
         return logits
+
+    def _prompt_logits(self, ids, positions):
+        """The logits [B, vocab] of a prompt's last position."""
+        return self.model(ids, positions, self.cache)[:, -1]
 
     @torch.no_grad()
     def decode(self, steps: int, use_graph: bool = True):
@@ -746,6 +755,24 @@ class FusedDecoder(GraphDecoder):
     def _check(self, status, what):
         self._lib.check(status, what)
 
+    def _head(self, x, out, stream):
+        """The final RMS norm folded into the lm_head launch; float32 logits straight from it (with a bias, the
+        dtype logits, the bias added in dtype, then widened, as the torch head rounds). x [batch, hidden]."""
+        hw = self.head_weight
+        self._check(self.lib.nq_dense_gemv(self.dcode, hw.data_ptr(), x.data_ptr(), self.norm_weight.data_ptr(),
+                                           self.model.model.norm.eps, out.data_ptr(), int(self.head_bias is None),
+                                           self.batch, hw.shape[1], hw.shape[0], out.shape[1], stream), "lm_head")
+        return out if self.head_bias is None else (out + self.head_bias).float()
+
+    def _prompt_logits(self, ids, positions):
+        # the last position's logits only, through the step's norm and lm_head launch
+        def head(x):
+            last = x[:, -1].contiguous()
+            out = torch.empty_like(self.logits if self.head_bias is None else self.logits16)
+            with torch.cuda.device(self.device):
+                return self._head(last, out, self._lib.stream_of(self.device))
+        return self.model(ids, positions, self.cache, head=head)
+
     def _linear_residual(self, plan, x, n, stream, what):
         """One linear and its residual. It has no norm to fold in, so its stage 1 is the plain GEMV's, which at
         several batch rows splits wide inputs over the grid (a one-item group has the GEMV's workspace)."""
@@ -811,15 +838,7 @@ class FusedDecoder(GraphDecoder):
             self._check(lib.nq_gemv_group_stage1(dt, n, items, h, B, s.hidden, plan["eps2"], ws, wsb, st), "gu 1")
             self._check(lib.nq_gemv_group_stage2(dt, n, items, B, self._lib.NQ_EPI_GATED, ws, wsb, st), "gu 2")
             self._linear_residual(plan["down"], act, s.ffn, st, "down")
-        # the final RMS norm folded into the lm_head launch; float32 logits straight from it (with a
-        # bias, the dtype logits, the bias added in dtype, then widened, as the torch head rounds)
-        norm = self.model.model.norm
-        hw = self.head_weight
-        out = self.logits if self.head_bias is None else self.logits16
-        self._check(lib.nq_dense_gemv(dt, hw.data_ptr(), self.x.data_ptr(), self.norm_weight.data_ptr(), norm.eps,
-                                      out.data_ptr(), int(self.head_bias is None), B, hw.shape[1], hw.shape[0],
-                                      out.shape[1], st), "lm_head")
-        logits = self.logits if self.head_bias is None else (self.logits16 + self.head_bias).float()
+        logits = self._head(self.x, self.logits if self.head_bias is None else self.logits16, st)
         self._check(lib.nq_argmax_rows(logits.data_ptr(), B, logits.shape[1], logits.stride(0), self.tok.data_ptr(),
                                        st), "argmax")
         self.pos.add_(1)
