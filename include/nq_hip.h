@@ -92,6 +92,18 @@ int nq_unpack_marlin(const uint32_t* words, int8_t* weight, int64_t O, int64_t K
 int nq_repack_marlin(const uint32_t* src, int64_t O, int64_t K, int method, uint32_t* dst, int64_t O_pad,
                      int64_t K_pad, nq_stream_t stream);
 
+/* A whole layer for the prefill GEMM in one launch: the Marlin words of V (outputs padded with +1 from r to
+ * r_pad) and of U (k padded from r to r_pad), the three permuted scales (scale_l's padding zero) and
+ * `workspace_words` zeroed words (workspace may be NULL when there are none). `packed` 0: v int8 [r, n] and
+ * u int8 [m, r], 16-byte aligned, r % 16 == 0 (`method` unused but valid); 1: their sign words in `method`
+ * order, bits past a row's last column ignored. n % 16 == 0, m % 64 == 0, r_pad % 64 == 0. The words are those
+ * of nq_pack_marlin / nq_repack_marlin, the scales those of nq_permute_marlin_scales. Replaces
+ * pack_binary_marlin_fused (src/nanoquant/kernel/utils.py:217-284). */
+int nq_marlin_fused(int packed, const void* v, const void* u, int method, const uint16_t* scale_g,
+                    const uint16_t* scale_l, const uint16_t* scale_h, int64_t n, int64_t r, int64_t m, int64_t r_pad,
+                    uint32_t* v_words, uint32_t* u_words, uint16_t* g_out, uint16_t* l_out, uint16_t* h_out,
+                    int32_t* workspace, int64_t workspace_words, nq_stream_t stream);
+
 /* Scale permutations of pack_binary_marlin (src/nanoquant/kernel/utils.py:206-209), on
  * 16-bit elements: in  [K] -> out [K], natural 16c+8a+2b+d -> 16c+4b+2a+d (K % 16 == 0);
  *                  out [O] -> out [O], natural 32c+8a+2b+d -> 32c+8b+2a+d (O % 32 == 0).

@@ -4,7 +4,8 @@
 // All of them are HBM-bound integer work: one thread owns one output word (the
 // unpacker of whole-word rows: two 16-byte halves of int8 output) so every load
 // and store is a plain coalesced vector access and no thread needs another
-// thread's data.
+// thread's data. The Marlin packers, whose words take bits of eight rows, go
+// through a tile of sign words in LDS.
 #include "nq_common.h"
 
 namespace nq {
@@ -184,6 +185,15 @@ __global__ __launch_bounds__(kThreads) void pack_marlin_kernel(const int8_t* __r
     dst[t] = word;
 }
 
+// A matrix of sign words or int8 to be packed, padded with +1 to [O_pad, K_pad].
+struct MarlinJob {
+    const void* src;  // int8 [O, K] (16-byte aligned, K % 16 == 0) or sign words [O, ceil(K / 32)]
+    uint32_t* dst;    // [K_pad / 16, O_pad / 2]
+    int64_t O, K, O_pad, K_pad;
+    int64_t words;    // ceil(K / 32)
+    uint32_t k_blocks;  // blocks over K_pad
+};
+
 // The same words from a 16-byte aligned matrix, one block per 64 outputs x kMarlinTileK k: the
 // block's 64 row segments reach LDS by 16-byte loads (16 lanes over a row's 256 bytes, where one
 // thread per word made 2-byte loads spread over eight rows), then each thread assembles words
@@ -193,95 +203,160 @@ __global__ __launch_bounds__(kThreads) void pack_marlin_kernel(const int8_t* __r
 constexpr int kMarlinTileK = 256;
 constexpr int kMarlinRowStride = kMarlinTileK + 16;  // bytes: rows 4 banks apart, 16-byte aligned
 
-__global__ __launch_bounds__(kThreads) void pack_marlin_tiled_kernel(const int8_t* __restrict__ w,
-                                                                     uint32_t* __restrict__ dst, int64_t O,
-                                                                     int64_t K) {
-    __shared__ __attribute__((aligned(16))) int8_t tile[64 * kMarlinRowStride];
-    const int t = static_cast<int>(threadIdx.x);
-    const int64_t tile_out = blockIdx.y;
-    const int64_t k0 = static_cast<int64_t>(blockIdx.x) * kMarlinTileK;
-    const int kn = static_cast<int>(K - k0 < kMarlinTileK ? K - k0 : kMarlinTileK);  // a multiple of 16
-    constexpr int kChunks = kMarlinTileK / 16;  // 16-byte chunks of a full row segment
-    constexpr int kPer = 64 * kChunks / kThreads;  // 16-byte loads per thread, all issued before their stores
-    u32x4 v[kPer];
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-        const int i = t + j * kThreads;
-        const int r = i / kChunks, c = i - r * kChunks;
-        v[j] = 16 * c < kn ? *reinterpret_cast<const u32x4*>(w + (tile_out * 64 + r) * K + k0 + 16 * c) : u32x4{0, 0, 0, 0};
-    }
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-        const int i = t + j * kThreads;
-        const int r = i / kChunks, c = i - r * kChunks;
-        if (16 * c < kn) *reinterpret_cast<u32x4*>(tile + r * kMarlinRowStride + 16 * c) = v[j];
-    }
-    __syncthreads();
-    const int64_t half_o = O / 2;
-    for (int i = t; i < (kn / 16) * 32; i += kThreads) {
-        const int trl = i / 32, cl = i - trl * 32;
-        const int o1 = cl / 4, r2 = cl % 4;
-        uint32_t word = 0;
-#pragma unroll
-        for (int o16 = 0; o16 < 4; ++o16) {
-#pragma unroll
-            for (int o8 = 0; o8 < 2; ++o8) {
-#pragma unroll
-                for (int r8 = 0; r8 < 2; ++r8) {
-                    const int row = o16 * 16 + o8 * 8 + o1;
-                    const int kk = trl * 16 + r8 * 8 + r2 * 2;
-                    const uint16_t pair = *reinterpret_cast<const uint16_t*>(tile + row * kMarlinRowStride + kk);
-                    const uint32_t neg_lo = (pair >> 7) & 1u;   // element k   (r1 = 0)
-                    const uint32_t neg_hi = (pair >> 15) & 1u;  // element k+1 (r1 = 1)
-                    const int bit = 15 - (2 * o8 + r8) - 4 * o16;
-                    word |= (neg_lo << bit) | (neg_hi << (bit + 16));
-                }
-            }
-        }
-        dst[(k0 / 16 + trl) * half_o + tile_out * 32 + cl] = word;
-    }
-}
+// From sign words: a block takes 64 outputs x kTileWords words of k, brings them into LDS as half2 words
+// (rows 17 words apart: the eight rows a Marlin word reads lie in eight banks) and assembles its words.
+//
+// In a half2 word the pair (k, k + 1), k = 2 a, has its signs on bits 15 - a and 31 - a; the Marlin word
+// wants the pair a = 8 (tr % 2) + 4 r8 + r2 of row (o16, o8) on bits 15 - b and 31 - b, b = 2 o8 + r8 + 4 o16.
+// So each of the word's 16 pairs is one rotate by a - b and one and-or under 0x80008000 >> b.
+//
+// Measured (MI355X, us; one thread per word, gathering single bits of eight rows -> this): [3520, 8192] 11.7 ->
+// 5.3, [28672, 3520] 33.1 -> 11.9 (25 MB; tiles of 8 words 13.6, of 32 12.6). int8 through the same LDS
+// words was slower than the int8 tile above (5.2 against 4.5 on [1792, 11008]).
+constexpr int kTileWords = 16;
+constexpr int kTileStride = kTileWords + 1;
 
-// Marlin words [K_pad/16, O_pad/2] straight from the sign words of a [O, K] matrix (lsb_first
-// or half2, ceil(K/32) words a row), as a checkpoint stores V [r, n] and U [m, r]; elements past
-// O or K are +1 (bit 0). Each output word's four k lie in one 16-k group, so in one source word
-// per row.
-__global__ __launch_bounds__(kThreads) void repack_marlin_kernel(const uint32_t* __restrict__ src, int64_t O,
-                                                                 int64_t K, int64_t words, int method,
-                                                                 uint32_t* __restrict__ dst, int64_t O_pad,
-                                                                 int64_t K_pad) {
-    const int64_t half_o = O_pad / 2;
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-    if (t >= (K_pad / 16) * half_o) return;
-    const int64_t tr = t / half_o;
-    const int64_t col = t - tr * half_o;
-    const int64_t tile_out = col / 32;
-    const int o1 = static_cast<int>((col % 32) / 4);
-    const int r2 = static_cast<int>(col % 4);
-    const int64_t k0 = tr * 16 + r2 * 2;  // the word's k: k0 + 8*r8 + r1
-    uint32_t word = 0;
-    if (k0 < K) {
-        const int64_t kw = k0 / 32;
+// Dwords of LDS a block takes.
+constexpr int tile_dwords(bool dense) { return dense ? 64 * kMarlinRowStride / 4 : 64 * kTileStride; }
+
+// kPad false: an int8 matrix that is its own padding (the tests against its true sizes cost a tenth: 4.3 against
+// 4.7 us on [1792, 11008]).
+template <bool kDense, bool kPad>
+__device__ inline void marlin_tile(const MarlinJob& j, int64_t to, int64_t kb, int method, uint32_t* lds) {
+    const int t = static_cast<int>(threadIdx.x);
+    const int64_t half_o = j.O_pad / 2;
+    if constexpr (kDense) {
+        int8_t* tile = reinterpret_cast<int8_t*>(lds);
+        const auto* w = static_cast<const int8_t*>(j.src);
+        const int64_t k0 = kb * kMarlinTileK;
+        const int kn = static_cast<int>(min<int64_t>(j.K_pad - k0, kMarlinTileK));  // multiples of 16, as the matrix's part
+        const int kv = static_cast<int>(max<int64_t>(min<int64_t>(j.K - k0, kMarlinTileK), 0));
+        const int rv = static_cast<int>(max<int64_t>(min<int64_t>(j.O - to * 64, 64), 0));
+        const int8_t* src = w + to * 64 * j.K + k0;
+        constexpr int kChunks = kMarlinTileK / 16;  // 16-byte chunks of a full row segment
+        constexpr int kPer = 64 * kChunks / kThreads;  // 16-byte loads per thread, all issued before their stores
+        u32x4 v[kPer];
 #pragma unroll
-        for (int o16 = 0; o16 < 4; ++o16) {
+        for (int i = 0; i < kPer; ++i) {
+            const int e = t + i * kThreads;
+            const int r = e / kChunks, c = e - r * kChunks;
+            // zeros (not negative: +1) past the matrix
+            v[i] = 16 * c < (kPad ? kv : kn) && (!kPad || r < rv) ? *reinterpret_cast<const u32x4*>(src + static_cast<int64_t>(r) * j.K + 16 * c)
+                                         : u32x4{0, 0, 0, 0};
+        }
 #pragma unroll
-            for (int o8 = 0; o8 < 2; ++o8) {
-                const int64_t o = tile_out * 64 + o16 * 16 + o8 * 8 + o1;
-                if (o >= O) continue;
-                const uint32_t L = from_method(src[o * words + kw], method);
+        for (int i = 0; i < kPer; ++i) {
+            const int e = t + i * kThreads;
+            const int r = e / kChunks, c = e - r * kChunks;
+            if (16 * c < kn) *reinterpret_cast<u32x4*>(tile + r * kMarlinRowStride + 16 * c) = v[i];
+        }
+        __syncthreads();
+        for (int i = t; i < (kn / 16) * 32; i += kThreads) {
+            const int trl = i / 32, cl = i - trl * 32;
+            const int o1 = cl / 4, r2 = cl % 4;
+            uint32_t word = 0;
 #pragma unroll
-                for (int r8 = 0; r8 < 2; ++r8) {
+            for (int o16 = 0; o16 < 4; ++o16) {
 #pragma unroll
-                    for (int r1 = 0; r1 < 2; ++r1) {
-                        const int64_t k = k0 + 8 * r8 + r1;
-                        const uint32_t neg = k < K ? (L >> (k % 32)) & 1u : 0u;
-                        word |= neg << (15 - (2 * o8 + r8) - 4 * o16 + 16 * r1);
+                for (int o8 = 0; o8 < 2; ++o8) {
+#pragma unroll
+                    for (int r8 = 0; r8 < 2; ++r8) {
+                        const int row = o16 * 16 + o8 * 8 + o1;
+                        const int kk = trl * 16 + r8 * 8 + r2 * 2;
+                        const uint16_t pair = *reinterpret_cast<const uint16_t*>(tile + row * kMarlinRowStride + kk);
+                        const uint32_t neg_lo = (pair >> 7) & 1u;   // element k   (r1 = 0)
+                        const uint32_t neg_hi = (pair >> 15) & 1u;  // element k+1 (r1 = 1)
+                        const int bit = 15 - (2 * o8 + r8) - 4 * o16;
+                        word |= (neg_lo << bit) | (neg_hi << (bit + 16));
                     }
                 }
             }
+            j.dst[(k0 / 16 + trl) * half_o + to * 32 + cl] = word;
+        }
+    } else {
+        const int64_t w0 = kb * kTileWords;
+        constexpr int kPer = 64 * kTileWords / kThreads;
+        uint32_t v[kPer];
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            const int e = t + i * kThreads;
+            const int64_t row = to * 64 + e / kTileWords, w = w0 + e % kTileWords;
+            v[i] = row < j.O && w < j.words ? static_cast<const uint32_t*>(j.src)[row * j.words + w] : 0u;
+        }
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            const int e = t + i * kThreads;
+            const int64_t left = j.K - 32 * (w0 + e % kTileWords);  // bits past K are +1 whatever the source holds
+            if (left < 32 && left > 0) v[i] = to_method(from_method(v[i], method) & ((1u << left) - 1u), method);
+            lds[(e / kTileWords) * kTileStride + e % kTileWords] = method == NQ_PACK_HALF2 ? v[i] : lsb_to_half2(v[i]);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            const int e = t + i * kThreads;
+            const int trl = e / 32, col = e % 32;  // tile row and column of the block's 2 kTileWords x 32 words
+            const int64_t tr = 2 * w0 + trl;
+            if (16 * tr >= j.K_pad) continue;
+            const uint32_t* rows = lds + (col / 4) * kTileStride + trl / 2;
+            const int a0 = 8 * (trl & 1) + (col & 3);
+            uint32_t word = 0;
+#pragma unroll
+            for (int o16 = 0; o16 < 4; ++o16)
+#pragma unroll
+                for (int o8 = 0; o8 < 2; ++o8) {
+                    const uint32_t h = rows[(16 * o16 + 8 * o8) * kTileStride];
+#pragma unroll
+                    for (int r8 = 0; r8 < 2; ++r8) {
+                        const int b = 2 * o8 + r8 + 4 * o16;
+                        word |= __builtin_rotateleft32(h, static_cast<uint32_t>(a0 + 4 * r8 - b) & 31u) & (0x80008000u >> b);
+                    }
+                }
+            j.dst[tr * half_o + to * 32 + col] = word;
         }
     }
-    dst[t] = word;
+}
+
+template <bool kDense>
+__global__ __launch_bounds__(kThreads) void marlin_kernel(const MarlinJob job, int method) {
+    __shared__ __attribute__((aligned(16))) uint32_t lds[tile_dwords(kDense)];
+    if (kDense) marlin_tile<kDense, false>(job, blockIdx.y, blockIdx.x, method, lds);
+    else marlin_tile<kDense, true>(job, blockIdx.x / job.k_blocks, blockIdx.x % job.k_blocks, method, lds);
+}
+
+// Position of element i of an input (16-blocks 8a + 2b + d) or output (32-blocks) scale in its permuted vector.
+__device__ inline int64_t perm_scale_in(int64_t i) {
+    return (i & ~int64_t{15}) + 4 * ((i % 8) / 2) + 2 * ((i % 16) / 8) + i % 2;
+}
+__device__ inline int64_t perm_scale_out(int64_t i) {
+    return (i & ~int64_t{31}) + 8 * ((i % 8) / 2) + 2 * ((i % 32) / 8) + i % 2;
+}
+
+// Measured: a 7B down_proj from int8 (3 launches of torch byte transposes and copies a factor before) 256 -> 44 us
+// a call with its four packed outputs, a 70B gate_proj from words 90 -> 43; 14 launches -> one.
+// A whole layer: V's blocks, U's blocks, then the blocks of the three scales (the rank's padded with zeros)
+// and of the zeroed workspace.
+struct MarlinFused {
+    MarlinJob v, u;
+    uint32_t v_blocks, u_blocks;
+    const uint16_t *g, *l, *h;
+    uint16_t *g_out, *l_out, *h_out;
+    int64_t n, r, r_pad, m;
+    int32_t* workspace;
+    int64_t workspace_words;
+};
+
+template <bool kDense>
+__global__ __launch_bounds__(kThreads) void marlin_fused_kernel(const MarlinFused f, int method) {
+    __shared__ __attribute__((aligned(16))) uint32_t lds[tile_dwords(kDense)];
+    uint32_t block = blockIdx.x;
+    if (block < f.v_blocks) return marlin_tile<kDense, true>(f.v, block / f.v.k_blocks, block % f.v.k_blocks, method, lds);
+    block -= f.v_blocks;
+    if (block < f.u_blocks) return marlin_tile<kDense, true>(f.u, block / f.u.k_blocks, block % f.u.k_blocks, method, lds);
+    const int64_t i = static_cast<int64_t>(block - f.u_blocks) * kThreads + threadIdx.x;
+    if (i < f.n) f.g_out[perm_scale_in(i)] = f.g[i];
+    if (i < f.r_pad) f.l_out[perm_scale_out(i)] = i < f.r ? f.l[i] : uint16_t(0);
+    if (i < f.m) f.h_out[perm_scale_out(i)] = f.h[i];
+    if (i < f.workspace_words) f.workspace[i] = 0;
 }
 
 __global__ __launch_bounds__(kThreads) void unpack_marlin_kernel(const uint32_t* __restrict__ src,
@@ -317,17 +392,18 @@ __global__ __launch_bounds__(kThreads) void permute_scales_kernel(const uint16_t
                                                                   const uint16_t* __restrict__ s_out,
                                                                   uint16_t* __restrict__ s_out_out, int64_t O) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-    if (s_in != nullptr && i < K) {
-        const int64_t c = i / 16, a = (i % 16) / 8, b = (i % 8) / 2, d = i % 2;
-        s_in_out[16 * c + 4 * b + 2 * a + d] = s_in[i];
-    }
-    if (s_out != nullptr && i < O) {
-        const int64_t c = i / 32, a = (i % 32) / 8, b = (i % 8) / 2, d = i % 2;
-        s_out_out[32 * c + 8 * b + 2 * a + d] = s_out[i];
-    }
+    if (s_in != nullptr && i < K) s_in_out[perm_scale_in(i)] = s_in[i];
+    if (s_out != nullptr && i < O) s_out_out[perm_scale_out(i)] = s_out[i];
 }
 
 inline dim3 grid_for(int64_t items) { return dim3(static_cast<unsigned>(ceil_div(items, kThreads))); }
+
+// The blocks of one matrix, O_pad % 64 == 0.
+MarlinJob marlin_job(bool dense, const void* src, uint32_t* dst, int64_t O, int64_t K, int64_t O_pad, int64_t K_pad) {
+    return MarlinJob{src, dst, O, K, O_pad, K_pad, ceil_div(K, 32),
+                     static_cast<uint32_t>(ceil_div(K_pad, dense ? kMarlinTileK : 32 * kTileWords))};
+}
+int64_t marlin_blocks(const MarlinJob& j) { return static_cast<int64_t>(j.k_blocks) * (j.O_pad / 64); }
 
 int check_method(int method, const char* name) {
     if (method != NQ_PACK_LSB_FIRST && method != NQ_PACK_HALF2)
@@ -398,9 +474,10 @@ int nq_pack_marlin(const int8_t* weight, uint32_t* dst, int64_t O, int64_t K, nq
     if (O == 0 || K == 0) return NQ_OK;
     if (!weight || !dst) return fail(NQ_ERR_INVALID_ARGUMENT, "nq_pack_marlin: null pointer");
     if (!aligned(weight, 2)) return fail(NQ_ERR_ALIGNMENT, "nq_pack_marlin: weight must be 2-byte aligned");
+    const MarlinJob job = marlin_job(true, weight, dst, O, K, O, K);
     if (aligned(weight, 16))
-        pack_marlin_tiled_kernel<<<dim3(static_cast<unsigned>(ceil_div(K, kMarlinTileK)), static_cast<unsigned>(O / 64)),
-                                   kThreads, 0, as_stream(stream)>>>(weight, dst, O, K);
+        marlin_kernel<true><<<dim3(job.k_blocks, static_cast<unsigned>(O / 64)), kThreads, 0, as_stream(stream)>>>(
+            job, NQ_PACK_LSB_FIRST);
     else
         pack_marlin_kernel<<<grid_for((K / 16) * (O / 2)), kThreads, 0, as_stream(stream)>>>(weight, dst, O, K);
     return check_launch("nq_pack_marlin");
@@ -416,9 +493,53 @@ int nq_repack_marlin(const uint32_t* src, int64_t O, int64_t K, int method, uint
                     (long long)O_pad, (long long)K_pad);
     if (O_pad == 0 || K_pad == 0) return NQ_OK;
     if (!dst || (O > 0 && K > 0 && !src)) return fail(NQ_ERR_INVALID_ARGUMENT, "nq_repack_marlin: null pointer");
-    repack_marlin_kernel<<<grid_for((K_pad / 16) * (O_pad / 2)), kThreads, 0, as_stream(stream)>>>(
-        src, O, K, ceil_div(K, 32), method, dst, O_pad, K_pad);
+    const MarlinJob job = marlin_job(false, src, dst, O, K, O_pad, K_pad);
+    if (marlin_blocks(job) > INT32_MAX) return fail(NQ_ERR_UNSUPPORTED, "nq_repack_marlin: sizes too large");
+    marlin_kernel<false><<<dim3(static_cast<unsigned>(marlin_blocks(job))), kThreads, 0, as_stream(stream)>>>(job, method);
     return check_launch("nq_repack_marlin");
+}
+
+int nq_marlin_fused(int packed, const void* v, const void* u, int method, const uint16_t* scale_g, const uint16_t* scale_l,
+                    const uint16_t* scale_h, int64_t n, int64_t r, int64_t m, int64_t r_pad, uint32_t* v_words,
+                    uint32_t* u_words, uint16_t* g_out, uint16_t* l_out, uint16_t* h_out, int32_t* workspace,
+                    int64_t workspace_words, nq_stream_t stream) {
+    const char* name = "nq_marlin_fused";
+    if (int s = check_method(method, name)) return s;
+    if (n <= 0 || r <= 0 || m <= 0 || workspace_words < 0)
+        return fail(NQ_ERR_INVALID_ARGUMENT, "%s: bad sizes", name);
+    if (n % 16 || m % 64 || r_pad % 64 || r_pad < r || (!packed && r % 16))
+        return fail(NQ_ERR_SHAPE, "%s: need n %% 16 == 0, m %% 64 == 0, r <= r_pad, r_pad %% 64 == 0 (and r %% 16 == 0 for int8)",
+                    name);
+    if (!v || !u || !scale_g || !scale_l || !scale_h || !v_words || !u_words || !g_out || !l_out || !h_out ||
+        (workspace_words > 0 && !workspace))
+        return fail(NQ_ERR_INVALID_ARGUMENT, "%s: null pointer", name);
+    if (!aligned(v, packed ? 4 : 16) || !aligned(u, packed ? 4 : 16))
+        return fail(NQ_ERR_ALIGNMENT, "%s: int8 factors must be 16-byte aligned", name);
+    MarlinFused f;
+    f.v = marlin_job(!packed, v, v_words, r, n, r_pad, n);
+    f.u = marlin_job(!packed, u, u_words, m, r, m, r_pad);
+    f.g = scale_g;
+    f.l = scale_l;
+    f.h = scale_h;
+    f.g_out = g_out;
+    f.l_out = l_out;
+    f.h_out = h_out;
+    f.n = n;
+    f.r = r;
+    f.r_pad = r_pad;
+    f.m = m;
+    f.workspace = workspace;
+    f.workspace_words = workspace_words;
+    int64_t rest = n;
+    for (int64_t c : {r_pad, m, workspace_words}) rest = c > rest ? c : rest;
+    const int64_t blocks = marlin_blocks(f.v) + marlin_blocks(f.u) + ceil_div(rest, kThreads);
+    if (blocks > INT32_MAX) return fail(NQ_ERR_UNSUPPORTED, "%s: sizes too large", name);
+    f.v_blocks = static_cast<uint32_t>(marlin_blocks(f.v));
+    f.u_blocks = static_cast<uint32_t>(marlin_blocks(f.u));
+    const dim3 grid(static_cast<unsigned>(blocks));
+    if (packed) marlin_fused_kernel<false><<<grid, kThreads, 0, as_stream(stream)>>>(f, method);
+    else marlin_fused_kernel<true><<<grid, kThreads, 0, as_stream(stream)>>>(f, method);
+    return check_launch(name);
 }
 
 int nq_unpack_marlin(const uint32_t* words, int8_t* weight, int64_t O, int64_t K, nq_stream_t stream) {

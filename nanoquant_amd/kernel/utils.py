@@ -190,6 +190,36 @@ def pack_binary_marlin(weight: torch.Tensor, scale_in: torch.Tensor,
     return words, s_in, s_out, workspace_size
 
 
+def _fused_on_gpu(packed: bool, V, U, sizes, method: int, scales):
+    """One launch for a whole layer (``nq_marlin_fused``): V and U as int8 [r, n] and [m, r] or as their sign words;
+    returns the fused packer's tuple. None when a size, type or device needs the general route (which also
+    raises its errors)."""
+    n, r, m = sizes
+    if not (V.is_cuda and n > 0 and m > 0 and r > 0 and n % 16 == 0 and m % 64 == 0 and (packed or r % 32 == 0)):
+        return None
+    if not all(s.device == V.device and s.dim() == 1 and s.element_size() == 2 for s in scales) or U.device != V.device:
+        return None
+    if tuple(s.shape[0] for s in scales) != (n, r, m):
+        return None
+    V, U = V.contiguous(), U.contiguous()
+    if not packed and (V.data_ptr() % 16 or U.data_ptr() % 16):
+        return None
+    r_pad = marlin_rank(r)
+    g, l, h = (s.contiguous() for s in scales)
+    new = dict(device=V.device, dtype=torch.int32)
+    V_bits, U_bits = torch.empty((n // 16, r_pad // 2), **new), torch.empty((r_pad // 16, m // 2), **new)
+    g_out, l_out, h_out = torch.empty_like(g), torch.empty(r_pad, device=V.device, dtype=l.dtype), torch.empty_like(h)
+    workspace = torch.empty(max(r_pad, m) // 128 * MARLIN_MIN_MAX_PAR, **new)
+    lib = _lib.load()
+    with torch.cuda.device(V.device):
+        status = lib.nq_marlin_fused(int(packed), V.data_ptr(), U.data_ptr(), method, g.data_ptr(), l.data_ptr(),
+                                     h.data_ptr(), n, r, m, r_pad, V_bits.data_ptr(), U_bits.data_ptr(),
+                                     g_out.data_ptr(), l_out.data_ptr(), h_out.data_ptr(), workspace.data_ptr(),
+                                     workspace.numel(), _lib.stream_of(V.device))
+    _lib.check(status, "pack_binary_marlin_fused")
+    return V_bits, U_bits, g_out, l_out, h_out, workspace
+
+
 def pack_binary_marlin_fused(V_sign: torch.Tensor, U_sign: torch.Tensor, scale_g: torch.Tensor,
                              scale_l: torch.Tensor, scale_h: torch.Tensor):
     """Pack both binary factors for ``marlin_nanoquant_forward`` (kernel/utils.py:217-284).
@@ -205,6 +235,10 @@ def pack_binary_marlin_fused(V_sign: torch.Tensor, U_sign: torch.Tensor, scale_g
     N = scale_g.shape[0]
     R = scale_l.shape[0]
     M = scale_h.shape[0]
+    if V_sign.dtype == U_sign.dtype == torch.int8 and tuple(V_sign.shape) == (N, R) and tuple(U_sign.shape) == (R, M):
+        fused = _fused_on_gpu(False, V_sign.T, U_sign.T, (N, R, M), _lib.NQ_PACK_LSB_FIRST, (scale_g, scale_l, scale_h))
+        if fused is not None:
+            return fused
     p = 32
     if R % p != 0:
         R = ((R // p) + 1) * p
@@ -281,6 +315,11 @@ def pack_binary_marlin_fused_from_packed(V_packed: torch.Tensor, V_shape: Tuple[
     if r_u != r or scale_l.shape[0] != r or scale_g.shape[0] != n or scale_h.shape[0] != m:
         raise ValueError(f"factor shapes disagree: V {tuple(V_shape)}, U {tuple(U_shape)}, scales "
                          f"{scale_g.shape[0]}, {scale_l.shape[0]}, {scale_h.shape[0]}")
+    if (V_packed.dtype in (torch.int32, torch.uint32) and U_packed.dtype in (torch.int32, torch.uint32)
+            and tuple(V_packed.shape) == (r, (n + 31) // 32) and tuple(U_packed.shape) == (m, (r + 31) // 32)):
+        fused = _fused_on_gpu(True, V_packed, U_packed, (n, r, m), _method_code(src_method), (scale_g, scale_l, scale_h))
+        if fused is not None:
+            return fused
     r_pad = marlin_rank(r)
     V_bits = repack_binary_marlin(V_packed, (r, n), (r_pad, n), src_method)
     U_bits = repack_binary_marlin(U_packed, (m, r), (m, r_pad), src_method)
