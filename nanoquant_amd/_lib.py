@@ -14,6 +14,7 @@ import torch  # noqa: F401  (must precede the CDLL load, see module docstring)
 
 LIB_NAME = "libnq_hip.so"
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
+OPS_PATH = os.path.join(os.path.dirname(LIB_PATH), "libnq_ops.so")  # the torch operators in C++
 
 NQ_OK = 0
 NQ_ERR_INVALID_ARGUMENT = 1
@@ -98,8 +99,24 @@ SIGNATURES = {
 }
 
 
+# The functions that libnq_ops.so (the torch operators) calls, in the order of its nq_ops_bind.
+OPS_FUNCTIONS = ("nq_gemv_workspace_bytes", "nq_gemv", "nq_gemm_onebit_workspace_bytes", "nq_gemm_onebit",
+                 "nq_gemm_nanoquant_workspace_bytes", "nq_gemm_nanoquant")
+
 _lock = threading.Lock()
 _lib = None
+ops = None  # the C++ operators' library, set by binary_kernels where it registers them
+
+
+def _bind_ops(lib: ctypes.CDLL) -> None:
+    """Hand the C++ operators the library's functions."""
+    if ops is None:
+        return
+    table = (_vp * len(OPS_FUNCTIONS))(*(ctypes.cast(getattr(lib, name), _vp).value for name in OPS_FUNCTIONS))
+    bind = ops.nq_ops_bind
+    bind.restype, bind.argtypes = _int, [ctypes.POINTER(_vp), _int]
+    if bind(table, len(OPS_FUNCTIONS)) != 0:
+        raise ImportError(f"{OPS_PATH} and this package disagree; run `python -m nanoquant_amd.build`")
 
 
 class NQError(RuntimeError):
@@ -125,6 +142,7 @@ def load() -> ctypes.CDLL:
                 fn = getattr(lib, name)
                 fn.restype = res
                 fn.argtypes = args
+            _bind_ops(lib)
             _lib = lib
     return _lib
 

@@ -7,6 +7,13 @@ with a CUDA (= HIP on ROCm) implementation that calls the C ABI and a fake
 ``gemm.cpp:100-110,124-134``). There is no CPU implementation: a CPU tensor fails
 in the dispatcher as it does with the reference.
 
+The CUDA implementations are C++ (``csrc/torch_ops/nq_ops.cpp``, ``libnq_ops.so``): at decode
+sizes a call is bound by its host path, 24 us through the functions of this module and 11
+through those. They take every well-formed call; the functions here, registered as the same
+operators of the namespace ``nanoquant_amd``, take the rest: the first call (they load the
+HIP library), empty sizes, and every call to be refused, so that checks and messages stand
+here once. Without a built ``libnq_ops.so`` they serve ``binary_kernels`` directly.
+
 Argument checks and their messages follow the reference: RuntimeError for
 device/contiguity/dtype/size problems (``cuda_utils.cuh:13-50``,
 ``gemv_kernel.cu:316-338``, ``gemm.cpp:44-52,90``) and ValueError for tuning ints
@@ -17,6 +24,9 @@ multiples of their tiles, >2-D inputs) are computed correctly here, and the
 packed operand shapes are checked, which the reference does not do.
 """
 from __future__ import annotations
+
+import ctypes
+import os
 
 import torch
 
@@ -251,18 +261,26 @@ def marlin_nanoquant_forward_fake(x, weight_u, weight_v, scale_g, scale_l, scale
 
 # --------------------------------------------------------------------------- registration
 
+_GENERAL_NS = "nanoquant_amd"
+
+
 def _register():
-    lib = torch.library.Library(_NS, "DEF")
-    lib.define(GEMV_SCHEMA)
-    lib.define(ONEBIT_SCHEMA)
-    lib.define(NANOQUANT_SCHEMA)
-    lib.impl("nanoquant_dyn_forward", nanoquant_dyn_forward_cuda, "CUDA")
-    lib.impl("marlin_onebit_forward", marlin_onebit_forward_cuda, "CUDA")
-    lib.impl("marlin_nanoquant_forward", marlin_nanoquant_forward_cuda, "CUDA")
-    torch.library.register_fake(f"{_NS}::nanoquant_dyn_forward", nanoquant_dyn_forward_fake, lib=lib)
-    torch.library.register_fake(f"{_NS}::marlin_onebit_forward", marlin_onebit_forward_fake, lib=lib)
-    torch.library.register_fake(f"{_NS}::marlin_nanoquant_forward", marlin_nanoquant_forward_fake, lib=lib)
-    return lib
+    ops = ((GEMV_SCHEMA, nanoquant_dyn_forward_cuda, nanoquant_dyn_forward_fake),
+           (ONEBIT_SCHEMA, marlin_onebit_forward_cuda, marlin_onebit_forward_fake),
+           (NANOQUANT_SCHEMA, marlin_nanoquant_forward_cuda, marlin_nanoquant_forward_fake))
+    lib, general = torch.library.Library(_NS, "DEF"), torch.library.Library(_GENERAL_NS, "DEF")
+    native = os.path.exists(_lib.OPS_PATH)
+    for schema, cuda, fake in ops:
+        name = schema[:schema.index("(")]
+        lib.define(schema)
+        general.define(schema)
+        general.impl(name, cuda, "CUDA")
+        if not native:
+            lib.impl(name, cuda, "CUDA")
+        torch.library.register_fake(f"{_NS}::{name}", fake, lib=lib)
+    if native:
+        _lib.ops = ctypes.CDLL(_lib.OPS_PATH)  # registers its implementations as it is loaded
+    return lib, general
 
 
 _LIBRARY = _register()

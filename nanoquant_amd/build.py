@@ -1,8 +1,10 @@
-"""Build recipe of the HIP library ``nanoquant_amd/libnq_hip.so`` (gfx950).
+"""Build recipe of the HIP library ``nanoquant_amd/libnq_hip.so`` (gfx950) and of
+``nanoquant_amd/libnq_ops.so``, the C++ implementations of the torch operators.
 
 ``python -m nanoquant_amd.build`` compiles every source under ``csrc/`` with hipcc
-and links the shared library in place, next to this file, so that it travels
-with the source tree. Objects go to ``_build/`` (git-ignored).
+and ``csrc/torch_ops/`` with g++ against torch's headers, and links the shared
+libraries in place, next to this file, so that they travel with the source tree.
+Objects go to ``_build/`` (git-ignored).
 """
 from __future__ import annotations
 
@@ -17,6 +19,8 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD_DIR = os.path.join(os.path.dirname(HERE), "_build")
 LIB_NAME = "libnq_hip.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
+OPS_SOURCE = os.path.join(CSRC, "torch_ops", "nq_ops.cpp")
+OPS_PATH = os.path.join(HERE, "libnq_ops.so")
 ARCH = os.environ.get("NQ_OFFLOAD_ARCH", "gfx950")
 
 COMMON_FLAGS = [
@@ -61,12 +65,33 @@ def _compile(src: str) -> str:
     return obj
 
 
+def build_ops() -> str:
+    """Compile the torch operators (host code only); returns the library's path."""
+    import torch
+    from torch.utils import cpp_extension
+
+    lib_dir = os.path.join(os.path.dirname(torch.__file__), "lib")
+    tmp = OPS_PATH + ".tmp"
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+    for path in cpp_extension.include_paths("cuda"):
+        cmd += ["-isystem", path]
+    cmd += [OPS_SOURCE, "-o", tmp, f"-L{lib_dir}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"compile failed: {' '.join(cmd)}\n{proc.stdout}\n{proc.stderr}")
+    os.replace(tmp, OPS_PATH)
+    return OPS_PATH
+
+
 def build(verbose: bool = True) -> str:
-    """Compile and link the library; returns its path."""
+    """Compile and link the libraries; returns the HIP library's path."""
     os.makedirs(BUILD_DIR, exist_ok=True)
     srcs = sources()
-    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
+    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(srcs) + 1)) as ex:
+        ops = ex.submit(build_ops)
         objs = list(ex.map(_compile, srcs))
+        ops.result()
     tmp = LIB_PATH + ".tmp"
     cmd = [hipcc(), "-shared", "-fPIC", f"--offload-arch={ARCH}", *objs, "-o", tmp]
     proc = subprocess.run(cmd, capture_output=True, text=True)
