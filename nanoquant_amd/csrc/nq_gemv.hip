@@ -37,6 +37,7 @@
 
 #include "nq_common.h"
 #include "nq_gemv_rows.h"
+#include "nq_gemv_split.h"
 
 // Phase marks of the fast kernels; empty in the library (a timing build may define them).
 #ifndef NQ_STAMP
@@ -2585,7 +2586,7 @@ inline bool s2t_applies(const void* z_hi, const void* z_lo, const uint32_t* u_bi
 // 38.7 / 13.1 at 128; down, 4096 rows: 4.0 / 5.3 at 16 and 5.0 / 5.5 at 32 stay with s2t, 9.1 / 6.05
 // at 64, 16.0 / 7.1 at 128). Every shape gives each wave one row tile against one to four column
 // tiles. Over 512 or more row tiles: 64-row blocks (WR = 4) of 16 batch rows up to 64 rows, 32
-// beyond, two-word chunks (640-1023 tiles at 16 rows or fewer: as below 512). Below: 32-row blocks (WR = 2) of 16 batch rows and four-word chunks up
+// beyond, two-word chunks. Below: 32-row blocks (WR = 2) of 16 batch rows and four-word chunks up
 // to 64 rows, 32 batch rows and two-word chunks beyond. Smaller chunks leave room in LDS for more
 // resident blocks, which is what these latency-bound blocks gain from.
 constexpr int64_t kS2bMinWork = 160 * 1024;
@@ -2611,14 +2612,39 @@ inline bool s2b_chosen(int batch, int m, const Plan& plan, int items = 1) {
            ceil_div(batch, s2t_rows_per_pass(batch, items * plan.s2_qw)) >= 2;
 }
 
+// When the kernels that split the rank over a block's waves (nq_gemv_split.hip) take a stage 2, or a gated pair
+// (`items` 2), before the two above. `work` is words of U times batch rows; us, those against these.
+// Single, from two batch rows: where s2t_kernel would need several passes over U and there is work for the grid (m =
+// 4096, r = 2976 at 16 rows 6.2 / 5.4, m = 8192, r = 1120 at 16 4.4 / 4.3, against m = 4096, r = 1632 at 16 4.1 / 4.2, m =
+// 1024, r = 896 at 16 3.0 / 3.3), but not over 16384 rows or more beyond 8 batch rows, where s2b_kernel's blocks of 64
+// rows fill the chip (m = 28672, r = 3520 at 16 rows 12.7 / 14.8), nor beyond 16 batch rows over more than 8192 rows
+// or below 64 words (m = 11008, r = 1632 at 32 7.2 / 8.1; m = 8192, r = 1120 at 32 5.35 / 5.6, r = 2240 8.2 / 6.9); and
+// the largest U up to 8 batch rows in any case (m = 28672, r = 3520 at 2 / 4 rows 11.45 / 10.6, 12.6 / 10.45; m = 20480
+// at 4 9.5 / 9.9).
+// Pair, from three batch rows: s2t_kernel holds half as many batch rows a pass (m = 11008, r = 1632 at 2 / 3 rows 6.7 /
+// 8.1, 9.5 / 8.0; m = 4096, r = 1632 at 4 / 6 rows 5.2 / 5.4, 7.15 / 5.4), and beyond 16 but for the largest U (m =
+// 28672, r = 3520 at 32 rows 42.9 / 43.4; m = 11008, r = 2976 23.0 / 20.0); the largest U from two (24.4 / 20.9).
+constexpr int64_t kSplitWork = 3500000, kSplitPairWork = 900000, kSplitPairOnePassWork = 1500000;
+constexpr int64_t kSplitLargeWords = 3000000;
+constexpr int kSplitTallRows = 16384, kSplitWideRows = 8192, kSplitWideWords = 64;
+inline bool split_chosen(int batch, int m, const Plan& plan, int items = 1) {
+    if (batch < 2 || batch > kSplitMaxBatch || plan.s2_qw == 0 || plan.wr > kSplitMaxWords) return false;
+    const int64_t words = static_cast<int64_t>(m) * plan.wr, work = words * batch;
+    const int64_t passes = ceil_div(batch, s2t_rows_per_pass(batch, items * plan.s2_qw));
+    if (items == 2) {
+        if (batch <= 2) return words >= kSplitLargeWords;
+        if (batch > 16 && words >= kSplitLargeWords) return false;
+        return work >= (passes >= 2 ? kSplitPairWork : kSplitPairOnePassWork);
+    }
+    if (batch <= 8 && words >= kSplitLargeWords) return true;
+    if (passes < 2 || work < kSplitWork || (batch > 8 && m >= kSplitTallRows)) return false;
+    return batch <= 16 || (m <= kSplitWideRows && plan.wr >= kSplitWideWords);
+}
+
 template <typename T, int EPI>
 int launch_stage2_batched(const S2bCall& a) {
     const int64_t tiles = ceil_div(a.m, 16);
     if (tiles >= 512) {
-        // 640-1023 row tiles (the 11008-row gate/up factors) at 16 rows or fewer: 32-row blocks with
-        // four-word chunks (same-box, r = 1632 / 2976: 14.52 / 18.67 -> 13.93 / 17.42 us per GEMV; at
-        // 1792 tiles, Llama-3-70B gate/up, they lose 12-25%, at 512 they tie, at 24 rows they lose)
-        if (tiles >= 640 && tiles < 1024 && a.batch <= 16) return launch_s2b_cfg<T, 2, 2, 1, 4, EPI>(a);
         if (a.batch <= 64) return launch_s2b_cfg<T, 4, 4, 2, 2, EPI>(a);
         return launch_s2b_cfg<T, 4, 4, 4, 2, EPI>(a);
     }
@@ -2631,6 +2657,12 @@ int launch_stage2(const GemvArgs& a) {
     RowsPlan rp;
     if (s2t_applies(a.z_hi, a.z_lo, a.u_bits, a.m, a.plan) && rows_stage2_plan(a.batch, a.m, a.plan.wr, rp))
         return launch_stage2_rows<T>(a, rp);
+    if (s2t_applies(a.z_hi, a.z_lo, a.u_bits, a.m, a.plan) && split_chosen(a.batch, a.m, a.plan)) {
+        SplitTable tab;
+        tab.count = 1;
+        tab.item[0] = SplitItem{a.u_bits, a.s_out, a.y, nullptr, a.z_hi, a.z_lo, a.m, a.plan.wr, a.plan.zpitch, a.m, 0, 0};
+        return launch_split(dtype_code<T>(), tab, a.batch, kSplitStore, split_plan(a.batch, a.m, a.plan.wr), a.stream);
+    }
     if (s2t_applies(a.z_hi, a.z_lo, a.u_bits, a.m, a.plan) && s2b_chosen(a.batch, a.m, a.plan))
         return launch_stage2_batched<T, kEpiStore>(S2bCall{a.u_bits, a.s_out, a.y, nullptr, a.z_hi, a.z_lo, a.m, a.m,
                                                            a.batch, a.plan, a.stream});
@@ -3119,10 +3151,33 @@ int group_stage2(const char* name, int dtype, int64_t count, const nq_gemv_item*
     const int b = static_cast<int>(batch);
     hipStream_t st = as_stream(stream);
     bool done[kMaxItems] = {false, false, false, false};
+    if (rope == nullptr) {  // the rank split over a block's waves: one launch for the items that take it and, with
+        // them, the small ones left (which would need a launch of their own)
+        const int pair = epilogue == NQ_EPI_GATED ? 2 : 1;
+        SplitTable tab;
+        tab.count = 0;
+        int64_t lead = -1;  // the largest chosen item's block shape serves all
+        for (int64_t k = 0; k < count; ++k)
+            if (split_chosen(b, all[k].m, g.plan[k], pair) && (lead < 0 || all[k].m > all[lead].m)) lead = k;
+        for (int64_t k = 0; k < count && lead >= 0; ++k) {
+            if (!split_chosen(b, all[k].m, g.plan[k], pair) &&
+                (all[k].wr > kSplitMaxWords || all[k].m > all[lead].m || s2b_chosen(b, all[k].m, g.plan[k], pair)))
+                continue;
+            tab.item[tab.count++] = SplitItem{all[k].u_bits, all[k].s_out, all[k].y, all[k].resid, all[k].z_hi, all[k].z_lo,
+                                              all[k].m, all[k].wr, all[k].zpitch, all[k].ystride, 0, 0};
+            done[k] = true;
+        }
+        if (lead >= 0) {
+            const SplitEpilogue e = epilogue == NQ_EPI_STORE      ? kSplitStore
+                                    : epilogue == NQ_EPI_RESIDUAL ? kSplitResidual
+                                                                  : kSplitGated;
+            if (int s = launch_split(dtype, tab, b, e, split_plan(b, all[lead].m, all[lead].wr), st)) return s;
+        }
+    }
     if (rope == nullptr) {  // items whose batch the batched kernel serves better: a launch each
         const int pair = epilogue == NQ_EPI_GATED ? 2 : 1;
         for (int64_t k = 0; k < count; ++k) {
-            if (!s2b_chosen(b, all[k].m, g.plan[k], pair)) continue;
+            if (done[k] || !s2b_chosen(b, all[k].m, g.plan[k], pair)) continue;
             S2bCall c{all[k].u_bits, all[k].s_out, all[k].y, all[k].resid, all[k].z_hi, all[k].z_lo, all[k].m,
                       all[k].ystride, b, g.plan[k], st};
             if (pair == 2) {  // the gate into y of item 0, then up against it
