@@ -382,6 +382,25 @@ int nq_dense_gemv(int dtype, const void* w, const void* x, const void* norm_weig
  * which torch runs as its own reduction launches. */
 int nq_argmax_rows(const float* x, int64_t rows, int64_t n, int64_t ldx, int64_t* out, nq_stream_t stream);
 
+/* The end of a greedy decode step in one launch: nq_argmax_rows over the logits into tok [rows], the token stored at
+ * ids[b * max_len + *position + 1] (not stored where that is outside the row), and *position advanced by one. `counter`:
+ * four bytes of device memory, zero before the launch and zero again after it; launches that may overlap need counters
+ * and positions of their own. No counterpart in the reference (its harness does these in torch,
+ * src/nanoquant/kernel/test_decode.py:350-353). */
+int nq_decode_end(const float* logits, int64_t rows, int64_t n, int64_t ldx, int64_t* tok, int64_t* ids, int64_t max_len,
+                  int64_t* position, uint32_t* counter, nq_stream_t stream);
+
+/* The beginning of a decode step in one launch, from the step's tokens tok [batch] and *position (device memory):
+ *   x [batch][hidden] = embed[tok[b]] (zeros for a token outside [0, vocab)), unless embed is null;
+ *   with a table [max_len][row] of 16-bit elements, its row of the position into table_out (zeros outside);
+ *   with scores (scores_rows rows of [max_len][groups]), the additive causal mask: 0 for positions up to *position, -inf
+ *   past it.
+ * dtype: of embed, x and scores. hidden a multiple of 8; embed, x and scores 16-byte aligned. No counterpart in the
+ * reference (torch ops of its model). */
+int nq_decode_begin(int dtype, const void* embed, int64_t vocab, int64_t hidden, const int64_t* tok, void* x, int64_t batch,
+                    const int64_t* position, int64_t max_len, const void* table, int64_t row, void* table_out, void* scores,
+                    int64_t scores_rows, int64_t groups, nq_stream_t stream);
+
 /* ---------------------------------------------------------------- measurement aid */
 
 /* Enqueue a one-thread kernel that writes the GPU's constant-rate wall clock to *dst (device

@@ -550,11 +550,16 @@ void launch_dense_gemv(const uint16_t* w, const uint16_t* x, const uint16_t* g, 
 
 // ------------------------------------------------------------------ greedy argmax over the logits
 //
-// One block per batch row: each thread scans every kArgmaxThreads-th logit, then the wave and the
-// block reduce (value, index) pairs. The order is torch.argmax's: a NaN beats every number (the
+// One block per batch row: each thread scans its share of the logits, then the wave and the block
+// reduce (value, index) pairs. The order is torch.argmax's: a NaN beats every number (the
 // first NaN wins), otherwise the larger value, and of equal values (-0 equal to +0) the smaller
-// index, so the result is the first maximal logit. One 32000-logit row: 8.4 us graph-replayed
-// against 10.5 us for torch.argmax (a variant issuing each thread's 32 loads at once took 9.0).
+// index, so the result is the first maximal logit. The time is that of a row's loads through one
+// CU, so they are 16 bytes each and all of a 32000-logit row's in flight (in a decode step of 16 rows 13.9 us, 4 bytes
+// each, -> 10.0 with the stores below).
+//
+// step_end_kernel is the same launch with what follows the choice in a decode step: the token goes into
+// the step's input and into the sequence at the next position, and the position advances, once every row's block
+// has read it (a counter, back at zero when the launch ends).
 constexpr int kArgmaxThreads = 1024;
 
 __device__ inline bool argmax_before(float a, int ia, float b, int ib) {
@@ -563,43 +568,147 @@ __device__ inline bool argmax_before(float a, int ia, float b, int ib) {
     return a > b || (a == b && ia < ib);
 }
 
-__global__ __launch_bounds__(kArgmaxThreads) void argmax_rows_kernel(const float* __restrict__ x, int n, int64_t ldx,
-                                                                     int64_t* __restrict__ out) {
-    const float* row = x + static_cast<int64_t>(blockIdx.x) * ldx;
+// The block's choice over one row, valid in thread 0. `vec`: the row is whole and aligned 16-byte pieces.
+__device__ inline int argmax_row(const float* __restrict__ row, int n, int vec) {
     float bv = -INFINITY;
     int bi = INT32_MAX;  // loses to every element, a -inf one included (equal value, smaller index)
-#pragma unroll 8
-    for (int i = static_cast<int>(threadIdx.x); i < n; i += kArgmaxThreads) {
-        const float v = row[i];
+    auto take = [&](float v, int i) {
         if (argmax_before(v, i, bv, bi)) {
             bv = v;
             bi = i;
         }
-    }
+    };
+    const int t = static_cast<int>(threadIdx.x);
+    if (vec) {
+        constexpr int kAhead = 8;  // 16-byte loads of a thread in flight
+        const rsrc_t rs = make_rsrc(row, static_cast<uint32_t>(n) * 4u);
+        for (int base = 4 * t; base < n; base += 4 * kArgmaxThreads * kAhead) {
+            u32x4 d[kAhead];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const float ov = __shfl_xor(bv, off, 64);
-        const int oi = __shfl_xor(bi, off, 64);
-        if (argmax_before(ov, oi, bv, bi)) {
-            bv = ov;
-            bi = oi;
+            for (int u = 0; u < kAhead; ++u)  // past the row: not read (zeros), not taken
+                d[u] = load_b128(rs, 4u * static_cast<uint32_t>(base + 4 * kArgmaxThreads * u));
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                const int i = base + 4 * kArgmaxThreads * u;
+                if (i < n) {
+                    take(__uint_as_float(d[u].x), i);
+                    take(__uint_as_float(d[u].y), i + 1);
+                    take(__uint_as_float(d[u].z), i + 2);
+                    take(__uint_as_float(d[u].w), i + 3);
+                }
+            }
         }
+    } else {
+#pragma unroll 8
+        for (int i = t; i < n; i += kArgmaxThreads) take(row[i], i);
     }
-    __shared__ float wv[kArgmaxThreads / 64];
-    __shared__ int wi[kArgmaxThreads / 64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    auto reduce = [&](int from) {
+#pragma unroll
+        for (int off = from; off > 0; off >>= 1) {
+            const float ov = __shfl_xor(bv, off, 64);
+            take(ov, __shfl_xor(bi, off, 64));
+        }
+    };
+    reduce(32);
+    constexpr int kWaves = kArgmaxThreads / 64;
+    __shared__ float wv[kWaves];
+    __shared__ int wi[kWaves];
+    const int lane = t & 63;
     if (lane == 0) {
-        wv[wave] = bv;
-        wi[wave] = bi;
+        wv[t >> 6] = bv;
+        wi[t >> 6] = bi;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < kArgmaxThreads / 64; ++w)
-            if (argmax_before(wv[w], wi[w], bv, bi)) {
-                bv = wv[w];
-                bi = wi[w];
-            }
-        out[blockIdx.x] = bi;
+    if (t >= 64) return 0;
+    bv = wv[lane % kWaves];
+    bi = wi[lane % kWaves];
+    reduce(kWaves / 2);
+    return bi;
+}
+
+__global__ __launch_bounds__(kArgmaxThreads) void argmax_rows_kernel(const float* __restrict__ x, int n, int64_t ldx,
+                                                                     int vec, int64_t* __restrict__ out) {
+    const int best = argmax_row(x + static_cast<int64_t>(blockIdx.x) * ldx, n, vec);
+    if (threadIdx.x == 0) out[blockIdx.x] = best;
+}
+
+__global__ __launch_bounds__(kArgmaxThreads) void step_end_kernel(const float* __restrict__ x, int n, int64_t ldx, int vec,
+                                                                  int64_t* __restrict__ tok, int64_t* __restrict__ ids,
+                                                                  int64_t max_len, int64_t* pos, uint32_t* counter) {
+    const int64_t next = *pos + 1;
+    const int best = argmax_row(x + static_cast<int64_t>(blockIdx.x) * ldx, n, vec);
+    if (threadIdx.x != 0) return;
+    tok[blockIdx.x] = best;
+    if (next >= 0 && next < max_len) ids[static_cast<int64_t>(blockIdx.x) * max_len + next] = best;
+    // the position has been read (its value was needed above) before this block counts itself
+    if (gridDim.x > 1) {
+        wait_vmcnt<0>();
+        if (atomicAdd(counter, 1u) != gridDim.x - 1) return;
+        atomicExch(counter, 0u);
+    }
+    *pos = next;
+}
+
+// ------------------------------------------------------------------ the beginning of a decode step
+//
+// What a step prepares from its input token and position, in one launch: the token's embedding row for each
+// sequence, the rotary table's row of the position, and the causal mask in the attention scores of every layer (0 up to
+// the position, -inf past it). As torch ops these were two row selections, a comparison over the mask's size and a
+// select, 2.4 + 2.4 + 7.0 + 4.0 us for 4 layers of 32 heads (3.2 here), and the row selection of 16 tokens at hidden
+// 8192 took 10.0 (4.8 here).
+struct StepBegin {
+    const uint16_t* embed;  // [vocab][hidden]
+    const int64_t* tok;
+    uint16_t* x;  // [batch][hidden]
+    const int64_t* pos;
+    const uint16_t* table;  // [max_len][row], or nullptr
+    uint16_t* table_out;
+    uint16_t* scores;  // [scores_total], rows of max_len * groups, or nullptr
+    int64_t vocab, max_len, scores_total;
+    int hidden, row, groups;
+    int x_blocks, x_pieces;  // blocks over the embedding rows, 8-element pieces of a row
+    uint32_t minus_inf;      // a pair
+};
+constexpr int kBeginThreads = 256;
+
+__global__ __launch_bounds__(kBeginThreads) void step_begin_kernel(const StepBegin a) {
+    const int t = static_cast<int>(threadIdx.x);
+    const int block = static_cast<int>(blockIdx.x);
+    if (block < a.x_blocks) {
+        const int per_row = (a.x_pieces + kBeginThreads - 1) / kBeginThreads;
+        const int b = block / per_row;
+        const int piece = (block - b * per_row) * kBeginThreads + t;
+        const int64_t tok = a.tok[b];
+        if (piece >= a.x_pieces) return;
+        u32x4 v = u32x4{0u, 0u, 0u, 0u};  // a token outside the vocabulary
+        if (tok >= 0 && tok < a.vocab) v = *reinterpret_cast<const u32x4*>(a.embed + tok * a.hidden + 8 * piece);
+        *reinterpret_cast<u32x4*>(a.x + static_cast<int64_t>(b) * a.hidden + 8 * piece) = v;
+        return;
+    }
+    const int64_t p = *a.pos;
+    if (a.table != nullptr && block == a.x_blocks) {
+        for (int e = t; e < a.row; e += kBeginThreads)
+            a.table_out[e] = p >= 0 && p < a.max_len ? a.table[p * a.row + e] : uint16_t{0};
+        return;
+    }
+    // 8 elements of the mask a thread; scores row element e belongs to position e / groups
+    const int64_t first = block - a.x_blocks - (a.table != nullptr ? 1 : 0);
+    const int64_t e0 = (first * kBeginThreads + t) * 8;
+    if (e0 >= a.scores_total) return;
+    const int64_t period = a.max_len * a.groups, visible = (p + 1) * a.groups;
+    uint32_t at = a.scores_total <= UINT32_MAX ? static_cast<uint32_t>(e0) % static_cast<uint32_t>(period)
+                                               : static_cast<uint32_t>(e0 % period);
+    uint16_t m[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        m[k] = static_cast<int64_t>(at) < visible ? uint16_t{0} : static_cast<uint16_t>(a.minus_inf);
+        if (++at == static_cast<uint32_t>(period)) at = 0;
+    }
+    if (e0 + 8 <= a.scores_total) {
+        *reinterpret_cast<u32x4*>(a.scores + e0) = u32x4{m[0] | (uint32_t(m[1]) << 16), m[2] | (uint32_t(m[3]) << 16),
+                                                         m[4] | (uint32_t(m[5]) << 16), m[6] | (uint32_t(m[7]) << 16)};
+    } else {
+        for (int k = 0; k < 8 && e0 + k < a.scores_total; ++k) a.scores[e0 + k] = m[k];
     }
 }
 
@@ -607,6 +716,13 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_rows_kernel(const float
 }  // namespace nq
 
 using namespace nq;
+
+namespace {
+// Whether a row of logits is whole and aligned 16-byte pieces (within the 32-bit byte offsets of the kernel's loads).
+int argmax_vec(const float* x, int64_t n, int64_t ldx) {
+    return n % 4 == 0 && ldx % 4 == 0 && aligned(x, 16) && n <= INT32_MAX / 8;
+}
+}  // namespace
 
 extern "C" {
 
@@ -747,7 +863,67 @@ int nq_argmax_rows(const float* x, int64_t rows, int64_t n, int64_t ldx, int64_t
     if (!x || !out) return fail(NQ_ERR_INVALID_ARGUMENT, "%s: null pointer", name);
     if (!aligned(x, 4) || !aligned(out, 8)) return fail(NQ_ERR_ALIGNMENT, "%s: misaligned x or out", name);
     argmax_rows_kernel<<<static_cast<unsigned>(rows), kArgmaxThreads, 0, as_stream(stream)>>>(
-        x, static_cast<int>(n), ldx, out);
+        x, static_cast<int>(n), ldx, argmax_vec(x, n, ldx), out);
+    return check_launch(name);
+}
+
+int nq_decode_end(const float* logits, int64_t rows, int64_t n, int64_t ldx, int64_t* tok, int64_t* ids, int64_t max_len,
+                  int64_t* position, uint32_t* counter, nq_stream_t stream) {
+    const char* name = "nq_decode_end";
+    if (rows < 0 || n <= 0 || ldx < n || max_len <= 0)
+        return fail(NQ_ERR_INVALID_ARGUMENT, "%s: bad sizes (rows %lld, n %lld, ldx %lld, max_len %lld)", name,
+                    (long long)rows, (long long)n, (long long)ldx, (long long)max_len);
+    if (n > INT32_MAX / 4 || rows > 65535 * 32 || rows * max_len > ((int64_t)1 << 40))
+        return fail(NQ_ERR_UNSUPPORTED, "%s: sizes too large", name);
+    if (rows == 0) return NQ_OK;
+    if (!logits || !tok || !ids || !position || !counter) return fail(NQ_ERR_INVALID_ARGUMENT, "%s: null pointer", name);
+    if (!aligned(logits, 4) || !aligned(tok, 8) || !aligned(ids, 8) || !aligned(position, 8) || !aligned(counter, 4))
+        return fail(NQ_ERR_ALIGNMENT, "%s: misaligned operand", name);
+    step_end_kernel<<<static_cast<unsigned>(rows), kArgmaxThreads, 0, as_stream(stream)>>>(
+        logits, static_cast<int>(n), ldx, argmax_vec(logits, n, ldx), tok, ids, max_len, position, counter);
+    return check_launch(name);
+}
+
+int nq_decode_begin(int dtype, const void* embed, int64_t vocab, int64_t hidden, const int64_t* tok, void* x, int64_t batch,
+                    const int64_t* position, int64_t max_len, const void* table, int64_t row, void* table_out, void* scores,
+                    int64_t scores_rows, int64_t groups, nq_stream_t stream) {
+    const char* name = "nq_decode_begin";
+    if (dtype != NQ_F16 && dtype != NQ_BF16) return fail(NQ_ERR_DTYPE, "%s: unsupported dtype %d", name, dtype);
+    if (batch < 0 || vocab <= 0 || hidden <= 0 || max_len <= 0 || (table && row <= 0) || (scores && (scores_rows < 0 || groups <= 0)))
+        return fail(NQ_ERR_INVALID_ARGUMENT, "%s: bad sizes", name);
+    if (hidden % 8) return fail(NQ_ERR_SHAPE, "%s: hidden must be a multiple of 8, got %lld", name, (long long)hidden);
+    const int64_t pieces = hidden / 8, x_blocks = embed ? batch * ceil_div(pieces, kBeginThreads) : 0;
+    if (hidden > INT32_MAX / 4 || vocab * hidden > ((int64_t)1 << 40) || batch > 65535 * 32 || x_blocks > INT32_MAX / 4 ||
+        (table && (row > INT32_MAX / 4 || max_len * row > ((int64_t)1 << 40))) ||
+        (scores && (groups > 65535 || max_len * groups > INT32_MAX / 4 || scores_rows > INT32_MAX / 4 ||
+                    scores_rows * max_len * groups > ((int64_t)1 << 38))))
+        return fail(NQ_ERR_UNSUPPORTED, "%s: sizes too large", name);
+    if (batch == 0) return NQ_OK;
+    if (!position || (embed && (!tok || !x)) || (table && !table_out)) return fail(NQ_ERR_INVALID_ARGUMENT, "%s: null pointer", name);
+    if (!aligned(embed, 16) || !aligned(x, 16) || !aligned(tok, 8) || !aligned(position, 8) || !aligned(table, 2) ||
+        !aligned(table_out, 2) || !aligned(scores, 16))
+        return fail(NQ_ERR_ALIGNMENT, "%s: misaligned operand (embed, x and scores need 16 bytes)", name);
+    StepBegin a{};
+    a.embed = static_cast<const uint16_t*>(embed);
+    a.tok = tok;
+    a.x = static_cast<uint16_t*>(x);
+    a.pos = position;
+    a.table = static_cast<const uint16_t*>(table);
+    a.table_out = static_cast<uint16_t*>(table_out);
+    a.scores = static_cast<uint16_t*>(scores);
+    a.vocab = vocab;
+    a.max_len = max_len;
+    a.groups = scores ? static_cast<int>(groups) : 1;
+    a.scores_total = scores ? scores_rows * max_len * groups : 0;
+    a.hidden = static_cast<int>(hidden);
+    a.row = static_cast<int>(row);
+    a.x_blocks = static_cast<int>(x_blocks);
+    a.x_pieces = static_cast<int>(pieces);
+    a.minus_inf = dtype == NQ_F16 ? 0xFC00u : 0xFF80u;
+    const int64_t blocks = x_blocks + (table ? 1 : 0) + ceil_div(a.scores_total, 8 * kBeginThreads);
+    if (blocks == 0) return NQ_OK;
+    if (blocks > INT32_MAX / 2) return fail(NQ_ERR_UNSUPPORTED, "%s: sizes too large", name);
+    step_begin_kernel<<<static_cast<unsigned>(blocks), kBeginThreads, 0, as_stream(stream)>>>(a);
     return check_launch(name);
 }
 

@@ -599,8 +599,8 @@ class FusedDecoder(GraphDecoder):
     3. rotary embedding, KV-cache write and attention: in torch ops (``attention="torch"``, the
        default, as the benchmark's end-to-end configuration keeps the non-linear ops in
        PyTorch; step 2 then also writes the value row into its cache,
-       ``nq_gemv_group_stage2_kv``, and the step's causal mask goes into every layer's scores
-       buffer in one launch per step), or the rotary embedding and cache write folded into step
+       ``nq_gemv_group_stage2_kv``, and the step's causal mask is in every layer's scores
+       buffer from the step's first launch), or the rotary embedding and cache write folded into step
        2's stores (``nq_gemv_group_stage2_rope``) and the attention products in torch
        (``attention="rope"``), or all of it in one HIP launch pair (``attention="hip"``,
        ``nq_attention_decode``);
@@ -610,8 +610,9 @@ class FusedDecoder(GraphDecoder):
     8, 9. down_proj, its stage 2 adding the residual.
     The final norm and the lm_head run as one dense GEMV of the library (``nq_dense_gemv`` with
     its RMS-norm prologue: torch's linear reads the head's weights, cold after the layers, at a
-    fraction of the bandwidth), which writes the float32 logits; the embedding lookup and argmax
-    stay torch ops. The logits a step returns live in a buffer the next step overwrites. Prefill runs the unfused model (it fills the same cache
+    fraction of the bandwidth), which writes the float32 logits. One launch before the layers looks up
+    the embeddings and prepares the position's rotary row and mask (``nq_decode_begin``), one after the
+    head takes the argmax and advances the position (``nq_decode_end``). The logits a step returns live in a buffer the next step overwrites. Prefill runs the unfused model (it fills the same cache
     layout). Needs the model packed for the ``gemv`` kernel in float16 or bfloat16 and head_dim 128.
     """
 
@@ -647,8 +648,8 @@ class FusedDecoder(GraphDecoder):
         # attention scores of the rope step [B * KV, L, G]: the q/k/v launch writes the step's causal
         # mask into it, the scores product adds into it in place
         self.scores = torch.zeros(batch * KV, max_len, H // KV, device=dev, dtype=dt)
-        # the torch step's scores, one buffer per layer: the step's causal mask is copied into all of
-        # them by one launch, and each layer's scores product adds into its own in place
+        # the torch step's scores, one buffer per layer: the step's causal mask is written into all of
+        # them by its first launch, and each layer's scores product adds into its own in place
         self.scores_all = (torch.zeros(s.layers, batch * KV, max_len, H // KV, device=dev, dtype=dt)
                            if attention == "torch" else None)
         head = model.lm_head
@@ -665,8 +666,10 @@ class FusedDecoder(GraphDecoder):
         self.act = torch.zeros(batch, s.ffn, device=dev, dtype=dt)
         cos, sin = model.rope(torch.arange(max_len, device=dev), dt)
         self.rope_cos, self.rope_sin = cos.contiguous(), sin.contiguous()
-        self.rope_cs = torch.stack((self.rope_cos, self.rope_sin), dim=1).contiguous()  # [max_len, 2, D]
+        # the torch step's rotary table: row p holds position p's cos and sin
+        self.rope_table = torch.cat((self.rope_cos, self.rope_sin), dim=1).contiguous()  # [max_len, 2 D]
         self.tok = torch.zeros(batch, dtype=torch.long, device=dev)  # the step's input token ids
+        self.counter = torch.zeros(1, dtype=torch.int32, device=dev)  # nq_decode_end's, zero between launches
         self.step_consts = step_constants(D, dt, dev)
         # the torch step in float16 rotates q and k as one complex product: their features in pair
         # order (feature j of a head, then j + D/2, ...), the cache's keys too (dot products do not
@@ -677,9 +680,10 @@ class FusedDecoder(GraphDecoder):
             self.head_order = (j // 2) + (j % 2) * (D // 2)  # position i of a head holds feature head_order[i]
             self.q_order = (torch.arange(H, device=dev)[:, None] * D + self.head_order).reshape(-1)
             self.k_order = (torch.arange(KV, device=dev)[:, None] * D + self.head_order).reshape(-1)
-            half = torch.stack((self.rope_cos[:, : D // 2], self.rope_sin[:, : D // 2]), dim=-1).contiguous()
-            self.rope_freqs = torch.view_as_complex(half)  # [max_len, D / 2] complex32: cos + i sin
+            half = torch.stack((self.rope_cos[:, : D // 2], self.rope_sin[:, : D // 2]), dim=-1)
+            self.rope_table = half.reshape(max_len, D).contiguous()  # cos + i sin, D / 2 complex pairs
             self.rot = torch.zeros(batch, H + KV, D, device=dev, dtype=dt)
+        self.rope_row = torch.zeros(self.rope_table.shape[1], device=dev, dtype=dt)  # the step's row of it
         self._keep = []  # tensors whose addresses the item tables hold
         self.plans = [self._layer_plan(layer) for layer in model.model.layers]
         need = 0
@@ -788,15 +792,23 @@ class FusedDecoder(GraphDecoder):
         H, KV, D = s.heads, s.kv_heads, s.head_dim
         dt, ws, wsb = self.dcode, self.ws.data_ptr(), self.ws.numel()
         st = self._lib.stream_of(self.device)
-        torch.index_select(self.model.model.embed_tokens.weight, 0, self.tok, out=self.x)
+        # the embedding rows and, for the torch attention, the position's rotary row and causal mask
+        embed = self.model.model.embed_tokens.weight
+        plain = embed.dtype == self.x.dtype and embed.is_contiguous() and embed.data_ptr() % 16 == 0 and embed.device == self.x.device
+        if not plain:
+            torch.index_select(embed, 0, self.tok, out=self.x)
+        table, scores = (self.rope_table, self.scores_all) if self.attention == "torch" else (None, None)
+        self._check(lib.nq_decode_begin(
+            dt, embed.data_ptr() if plain else None, embed.shape[0], s.hidden, self.tok.data_ptr(), self.x.data_ptr(), B, self.pos.data_ptr(),
+            self.max_len, self._lib.ptr(table), 0 if table is None else table.shape[1], self.rope_row.data_ptr(),
+            self._lib.ptr(scores), 0 if scores is None else s.layers * B * KV, H // KV, st), "step begin")
         if self.attention == "torch":
             if self.pair_order:
-                freqs = self.rope_freqs.index_select(0, self.pos)  # [1, D / 2]: cos + i sin of the position
+                freqs = torch.view_as_complex(self.rope_row.view(1, D // 2, 2))  # cos + i sin of the position
             else:
-                cs = self.rope_cs.index_select(0, self.pos)  # [1, 2, D]: cos, sin of the position
+                cs = self.rope_row.view(1, 2, D)  # cos, sin of the position
                 tables = rotary_step_tables(cs[:, 0], cs[:, 1], self.pos, self.cache, self.model.dtype,
                                             with_mask=False, consts=self.step_consts)
-            step_mask(self.pos, self.cache, self.step_consts[2], out=self.scores_all)
         x, h, qkv, attn, act = (t.data_ptr() for t in (self.x, self.h, self.qkv, self.attn, self.act))
         esz = self.qkv.element_size()
         for li, plan in enumerate(self.plans):
@@ -839,10 +851,9 @@ class FusedDecoder(GraphDecoder):
             self._check(lib.nq_gemv_group_stage2(dt, n, items, B, self._lib.NQ_EPI_GATED, ws, wsb, st), "gu 2")
             self._linear_residual(plan["down"], act, s.ffn, st, "down")
         logits = self._head(self.x, self.logits if self.head_bias is None else self.logits16, st)
-        self._check(lib.nq_argmax_rows(logits.data_ptr(), B, logits.shape[1], logits.stride(0), self.tok.data_ptr(),
-                                       st), "argmax")
-        self.pos.add_(1)
-        self.ids.index_copy_(1, self.pos, self.tok.view(-1, 1))
+        self._check(lib.nq_decode_end(logits.data_ptr(), B, logits.shape[1], logits.stride(0), self.tok.data_ptr(),
+                                      self.ids.data_ptr(), self.max_len, self.pos.data_ptr(), self.counter.data_ptr(), st),
+                    "step end")
         return logits
 
     @torch.no_grad()
