@@ -17,8 +17,10 @@
 //
 // The scores never reach memory: at 2048 tokens and 32 heads the torch path writes and reads them (256 MB
 // in T, 512 MB in fp32) eight times over. What bounds this kernel is issue: per tile and wave 32 MFMAs
-// (1024 cycles) and about as many VALU cycles for 32 exponentials and the packing of P^T, which two waves
-// per SIMD overlap. A block's K tile arrives by DMA (16-byte chunk p of row r holds the row's chunk
+// (1024 cycles) and 1500 cycles of VALU (32 exponentials take a third) in 5100 measured ones, a quarter of
+// them waits; a SIMD's two waves overlap while both have keys left. Reading operands four ahead of the MFMAs,
+// rescaling only when the maximum has grown by kSlack and loads through a uniform descriptor took 2048
+// tokens of 32 heads from 73.8 to 60.2 us (2 x 333 tokens, 64 heads over 8, 22.2 to 20.2). A block's K tile arrives by DMA (16-byte chunk p of row r holds the row's chunk
 // p ^ (r % 16)), its V tile through registers, transposed four keys at a time; both go into the buffer
 // that the tile after the current one reads.
 #include <algorithm>
@@ -31,6 +33,7 @@ namespace {
 constexpr int D = 128;
 constexpr int kRowsPerBlock = 128;
 constexpr int kKeys = 64;
+constexpr float kSlack = 8.0f;
 
 struct AttnArgs {
     const uint16_t* q;
@@ -117,14 +120,18 @@ __device__ inline uint32_t pack2(float a, float b) {
     return static_cast<uint32_t>(T::from_float(a)) | (static_cast<uint32_t>(T::from_float(b)) << 16);
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void prefill_attn_kernel(const AttnArgs a) {
-    __shared__ __attribute__((aligned(16))) uint16_t ks[2][kKeys * D];
-    __shared__ __attribute__((aligned(16))) uint16_t vt[2][D * kKeys];
+template <typename T, int KS>
+__global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(2))) void prefill_attn_kernel(const AttnArgs a) {
+    static_assert(KS == 1 || KS == 2, "one or two groups of waves");
+    __shared__ __attribute__((aligned(16))) uint16_t ksall[KS][2][kKeys * D];
+    __shared__ __attribute__((aligned(16))) uint16_t vtall[KS][2][D * kKeys];
     __shared__ int lims[4];
-    const int t = threadIdx.x;
+    const int grp = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);  // key group
+    const int t = static_cast<int>(threadIdx.x) & 255;
+    auto& ks = ksall[grp];
+    auto& vt = vtall[grp];
     const int lane = t & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);  // of its group
     const int c = lane & 31;
     const int kg = lane >> 5;
     const int heads = a.batch * a.kv_heads;
@@ -133,7 +140,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
     // way round, so that a CU gets a long block and a short one.
     const int n_tiles = static_cast<int>(gridDim.x) / heads;
     const int order = static_cast<int>(blockIdx.x) / heads;
-    const int tile = gridDim.x <= 512u && 2 * order >= n_tiles ? order - (n_tiles + 1) / 2 : n_tiles - 1 - order;
+    const int tile = KS == 1 && gridDim.x <= 512u && 2 * order >= n_tiles ? order - (n_tiles + 1) / 2 : n_tiles - 1 - order;
     const int bh = static_cast<int>(blockIdx.x) % heads;
     const int b = bh / a.kv_heads;
     const int kvh = bh - b * a.kv_heads;
@@ -157,6 +164,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
             rotate8<T>(qf[kt], qf[kt + 4], *vec(a.cos + tab + 16 * kt), *vec(a.sin + tab + 16 * kt),
                        *vec(a.cos + tab + 16 * kt + 64), *vec(a.sin + tab + 16 * kt + 64));
     }
+    // a positive factor, so that the largest product is the largest score: the queries take a negative
+    // factor's sign, and are zero for a factor of zero
+    const float scale = a.scale == 0.0f ? 1.0f : fabsf(a.scale);
+    if (!(a.scale > 0.0f)) {
+        const uint32_t keep = a.scale == 0.0f ? 0u : 0xffffffffu, flip = a.scale < 0.0f ? 0x80008000u : 0u;
+#pragma unroll
+        for (int kt = 0; kt < 8; ++kt)
+            qf[kt] = u32x4{(qf[kt].x ^ flip) & keep, (qf[kt].y ^ flip) & keep, (qf[kt].z ^ flip) & keep,
+                           (qf[kt].w ^ flip) & keep};
+    }
     // the last visible position of the wave's rows and of the block's, and the first row's
     int wmax = lim, wmin = R0 + c < rows ? lim : a.max_len;
 #pragma unroll
@@ -166,9 +183,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
     }
     wmax = __builtin_amdgcn_readfirstlane(wmax);
     wmin = __builtin_amdgcn_readfirstlane(wmin);
-    if (lane == 0) lims[wave] = wmax;
+    if (grp == 0 && lane == 0) lims[wave] = wmax;
     __syncthreads();
-    const int last = max(max(lims[0], lims[1]), max(lims[2], lims[3]));
+    const int last = __builtin_amdgcn_readfirstlane(max(max(lims[0], lims[1]), max(lims[2], lims[3])));
     const int tiles = last / kKeys + 1;  // one (all masked) where every position is below 0
 
     const size_t head = static_cast<size_t>(bh) * a.max_len * D;
@@ -216,17 +233,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
         for (int i = 0; i < 16; ++i) o[dt][i] = 0.0f;
     float m = -__builtin_huge_valf(), l = 0.0f;
 
-    load_v(0);
-    issue_k(0, 0);
+    // group g takes tiles g, g + KS, ...; all groups run the rounds of the longest (the barriers are the
+    // block's), a tile past the last one being loaded (keys clamped, values zero) and not computed
+    const int rounds = (tiles + KS - 1) / KS;
+    load_v(grp);
+    issue_k(grp, 0);
     wait_vmcnt<0>();
     store_v(0);
     barrier_keep_dma();
-    for (int it = 0; it < tiles; ++it) {
-        const int buf = it & 1;
-        const bool more = it + 1 < tiles;
+    for (int round = 0; round < rounds; ++round) {
+        const int it = round * KS + grp;
+        const int buf = round & 1;
+        const bool more = round + 1 < rounds;
         if (more) {
-            load_v(it + 1);
-            issue_k(it + 1, buf ^ 1);
+            load_v(it + KS);
+            issue_k(it + KS, buf ^ 1);
         }
         __builtin_amdgcn_sched_barrier(0);
         const int key0 = it * kKeys;
@@ -237,53 +258,82 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
 #pragma unroll
                 for (int i = 0; i < 16; ++i) s[h][i] = 0.0f;
             const uint16_t* kb = &ks[buf][c * D];
+            // operands are read four ahead of the four MFMAs that run; left to itself the compiler reads two and
+            // waits for them
+            u32x4 kf[2][4], vf[2][4];
+            auto read_k = [&](int g) {
 #pragma unroll
-            for (int kt = 0; kt < 8; ++kt)
+                for (int e = 0; e < 4; ++e)
+                    kf[g & 1][e] = *vec(kb + 32 * (e & 1) * D + 8 * ((2 * (2 * g + (e >> 1)) + kg) ^ (c & 15)));
+            };
+            auto read_v = [&](int kt) {
+#pragma unroll
+                for (int dt = 0; dt < 4; ++dt) {
+                    const int d = 32 * dt + c;
+                    vf[kt & 1][dt] = *vec(&vt[buf][d * kKeys + 8 * ((2 * kt + kg) ^ vswz(d))]);
+                }
+            };
+            read_k(0);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                if (g < 3) read_k(g + 1);
+                else read_v(0);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[e & 1] = mfma32x32x16<T>(kf[g & 1][e], qf[2 * g + (e >> 1)], s[e & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            const bool masked = key0 + kKeys - 1 > wmin;
+            if (masked) {
 #pragma unroll
                 for (int h = 0; h < 2; ++h)
-                    s[h] = mfma32x32x16<T>(*vec(kb + 32 * h * D + 8 * ((2 * kt + kg) ^ (c & 15))), qf[kt], s[h]);
-            const bool masked = key0 + kKeys - 1 > wmin;
+#pragma unroll
+                    for (int i = 0; i < 16; ++i)
+                        if (key0 + 32 * h + 8 * (i >> 2) + 4 * kg + (i & 3) > lim) s[h][i] = -__builtin_huge_valf();
+            }
             float mt = -__builtin_huge_valf();
 #pragma unroll
             for (int h = 0; h < 2; ++h)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    float v = s[h][i] * a.scale;
-                    if (masked && key0 + 32 * h + 8 * (i >> 2) + 4 * kg + (i & 3) > lim) v = -__builtin_huge_valf();
-                    s[h][i] = v;
-                    mt = fmaxf(mt, v);
-                }
-            mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-            const float mn = fmaxf(m, mt);
-            const float mu = mn == -__builtin_huge_valf() ? 0.0f : mn;  // a row with nothing visible yet
-            const float alpha = __builtin_amdgcn_exp2f(m - mu);
-            m = mn;
-            float sum = 0.0f;
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    s[h][i] = __builtin_amdgcn_exp2f(s[h][i] - mu);
-                    sum += s[h][i];
-                }
-            l = l * alpha + sum;
-            if (__any(alpha != 1.0f)) {
+                for (int i = 0; i < 16; ++i) mt = fmaxf(mt, s[h][i]);
+            mt = fmaxf(mt, __shfl_xor(mt, 32, 64)) * scale;
+            // the reference point of the exponentials follows the running maximum only once that is 8 above
+            // it: exponentials up to 2^8 round the same, and most tiles rescale nothing
+            if (__any(mt > m + kSlack)) {
+                const float mn = fmaxf(m, mt);
+                const float alpha = __builtin_amdgcn_exp2f(m - (mn == -__builtin_huge_valf() ? 0.0f : mn));
+                m = mn;
+                l *= alpha;
 #pragma unroll
                 for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
                     for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
             }
+            const float mu = m == -__builtin_huge_valf() ? 0.0f : m;  // a row with nothing visible yet
+            float sum = 0.0f;
 #pragma unroll
-            for (int kt = 0; kt < 4; ++kt) {
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    s[h][i] = __builtin_amdgcn_exp2f(fmaf(s[h][i], scale, -mu));
+                    sum += s[h][i];
+                }
+            l += sum;
+            auto pack_p = [&](int kt) {
                 const f32x16& p = s[kt >> 1];
                 const int i0 = 8 * (kt & 1);
-                const u32x4 pf = u32x4{pack2<T>(p[i0], p[i0 + 1]), pack2<T>(p[i0 + 2], p[i0 + 3]),
-                                       pack2<T>(p[i0 + 4], p[i0 + 5]), pack2<T>(p[i0 + 6], p[i0 + 7])};
+                return u32x4{pack2<T>(p[i0], p[i0 + 1]), pack2<T>(p[i0 + 2], p[i0 + 3]),
+                             pack2<T>(p[i0 + 4], p[i0 + 5]), pack2<T>(p[i0 + 6], p[i0 + 7])};
+            };
+            u32x4 pf = pack_p(0);
 #pragma unroll
-                for (int dt = 0; dt < 4; ++dt) {
-                    const int d = 32 * dt + c;
-                    o[dt] = mfma32x32x16<T>(*vec(&vt[buf][d * kKeys + 8 * ((2 * kt + kg) ^ vswz(d))]), pf, o[dt]);
-                }
+            for (int kt = 0; kt < 4; ++kt) {
+                if (kt < 3) read_v(kt + 1);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int dt = 0; dt < 4; ++dt) o[dt] = mfma32x32x16<T>(vf[kt & 1][dt], pf, o[dt]);
+                if (kt < 3) pf = pack_p(kt + 1);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
         if (more) {
@@ -292,12 +342,36 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
         }
         barrier_keep_dma();
     }
+    if constexpr (KS == 2) {  // group 1's sums join group 0's through the K buffers, its m and l behind 32 KB of V's
+        float* red = reinterpret_cast<float*>(&ksall[0][0][0]);
+        float* stat = reinterpret_cast<float*>(&vtall[1][0][0]);
+        static_assert(sizeof(ksall) >= 64 * 256 * 4, "the K buffers hold a group's sums");
+        if (grp == 1) {
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) red[(16 * dt + i) * 256 + t] = o[dt][i];
+            stat[t] = m;
+            stat[256 + t] = l;
+        }
+        __syncthreads();
+        if (grp == 1) return;
+        const float m1 = stat[t];
+        const float mn = fmaxf(m, m1);
+        const float mu = mn == -__builtin_huge_valf() ? 0.0f : mn;
+        const float a0 = __builtin_amdgcn_exp2f(m - mu), a1 = __builtin_amdgcn_exp2f(m1 - mu);
+        l = l * a0 + stat[256 + t] * a1;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) o[dt][i] = o[dt][i] * a0 + red[(16 * dt + i) * 256 + t] * a1;
+    }
     l += __shfl_xor(l, 32, 64);
     const float inv = 1.0f / l;
 
-    // the wave's rows through LDS (its quarter of the K buffers, 16-byte chunk ch of row r at ch ^ (r % 16)),
+    // the wave's rows through LDS (its 8 KB of the V buffers, 16-byte chunk ch of row r at ch ^ (r % 16)),
     // then whole 256-byte rows to memory
-    uint16_t* ob = &ks[0][0] + wave * 4096;
+    uint16_t* ob = &vtall[0][0][0] + wave * 4096;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
@@ -318,12 +392,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
     }
 }
 
+// Two groups of waves share a block's keys where the grid leaves a CU one block at most and its longest block
+// walks over twelve tiles or more (the host does not know the positions, only that the last token sees at
+// least the others): both launches, fp16, us, one group / two: 32 heads at 1000 tokens 43.1 / 40.4, 16 at 2000
+// 62.2 / 53.5, 8 at 2000 57.6 / 48.2. Shorter chains do not pay for the joining of the groups (32 heads at 64
+// tokens 12.7 / 15.5, two sequences of 512 32.8 / 33.5), and with two blocks to a CU these overlap better than
+// two groups that meet at one barrier (32 heads at 2048 tokens, this launch alone, 60.2 / 62.5; 336 blocks of
+// grouped heads 20.2 / 27.3).
+constexpr int64_t kSplitBlocks = 256, kSplitTokens = 768;
+
 template <typename T>
 void launch_prefill(const AttnArgs& a, hipStream_t st) {
     const int64_t kv_threads = static_cast<int64_t>(a.batch) * a.tokens * a.kv_heads * 16;
     kv_rows_kernel<T><<<dim3(static_cast<unsigned>(ceil_div(kv_threads, 256))), 256, 0, st>>>(a);
     const int64_t tiles = ceil_div(static_cast<int64_t>(a.tokens) * a.groups, kRowsPerBlock);
-    prefill_attn_kernel<T><<<dim3(static_cast<unsigned>(tiles * a.batch * a.kv_heads)), 256, 0, st>>>(a);
+    const int64_t blocks = tiles * a.batch * a.kv_heads;
+    if (blocks <= kSplitBlocks && a.tokens >= kSplitTokens)
+        prefill_attn_kernel<T, 2><<<dim3(static_cast<unsigned>(blocks)), 512, 0, st>>>(a);
+    else
+        prefill_attn_kernel<T, 1><<<dim3(static_cast<unsigned>(blocks)), 256, 0, st>>>(a);
 }
 
 }  // namespace

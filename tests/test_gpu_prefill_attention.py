@@ -11,9 +11,11 @@ from nanoquant_amd.decode import LlamaShape, StaticKVCache, rotary_attention
 pytestmark = pytest.mark.gpu
 
 # (heads, kv_heads, batch, tokens, past): fewer rows than a wave's, one row past a block, one key past a tile,
-# groups that do not divide a block, a chunk after a context, several blocks a head
+# groups that do not divide a block, a chunk after a context, several blocks a head; keys shared by two groups of
+# waves (few blocks of 768 tokens or more), with an odd number of tiles; more than one and two blocks a CU
 CASES = [(4, 4, 1, 2, 0), (4, 4, 2, 33, 0), (8, 2, 2, 64, 1), (8, 1, 1, 129, 63), (6, 2, 3, 65, 64), (5, 1, 1, 300, 0),
-         (2, 2, 1, 129, 511), (16, 2, 1, 700, 200)]
+         (2, 2, 1, 129, 511), (16, 2, 1, 700, 200), (2, 1, 1, 768, 0), (4, 2, 2, 800, 31), (1, 1, 1, 1025, 0), (16, 16, 2, 1030, 0),
+         (16, 16, 4, 1030, 0)]
 
 
 def _inputs(case, dtype, gap=37):
@@ -121,6 +123,28 @@ def test_prefill_attention_leaves_other_calls_to_torch(torch_ops):
     with FakeTensorMode(allow_non_fake_inputs=True):
         seen.append(takes(q, k, v, *tail))
     assert seen == [False, False, False]
+
+
+@pytest.mark.parametrize("tokens", [70, 800])
+@pytest.mark.parametrize("scale", [-0.09, 0.0, 3.0])
+def test_prefill_attention_scales(scale, tokens):
+    """Any factor of the scores, zero (the mean of the visible values) and negative ones too. P is rounded to float16
+    (2^-11 of each term) and so is the output: the error stays below 2^-10 of the result's norm, but that a large
+    factor makes the sum of rounded keys' errors count; the reference rounds them alike."""
+    from nanoquant_amd import _lib
+    shape, q, k, v, cos, sin, pos, cache = _inputs((2, 1, 1, tokens, 9), torch.float16)
+    out = torch.empty_like(q)
+    args = [t.data_ptr() for t in (cache.k[0], cache.v[0], cos, sin, pos, out)]
+    _lib.check(_lib.load().nq_attention_prefill(
+        _lib.NQ_F16, q.data_ptr(), 256, k.data_ptr(), 128, v.data_ptr(), 128, *args, 1, tokens, 2, 1, 128,
+        cache.k[0].shape[2], scale, _lib.stream_of(q.device)), "prefill")
+    split = q.view(1, tokens, 2, 128).transpose(1, 2)
+    rot = (split * cos) + torch.cat((-split[..., 64:], split[..., :64]), -1) * sin  # rounded as the kernel rounds
+    kc, vc = cache.k[0].double().cpu(), cache.v[0].double().cpu()
+    s = rot.double().cpu() @ kc.repeat_interleave(2, 1).transpose(2, 3).contiguous() * scale
+    hidden = torch.arange(kc.shape[2]) > pos.cpu().view(-1, 1)
+    ref = torch.softmax(s.masked_fill(hidden, -math.inf), -1) @ vc.repeat_interleave(2, 1)
+    assert _error(out.cpu(), ref.transpose(1, 2).reshape(1, tokens, 256)) <= 2 ** -10
 
 
 def test_prefill_attention_argument_errors():
