@@ -14,7 +14,7 @@
 //   3. per head: m = max_j s, e_j = exp(s_j - m), l = sum_j e_j (fp32);
 //   4. o[g][d] = sum_j e_j v[j][d] (fp32; lane pairs of d, waves over j, values loaded ahead);
 //   5. writes (m, l, o) to the workspace.
-// A second launch (attn_combine_kernel, one block per sequence and kv head) combines the chunks:
+// A second launch (attn_combine_kernel, one block per sequence and query head) combines the chunks:
 // M = max m, L = sum l exp(m - M), out = T(sum o exp(m - M) / L). (Combining inside the first
 // launch, by the last block to finish, needs device-scope fences, which write back the L2 of
 // each XCD and cost more than the second launch.)
@@ -235,54 +235,54 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(
     if (t < 2 * G) mypart[t] = mls[t >> 1][t & 1];
 }
 
-// Combine the chunks of one (sequence, kv head): thread e < G * 128 takes output element e.
+// Combine the chunks of one (sequence, query head): thread d takes output element d. What bounds it is latency:
+// the position, then one round of loads per R chunks. One block per (sequence, kv head) made its threads go
+// through the G heads one after the other, a round each (16 sequences, 64 heads over 8, 500 positions: 8.2 -> 4.9 us).
 template <typename T, int G>
-__global__ __launch_bounds__(kAttnThreads) void attn_combine_kernel(const float* __restrict__ parts,
-                                                                    const int64_t* __restrict__ position,
-                                                                    uint16_t* __restrict__ out, int kv_heads,
-                                                                    int max_len) {
+__global__ __launch_bounds__(kHeadDim) void attn_combine_kernel(const float* __restrict__ parts,
+                                                               const int64_t* __restrict__ position,
+                                                               uint16_t* __restrict__ out, int kv_heads, int max_len) {
     constexpr int D = kHeadDim;
     constexpr int PF = G * (2 + D);
     const int64_t p64 = *position;
     if (p64 < 0 || p64 >= max_len) return;  // the first launch wrote zeros
     const int n_chunks = (max_len + kChunk - 1) / kChunk;
     const int used = static_cast<int>(p64) / kChunk + 1;  // chunks holding positions <= p
-    const int bh = blockIdx.x;
+    const int bh = static_cast<int>(blockIdx.x) / G;
+    const int g = static_cast<int>(blockIdx.x) - bh * G;
     const int b = bh / kv_heads;
     const int kvh = bh - b * kv_heads;
     uint16_t* orow = out + (static_cast<size_t>(b) * kv_heads * G + static_cast<size_t>(kvh) * G) * D;
     const float* hp = parts + static_cast<size_t>(bh) * n_chunks * PF;
     constexpr int R = 16;  // chunks whose partials are loaded together
-    for (int e = threadIdx.x; e < G * D; e += kAttnThreads) {
-        const int g = e / D;
-        float M = -INFINITY, L = 0.0f, O = 0.0f;  // running combination
-        for (int c0 = 0; c0 < used; c0 += R) {
-            float m[R], l[R], o[R];
+    const int e = g * D + static_cast<int>(threadIdx.x);
+    float M = -INFINITY, L = 0.0f, O = 0.0f;  // running combination
+    for (int c0 = 0; c0 < used; c0 += R) {
+        float m[R], l[R], o[R];
 #pragma unroll
-            for (int i = 0; i < R; ++i) {
-                const int c = min(c0 + i, used - 1);
-                m[i] = hp[c * PF + 2 * g];
-                l[i] = hp[c * PF + 2 * g + 1];
-                o[i] = hp[c * PF + 2 * G + e];
-            }
-            float bm = M;
-#pragma unroll
-            for (int i = 0; i < R; ++i) bm = fmaxf(bm, m[i]);  // clamped entries repeat a used chunk
-            const float scale = expf(M - bm);  // 0 on the first batch (M = -inf, bm finite)
-            L *= scale;
-            O *= scale;
-#pragma unroll
-            for (int i = 0; i < R; ++i) {
-                if (c0 + i < used) {
-                    const float f = expf(m[i] - bm);
-                    L = fmaf(l[i], f, L);
-                    O = fmaf(o[i], f, O);
-                }
-            }
-            M = bm;
+        for (int i = 0; i < R; ++i) {
+            const int c = min(c0 + i, used - 1);
+            m[i] = hp[c * PF + 2 * g];
+            l[i] = hp[c * PF + 2 * g + 1];
+            o[i] = hp[c * PF + 2 * G + e];
         }
-        orow[e] = T::from_float(O / L);
+        float bm = M;
+#pragma unroll
+        for (int i = 0; i < R; ++i) bm = fmaxf(bm, m[i]);  // clamped entries repeat a used chunk
+        const float scale = expf(M - bm);  // 0 on the first batch (M = -inf, bm finite)
+        L *= scale;
+        O *= scale;
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            if (c0 + i < used) {
+                const float f = expf(m[i] - bm);
+                L = fmaf(l[i], f, L);
+                O = fmaf(o[i], f, O);
+            }
+        }
+        M = bm;
     }
+    orow[e] = T::from_float(O / L);
 }
 
 // Rotary embedding and KV-cache write of one new token per sequence, for a decode step whose
@@ -352,7 +352,7 @@ void launch_attn(const void* q, const void* k, const void* v, int64_t qkv_stride
         static_cast<int>(qkv_stride), static_cast<uint16_t*>(k_cache), static_cast<uint16_t*>(v_cache),
         static_cast<const uint16_t*>(rope_cos), static_cast<const uint16_t*>(rope_sin), position,
         static_cast<uint16_t*>(out), static_cast<int>(kv_heads), static_cast<int>(max_len), scaling, parts);
-    attn_combine_kernel<T, G><<<dim3(static_cast<unsigned>(batch * kv_heads)), kAttnThreads, 0, st>>>(
+    attn_combine_kernel<T, G><<<dim3(static_cast<unsigned>(batch * kv_heads * G)), kHeadDim, 0, st>>>(
         parts, position, static_cast<uint16_t*>(out), static_cast<int>(kv_heads), static_cast<int>(max_len));
 }
 
