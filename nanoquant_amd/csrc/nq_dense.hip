@@ -3,18 +3,19 @@
 // T(g[k] * T(x[k] * rsqrt(mean(x^2) + eps))).
 //
 // W is read once from HBM whatever the batch, so the launch is bound by streaming it, provided that the
-// arithmetic stays out of the way: v_mfma_f32_16x16x32 with A = 16 rows of W x 32 k, straight from global
-// memory (lane (c, g) loads the 16 bytes of row c at k = 8 g), and B = 16 batch rows of x. The eight waves
-// of a block split k, and each keeps its slice of x in registers (NF fragments per 16 batch rows) while the
-// block walks over 16-row tiles of W (a grid of one block per CU, every grid-th tile): x is read and
-// normalised once per block, and W's loads run G fragments ahead across tile ends. The waves' partial
-// tiles meet in LDS (two buffers, one barrier per tile).
+// arithmetic stays out of the way: v_mfma_f32_16x16x32 with A = 16 rows of W x 32 k and B = 16 batch rows of
+// x. The eight waves of a block split k, and each keeps its slice of x in registers (NF fragments per 16 batch
+// rows) while the block walks over 16-row tiles of W (a grid of one block per CU, every grid-th tile): x is
+// read and normalised once per block. Each wave streams its columns of W by DMA through a ring of its own in
+// LDS, stages of four fragments, three of four stages in flight across tile ends (96 KB a CU; no wave waits
+// for another). The waves' partial tiles meet in LDS (two buffers, one barrier per tile).
 //
-// Measured (MI355X, cold weights, 32000 rows, norm prologue, float32 out; us of the VALU kernel, which takes
-// up to four batch rows a pass over W, and of this one): n = 4096 at 3 / 8 / 16 / 32 rows 86 / 53, 131 / 55,
-// 239 / 57, 470 / 66; n = 8192 at 3 / 8 / 16 rows 164 / 101, 316 / 104, 608 / 111 (524 MB: 4.7 TB/s).
-// Sixteen fragments in flight instead of eight were slower (4096: 71, the registers of a second wave gone),
-// loads without the non-temporal hint too from n = 4096 on (8192: 119).
+// Measured (MI355X, cold weights, 32000 rows, norm prologue, float32 out; us at 3 / 16 / 32 rows), against
+// loads into registers eight fragments ahead (64 bytes of a row an instruction instead of 256, 64 KB in flight):
+//   n = 2048 32 / 35 / 44 -> 27 / 30 / 35, n = 4096 54 / 58 / 67 -> 44 / 50 / 61,
+//   n = 6144 85 / 91 / 183 -> 66 / 74 / 145, n = 8192 101 / 110 / 220 -> 90 / 98 / 191 (524 MB: 5.3 TB/s).
+// The VALU kernel, which takes up to four batch rows a pass over W: n = 4096 86 / 239 / 470, n = 8192 164 / 608.
+// The non-temporal hint is worth 7% at n = 8192.
 #include <algorithm>
 
 #include "nq_dense.h"
@@ -23,8 +24,6 @@ namespace nq {
 namespace {
 
 constexpr int kWaves = 8;
-constexpr int G = 8;  // fragments of W in flight per wave, and again in use
-
 // The barrier between the waves' LDS writes and their reads: waits for this wave's LDS accesses only (W's
 // loads stay in flight).
 __device__ inline void lds_barrier() { barrier_keep_dma(); }
@@ -32,8 +31,9 @@ __device__ inline void lds_barrier() { barrier_keep_dma(); }
 template <typename T, int NF, int CT, bool kNorm>
 __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2))) void dense_mfma_kernel(
     const DenseArgs a) {
-    static_assert(NF % G == 0, "whole groups of fragments");
-    constexpr int NG = NF / G;
+    static_assert(NF % 4 == 0, "whole stages of four fragments");
+    constexpr int NS = NF / 4;                  // stages of a tile
+    constexpr int kStages = CT == 1 ? 4 : 3;    // of a wave's ring, as the LDS holds beside the partial tiles
     __shared__ f32x4 part[2][kWaves][CT][64];
     __shared__ float ssum[kWaves][16 * CT];
     const int t = threadIdx.x;
@@ -46,21 +46,28 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2))
     const int b0 = static_cast<int>(blockIdx.y) * 16 * CT;
     const int tiles = (a.m + 15) / 16;
 
-    // fragment i of row tile `tile`: rows past m and fragments past the slice load zeros
-    const uint32_t lane_off = 2u * (static_cast<uint32_t>(c) * static_cast<uint32_t>(a.n) + static_cast<uint32_t>(k0 + 8 * g));
-    auto issue = [&](u32x4 (&dst)[G], int tile, int grp) {
+    // a stage is four fragments of a tile, 16 rows x 256 bytes, each DMA taking four rows; LDS chunk p of row r
+    // holds the row's 16-byte chunk p ^ r, so that a fragment's reads (one chunk of 16 rows) have no bank conflicts.
+    // Rows past m fetch row m - 1 (their sums are not stored), columns past the row its end (not multiplied).
+    __shared__ __attribute__((aligned(16))) uint16_t ring[kWaves][kStages][16 * 128];
+    const uint32_t lring =
+        __builtin_amdgcn_readfirstlane(lds_addr(&ring[0][0][0]) + static_cast<uint32_t>(wave) * sizeof(ring[0]));
+    auto issue_stage = [&](int tile, int grp, int slot) {
         const int row0 = min(tile, tiles - 1) * 16;
-        const uint32_t bytes = 2u * static_cast<uint32_t>(min(16, a.m - row0)) * static_cast<uint32_t>(a.n);
-        const rsrc_t rs = make_rsrc(a.w + static_cast<size_t>(row0) * static_cast<size_t>(a.n), bytes);
+        const uint16_t* base = a.w + static_cast<size_t>(row0) * static_cast<size_t>(a.n);
 #pragma unroll
-        for (int i = 0; i < G; ++i) {
-            const int fi = grp * G + i;
-            dst[i] = load_b128_stream(rs, fi < nf ? lane_off + 64u * static_cast<uint32_t>(fi) : bytes);
+        for (int j = 0; j < 4; ++j) {
+            const int r = 4 * j + (lane >> 4);
+            const int col = min(k0 + 128 * grp + 8 * ((lane & 15) ^ r), a.n - 8);
+            dma16_lds_stream(base, 2u * (static_cast<uint32_t>(min(r, a.m - 1 - row0)) * static_cast<uint32_t>(a.n) +
+                                         static_cast<uint32_t>(col)),
+                             lring + static_cast<uint32_t>(slot) * (16u * 256u) + static_cast<uint32_t>(j) * 1024u);
         }
     };
-    u32x4 wv[2][G];
     int tile = static_cast<int>(blockIdx.x);
-    issue(wv[0], tile, 0);
+    const int stride = static_cast<int>(gridDim.x);
+#pragma unroll
+    for (int st = 0; st < kStages; ++st) issue_stage(tile + st / NS * stride, st % NS, st);
 
     // the mean square of each batch row: every wave sums its slice, the slices meet in LDS
     auto load_x = [&](int b, int i) {
@@ -133,28 +140,30 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2))
         }
     }
 
+    int slot = 0;
     for (int it = 0; tile < tiles; ++it) {
-        const int next = tile + static_cast<int>(gridDim.x);
         f32x4 acc[CT][2];
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) acc[ct][0] = acc[ct][1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int grp = 0; grp < NG; ++grp) {
-            // the next group's loads go out before this group's MFMAs: the rest of this tile, else the
-            // start of the block's next one
-            const int cur = NG % 2 == 0 ? grp & 1 : 0;
-            if (grp + 1 < NG) issue(wv[NG % 2 == 0 ? cur ^ 1 : 1], tile, grp + 1);
-            else issue(wv[NG % 2 == 0 ? cur ^ 1 : 1], next, 0);
+        for (int st = 0; st < NS; ++st) {
+            wait_vmcnt<4 * (kStages - 1)>();  // the oldest stage's four DMAs (a store in flight only waits longer)
+            asm volatile("" ::: "memory");    // (the compiler does not know that the reads depend on it)
+            const uint16_t* src = &ring[wave][slot][128 * c];
+            u32x4 f[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) f[i] = *reinterpret_cast<const u32x4*>(src + 8 * ((4 * i + g) ^ c));
+            __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));  // lgkmcnt(0): read before the slot is filled again
+            asm volatile("" ::: "memory");
+            issue_stage(tile + (st + kStages) / NS * stride, (st + kStages) % NS, slot);
+            slot = slot + 1 == kStages ? 0 : slot + 1;
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int i = 0; i < G; ++i)
+            for (int i = 0; i < 4; ++i)
+                if (4 * st + i < nf)
 #pragma unroll
-                for (int ct = 0; ct < CT; ++ct)
-                    acc[ct][i & 1] = mfma16x16x32<T>(wv[cur][i], xf[ct][grp * G + i], acc[ct][i & 1]);
-            if (NG % 2 != 0) {
-#pragma unroll
-                for (int i = 0; i < G; ++i) wv[0][i] = wv[1][i];
-            }
+                    for (int ct = 0; ct < CT; ++ct)
+                        acc[ct][i & 1] = mfma16x16x32<T>(f[i], xf[ct][4 * st + i], acc[ct][i & 1]);
         }
         // C: lane (c, g) holds rows 4 g + i of the tile for batch row c
 #pragma unroll
@@ -177,8 +186,9 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2))
                 else static_cast<uint16_t*>(a.y)[at] = v;
             }
         }
-        tile = next;
+        tile += stride;
     }
+    wait_vmcnt<0>();  // the re-fetches past the last tile land before the block's LDS is released
 }
 
 template <typename T, int NF, int CT>
@@ -190,7 +200,7 @@ void launch_nf(const DenseArgs& a, hipStream_t st) {
 }
 
 // Sixteen batch rows a pass over W; 32 where two slices of x fit the registers beside the loads in flight
-// (n up to 4096: 24 rows 64 us in one pass, n = 8192 212 in two).
+// (n up to 4096: 32 rows 61 us in one pass, n = 8192 191 in two).
 template <typename T>
 void launch_dense(const DenseArgs& a, hipStream_t st) {
     const int nf = a.n / (32 * kWaves);
@@ -207,8 +217,8 @@ void launch_dense(const DenseArgs& a, hipStream_t st) {
 
 }  // namespace
 
-// From three batch rows: at one or two the VALU kernel streams W faster (n = 4096 41.5 / 49, n = 8192 82 / 87
-// us). Whole fragments per wave, as many as its registers hold; any other n keeps the VALU kernel.
+// From three batch rows: at one or two the VALU kernel streams W faster (n = 4096 41.5, n = 8192 82 us, against
+// 44 and 90 here). Whole fragments per wave, as many as its registers hold; any other n keeps the VALU kernel.
 bool dense_mfma_applies(int64_t batch, int64_t n) { return batch >= 3 && n % (32 * kWaves) == 0 && n <= 32 * 32 * kWaves; }
 
 void launch_dense_mfma(int dtype, const DenseArgs& a, hipStream_t st) {

@@ -11,6 +11,8 @@ CASES = [  # m, n, batch, ldy
     (4113, 1024, 16, 4200),  # more row tiles than blocks, the last one of one row; output rows wider than m
     (1003, 2048, 17, 1003),  # two batch tiles, the second of one row
     (500, 3072, 33, 500),   # 12 fragments of 16, a second pass of one batch row
+    (47, 1280, 4, 47),      # five fragments: the second stage of a wave holds one
+    (77, 2816, 20, 80),     # eleven fragments, two batch tiles
     (333, 6144, 5, 333),    # an odd number of fragment groups
     (4100, 8192, 19, 4100),  # the widest rows; 16 batch rows a pass
 ]
