@@ -22,8 +22,8 @@ struct RowsArgs {
     int kpad, zpitch;       // stage 1 output: columns [rows, kpad) and [kpad, zpitch) get zeros
 };
 
-// Features of a block (by 64 batch rows), and the wave groups its k steps are shared by.
-enum RowsTile { kRows256, kRows128x2, kRows128x4 };
+// Features of a block (by 64 batch rows; kRows256q32: by 32), and the wave groups its k steps are shared by.
+enum RowsTile { kRows256, kRows128x2, kRows128x4, kRows256q32 };
 
 struct RowsPlan {
     RowsTile tile;

@@ -481,14 +481,25 @@ bool rows_stage1_plan(int64_t batch, int64_t n, int64_t r, int64_t kpad, size_t 
 // 300 / 666 / 2048 rows 14.3 / 19.6, 29.6 / 22.2, 84 / 43; m = 11008, r = 1632 at 160 / 300 / 2048
 // 15.0 / 20.5, 26.5 / 22.5, 157 / 115; m = 28672, r = 3520 at 128 / 300 / 2048 55.7 / 43.3, 137 / 113,
 // 792 / 567; m = 1024, r = 512 at 666 / 2048 5.4 / 8.9, 10.7 / 9.2.
+//
+// A block of 32 batch rows takes a little more than half a step (each decoded sign feeds half the MFMAs) and
+// runs where its finer grid leaves the busiest CU less to do. The op, bf16, us, before and with it: m = 8192,
+// n = 8192, r = 2240 at 256 / 666 rows 46.6 / 41.3, 90.5 / 89.4; m = 28672, n = 8192, r = 3520 at 64 / 400 rows 51 / 45,
+// 197 / 183; m = n = 4096, r = 1120 at 400 / 512 rows 31.6 / 28.3, 34.0 / 29.9; m = n = 2048, r = 1024 at 666 rows
+// 35.4 / 27.3. Counted as 0.42 a step it also ran on m = 28672 at 512 rows, 201 / 206; with the other tile's start of
+// 2 us also on m = 15153, r = 512 at 94 rows, 14.3 / 15.1.
+constexpr double kStart = 2.0, kStep = 0.74, kHalfStart = 3.5, kHalfStep = 0.43;
 bool rows_stage2_plan(int64_t batch, int64_t m, int64_t wr, RowsPlan& p) {
     if (batch < kMidBatch) return false;
     const int64_t steps = ceil_div(wr, 2);
     const int64_t per_cu = ceil_div(ceil_div(m, 256) * ceil_div(batch, 64), 256);
-    const double rows = 2.0 + 0.74 * per_cu * steps;
+    const int64_t per_cu32 = ceil_div(ceil_div(m, 256) * ceil_div(batch, 32), 256);
+    const double rows64 = kStart + kStep * per_cu * steps, rows32 = kHalfStart + kHalfStep * per_cu32 * steps;
+    const bool half = rows32 < rows64;
+    const double rows = half ? rows32 : rows64;
     const double passes = 3.0 + 1e-6 * batch * m * wr * (m < 8192 ? 0.2 : 0.135);
     if (rows > passes) return false;
-    p = RowsPlan{kRows256, 1, static_cast<int>(steps), 0};
+    p = RowsPlan{half ? kRows256q32 : kRows256, 1, static_cast<int>(steps), 0};
     return true;
 }
 
@@ -498,6 +509,7 @@ static void launch_stage1_tile(const RowsArgs& a, const RowsPlan& p, hipStream_t
         case kRows256: return launch_tile<T, T, false, 256, 64, 16, 1>(a, p, st);
         case kRows128x2: return launch_tile<T, T, false, 128, 64, 8, 2>(a, p, st);
         case kRows128x4: return launch_tile<T, T, false, 128, 64, 8, 4>(a, p, st);
+        case kRows256q32: return;  // a stage 2 tile
     }
 }
 
@@ -506,9 +518,15 @@ void launch_rows_stage1(int dtype, const RowsArgs& a, const RowsPlan& p, hipStre
     else launch_stage1_tile<BF16>(a, p, st);
 }
 
+template <typename TO>
+static void launch_stage2_tile(const RowsArgs& a, const RowsPlan& p, hipStream_t st) {
+    if (p.tile == kRows256q32) launch_tile<BF16, TO, true, 256, 32, 8, 1>(a, p, st);
+    else launch_tile<BF16, TO, true, 256, 64, 8, 1>(a, p, st);
+}
+
 void launch_rows_stage2(int dtype, const RowsArgs& a, const RowsPlan& p, hipStream_t st) {
-    if (dtype == NQ_F16) launch_tile<BF16, F16, true, 256, 64, 8, 1>(a, p, st);
-    else launch_tile<BF16, BF16, true, 256, 64, 8, 1>(a, p, st);
+    if (dtype == NQ_F16) launch_stage2_tile<F16>(a, p, st);
+    else launch_stage2_tile<BF16>(a, p, st);
 }
 
 }  // namespace nq

@@ -25,6 +25,7 @@ CASES = [
     (520, 4096, 1632, 630, False),    # four k groups, no k range
     (11008, 4096, 1632, 300, True),   # 128-feature tiles; stage 2 on these kernels too
     (8200, 512, 4097, 700, False),    # the shortest rows, several tiles a CU; a large ragged rank, a ragged last tile
+    (8100, 1024, 2000, 161, False),   # stage 2 in blocks of 32 rows, the last one of one row; a ragged last tile
     (2048, 1024, 2240, 2048, True),   # 256-feature tiles on every CU, one range
 ]
 
