@@ -145,6 +145,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 4)))
             __builtin_amdgcn_s_waitcnt(0xF | (0x3 << 14) | (0x7 << 4));  // lgkmcnt(0): the chunk is in registers
             issue(f + kSplitRing);
             wait_vmcnt<(kSplitRing - 1) * kDma>();
+            asm volatile("" ::: "memory");  // the reads depend on it, which the compiler does not know
             read(nxt, f + 1);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
