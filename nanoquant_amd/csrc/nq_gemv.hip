@@ -2268,6 +2268,11 @@ inline bool s1w_applies(const uint16_t* x, const uint16_t* s_in, int n, int wn, 
     return n >= 8 && n % 8 == 0 && r > 0 && aligned(x, 16) && aligned(s_in, 16) && (wn <= 1024 || s1m_fits(n, wn));
 }
 
+// What the many-row stage 1 (nq_gemv_rows.hip) asks of its operands. Unlike the kernels of s1w_applies it takes rows of
+// any length: gated on them, n > 32768 ran the generic kernel from 33 batch rows (stage 1 alone, bf16, n = 40960, r =
+// 3520 at 64 rows: 1204 us with that one, 51 with the k-split kernel, 31 with these).
+inline bool rows_applies(const uint16_t* x, const uint16_t* s_in) { return aligned(x, 16) && aligned(s_in, 16); }
+
 inline S1Item s1_item_of(const GemvArgs& a) {
     S1Item it;
     it.v_bits = a.v_bits;
@@ -2407,7 +2412,7 @@ int launch_stage2_rows(const GemvArgs& a, const RowsPlan& p) {
 template <typename T>
 int launch_stage1(const GemvArgs& a) {
     RowsPlan rp;
-    if (s1w_applies(a.x, a.s_in, a.n, a.wn, a.r) && rows_stage1_plan(a.batch, a.n, a.r, a.plan.kpad, a.part_bytes, rp))
+    if (rows_applies(a.x, a.s_in) && rows_stage1_plan(a.batch, a.n, a.r, a.plan.kpad, a.part_bytes, rp))
         return launch_stage1_rows<T>(a, rp);
     SbPlan sp;
     if (sb1_plan(a, sp)) return launch_stage1_sb<T>(a, sp);

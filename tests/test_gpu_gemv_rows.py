@@ -27,6 +27,10 @@ CASES = [
     (8200, 512, 4097, 700, False),    # the shortest rows, several tiles a CU; a large ragged rank, a ragged last tile
     (8100, 1024, 2000, 161, False),   # stage 2 in blocks of 32 rows, the last one of one row; a ragged last tile
     (2048, 1024, 2240, 2048, True),   # 256-feature tiles on every CU, one range
+    (72, 33032, 130, 33, True),       # rows of more than 1024 words (n > 32768), n % 64 == 8
+    (300, 40960, 300, 64, False),     # the same in several k ranges
+    (64, 53248, 96, 100, True),
+    (130, 33024, 65, 200, False),
 ]
 
 
@@ -85,6 +89,34 @@ def test_rows_against_oracle(lib, case, dtype):
     y = _run(lib, c, dtype)
     assert _error(y, y64, dtype) <= BAR
     assert torch.equal(y, _run(lib, c, dtype)), "a second call over another workspace's bytes"
+
+
+def _stage1_us(lib, rows, n, r):
+    from nanoquant_amd import _lib
+    x, s_in = torch.randn(rows, n, device="cuda").half(), torch.rand(n, device="cuda").half()
+    V = torch.randint(-2 ** 31, 2 ** 31 - 1, (r, (n + 31) // 32), dtype=torch.int32, device="cuda")
+    nbytes = lib.nq_gemv_workspace_bytes(rows, n, r, 64)
+    ws = torch.zeros(nbytes, dtype=torch.uint8, device="cuda")
+    times = []
+    for _ in range(8):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        for _ in range(4):
+            _lib.check(lib.nq_gemv_stage1(_lib.NQ_F16, x.data_ptr(), s_in.data_ptr(), V.data_ptr(), None, rows, n, r, 64,
+                                          ws.data_ptr(), nbytes, _lib.stream_of(x.device)), "nq_gemv_stage1")
+        end.record()
+        torch.cuda.synchronize()
+        times.append(start.elapsed_time(end) * 250)
+    return min(times)
+
+
+@pytest.mark.parametrize("rows", [48, 64, 100])
+def test_rows_run_on_the_longest_inputs(lib, rows):
+    """n > 32768: the kernels planned for (and given a workspace) run, not the general one, which passes over V for every
+    eight batch rows and took 20 times the time of 32 rows where these take two to four times."""
+    print("\n[case] gemv rows, time", rows, flush=True)
+    few, many = _stage1_us(lib, 32, 53248, 1632), _stage1_us(lib, rows, 53248, 1632)
+    assert many < 8 * few, f"{rows} rows take {many:.0f} us, 32 rows {few:.0f}"
 
 
 @pytest.mark.parametrize("offset", [1, 4])
