@@ -1596,9 +1596,9 @@ __global__ __launch_bounds__(NW * 64) void sb_kernel(const SbArgs a) {
 
     // 1. DMA: the x slice and s_in, and the rows' words (divisions by a multiply: the issue loops
     //    are VALU work before the first MFMA). V's words come from HBM and the x slice mostly from
-    //    L2: the words go out first, so that part of their longer latency
+    //    L2: up to 64 batch rows the words go out first, so that part of their longer latency
     //    passes while the slice is issued (same-box A/B, down_proj and Llama-3-70B q/o at 16-64
-    //    rows: 1.1-1.9% faster).
+    //    rows: 1.1-1.9% faster); with more rows the larger slice goes first.
     auto dma_slice = [&]() {
         const uint32_t xchunks = static_cast<uint32_t>(XCOLS * kw4);
         const uint32_t kend = static_cast<uint32_t>(a.wpr) * 32u;  // elements of k
@@ -1630,8 +1630,13 @@ __global__ __launch_bounds__(NW * 64) void sb_kernel(const SbArgs a) {
             dma4(wbase + min(row, rlast) * static_cast<uint32_t>(a.wpr) + q, wl + l0);
         }
     };
-    dma_words();
-    dma_slice();
+    if constexpr (CT <= 4) {
+        dma_words();
+        dma_slice();
+    } else {
+        dma_slice();
+        dma_words();
+    }
     __builtin_amdgcn_s_waitcnt(0);  // this wave's DMAs have landed (vmcnt, expcnt and lgkmcnt all zero)
     __syncthreads();
     NQ_STAMP(1);
@@ -1839,9 +1844,8 @@ struct SbPlan {
 
 // When the batched stage 1 replaces s1m_kernel (measured crossovers, see sb_kernel): on rows of at
 // least 256 words, from a batch that falls with the row width (sb_min_batch) up to where the kernels of
-// nq_gemv_rows.hip take over (rows_stage1_plan: fewer than 64 rows, so four batch tiles), with an LDS
-// slice of at most 160 KB per block. On narrower rows s1m_kernel with two
-// or four row tiles per block is the faster one (n = 4096, r = 1632, 64 / 128 rows: 8.9 / 13.4 us
+// nq_gemv_rows.hip take over (rows_stage1_plan and sb_before_rows: at most 96 rows, so six batch tiles),
+// with an LDS slice of at most 160 KB per block. On narrower rows s1m_kernel with two or four row tiles per block is the faster one (n = 4096, r = 1632, 64 / 128 rows: 8.9 / 13.4 us
 // against 11.5 / 15.6).
 constexpr int kSbWideWords = 256;
 // The smallest batch that runs it, by words per row (same-box A/B of the GEMV op against the
@@ -1865,7 +1869,7 @@ inline int64_t sb_min_batch(int64_t wpr, int64_t rows) {
     if (wpr >= 320) return 8;
     return rows * wpr < 256 * 1024 ? 8 : 16;
 }
-constexpr int kSbMaxBatch = 64;
+constexpr int kSbMaxBatch = 96;
 constexpr int kSbLdsBytes = 160 * 1024;
 constexpr int kSbMaxBlocks = 256;
 // Rounds of blocks the search may take when no plan fits one round (see sb_plan_any).
@@ -1896,7 +1900,7 @@ inline bool sb_plan(int64_t batch, int64_t rows, int64_t wpr, int64_t kpad, SbPl
 // (other k ranges) was slower (21.58 -> 22.62), and four blocks per CU were no better.
 inline bool sb_plan_rounds(int64_t batch, int64_t rows, int64_t wpr, int64_t kpad, int max_rounds, SbPlan& p) {
     const int64_t occupancy = batch <= 32 ? 2 : 1;  // blocks per CU a round may count
-    const int ct = static_cast<int>(std::min<int64_t>(4, ceil_div(batch, 16)));
+    const int ct = static_cast<int>(std::min<int64_t>(kSbMaxBatch / 16, ceil_div(batch, 16)));
     const int passes = static_cast<int>(ceil_div(batch, 16LL * ct));
     const int xcols = 16 * ct + 1;
     double best = -1.0;
@@ -2308,7 +2312,9 @@ int launch_sb_rtw(const SbArgs& s, const SbPlan& p, hipStream_t st) {
         case 1: return launch_sb_cfg<T, RTW, 1>(s, p, st);
         case 2: return launch_sb_cfg<T, RTW, 2>(s, p, st);
         case 3: return launch_sb_cfg<T, RTW, 3>(s, p, st);
-        default: return launch_sb_cfg<T, RTW, 4>(s, p, st);
+        case 4: return launch_sb_cfg<T, RTW, 4>(s, p, st);
+        case 5: return launch_sb_cfg<T, RTW, 5>(s, p, st);
+        default: return launch_sb_cfg<T, RTW, 6>(s, p, st);
     }
 }
 
@@ -2317,6 +2323,19 @@ int launch_sb_rtw(const SbArgs& s, const SbPlan& p, hipStream_t st) {
 inline bool sb1_plan(const GemvArgs& a, SbPlan& p) {
     return a.n % 32 == 0 && a.r > 0 && aligned(a.x, 16) && aligned(a.s_in, 16) &&
            sb_plan(a.batch, a.r, a.wn, a.plan.kpad, p) && p.part_bytes <= a.part_bytes;
+}
+
+// Where both have a plan, the k-split kernel keeps a small V: the kernels of many rows are bound by their steps' latency
+// there, and share a decoded sign over fewer batch rows than their tiles hold. Stage 1 alone, bf16, us, k-split against
+// many rows: n = 16384 at 48 rows, r = 512 / 1632 / 2976 (0.26 / 0.84 / 1.5 M words of V) 10.6 / 13.2, 15.1 / 15.5, 19.1 /
+// 18.8; n = 8192 at 64 rows, r = 512 / 1632 / 4224 (0.13 / 0.42 / 1.1 M) 9.8 / 11.9, 13.4 / 15.3, 20.7 / 19.0; at 80 rows, r =
+// 1120 / 2240 (0.29 / 0.57 M) 12.9 / 14.3, 17.2 / 16.9; at 96 rows, r = 768 / 1632 (0.20 / 0.42 M) 12.9 / 13.4, 17.2 / 15.1.
+inline bool sb_before_rows(int64_t batch, int64_t r, int64_t words) {
+    const int64_t v_words = r * words;
+    if (batch <= 48) return v_words < 1400000;
+    if (batch <= 64) return v_words < 800000;
+    if (batch <= 80) return v_words < 500000;
+    return batch <= kSbMaxBatch && v_words < 300000;
 }
 
 template <typename T>
@@ -2412,10 +2431,12 @@ int launch_stage2_rows(const GemvArgs& a, const RowsPlan& p) {
 template <typename T>
 int launch_stage1(const GemvArgs& a) {
     RowsPlan rp;
+    SbPlan sp;
+    const bool sb_first = sb_before_rows(a.batch, a.r, a.wn);
+    if (sb_first && sb1_plan(a, sp)) return launch_stage1_sb<T>(a, sp);
     if (rows_applies(a.x, a.s_in) && rows_stage1_plan(a.batch, a.n, a.r, a.plan.kpad, a.part_bytes, rp))
         return launch_stage1_rows<T>(a, rp);
-    SbPlan sp;
-    if (sb1_plan(a, sp)) return launch_stage1_sb<T>(a, sp);
+    if (!sb_first && sb1_plan(a, sp)) return launch_stage1_sb<T>(a, sp);
     if (s1w_applies(a.x, a.s_in, a.n, a.wn, a.r)) {
         S1Table tab;
         tab.count = 1;
@@ -2714,8 +2735,12 @@ inline size_t gemv_part_bytes(int64_t batch, int64_t n, int64_t r, int64_t m) {
     size_t bytes = 0;
     SbPlan p;
     RowsPlan rp;
-    if (rows_stage1_plan(batch, n, r, pl.kpad, SIZE_MAX, rp)) bytes = rp.part_bytes;
-    else if (n % 32 == 0 && r > 0 && sb_plan(batch, r, ceil_div(n, 32), pl.kpad, p)) bytes = p.part_bytes;
+    const int64_t words = ceil_div(n, 32);
+    const bool sb_first = sb_before_rows(batch, r, words);
+    auto sb = [&] { return n % 32 == 0 && r > 0 && sb_plan(batch, r, words, pl.kpad, p); };
+    if (sb_first && sb()) bytes = p.part_bytes;
+    else if (rows_stage1_plan(batch, n, r, pl.kpad, SIZE_MAX, rp)) bytes = rp.part_bytes;
+    else if (!sb_first && sb()) bytes = p.part_bytes;
     return (bytes + 255) / 256 * 256;
 }
 

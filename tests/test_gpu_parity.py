@@ -248,6 +248,10 @@ GEMV_CASES = [
     ("sb_b64_r200", 1000, 2048, 200, 64, True),
     ("sb_b70_wide", 600, 8192, 500, 70, True),
     ("sb_b20_wide_ragged", 700, 9216, 333, 20, False),
+    ("sb_b96_wide", 300, 8192, 1000, 96, False),
+    ("rows_b97_wide", 300, 8192, 1000, 97, False),
+    ("sb_b40_n16384", 200, 16384, 700, 40, True),
+    ("rows_b49_n20480", 200, 20480, 1300, 49, False),
     ("sb_b3_n16384", 500, 16384, 300, 3, True),
     ("sb_b5_n20000_ragged", 300, 20000, 333, 5, False),
     ("sb_b8_n11008", 1000, 11008, 200, 8, True),
