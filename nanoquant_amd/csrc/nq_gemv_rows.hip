@@ -488,13 +488,20 @@ bool rows_stage1_plan(int64_t batch, int64_t n, int64_t r, int64_t kpad, size_t 
 // 197 / 183; m = n = 4096, r = 1120 at 400 / 512 rows 31.6 / 28.3, 34.0 / 29.9; m = n = 2048, r = 1024 at 666 rows
 // 35.4 / 27.3. Counted as 0.42 a step it also ran on m = 28672 at 512 rows, 201 / 206; with the other tile's start of
 // 2 us also on m = 15153, r = 512 at 94 rows, 14.3 / 15.1.
-constexpr double kStart = 2.0, kStep = 0.74, kHalfStart = 3.5, kHalfStep = 0.43;
+//
+// Short ranks do not hide a block's start behind its steps: up to 28 steps the 64-row block costs 4.8 us and 0.64 a
+// step. Counted by the long ranks' figures alone it ran where the passes are faster (stage 2, bf16, us, passes against
+// this one: m = 9728, r = 256 at 200 rows 5.5 / 6.8, m = 20480, r = 576 / 1120 at 128 rows 8.4 / 10.3, 14.1 / 16.0, m =
+// 12288, r = 640 at 200 rows 10.3 / 11.2; it stays on m = 28672, r = 512 at 128 rows, 11.9 / 10.2).
+constexpr double kStart = 2.0, kStep = 0.74, kShortStart = 4.8, kShortStep = 0.64;
+constexpr double kHalfStart = 3.5, kHalfStep = 0.43;
 bool rows_stage2_plan(int64_t batch, int64_t m, int64_t wr, RowsPlan& p) {
     if (batch < kMidBatch) return false;
     const int64_t steps = ceil_div(wr, 2);
     const int64_t per_cu = ceil_div(ceil_div(m, 256) * ceil_div(batch, 64), 256);
     const int64_t per_cu32 = ceil_div(ceil_div(m, 256) * ceil_div(batch, 32), 256);
-    const double rows64 = kStart + kStep * per_cu * steps, rows32 = kHalfStart + kHalfStep * per_cu32 * steps;
+    const double rows64 = std::max(kStart + kStep * per_cu * steps, kShortStart + kShortStep * per_cu * steps);
+    const double rows32 = kHalfStart + kHalfStep * per_cu32 * steps;
     const bool half = rows32 < rows64;
     const double rows = half ? rows32 : rows64;
     const double passes = 3.0 + 1e-6 * batch * m * wr * (m < 8192 ? 0.2 : 0.135);
