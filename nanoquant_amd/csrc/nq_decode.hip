@@ -678,17 +678,24 @@ __global__ __launch_bounds__(kBeginThreads) void step_begin_kernel(const StepBeg
         const int per_row = (a.x_pieces + kBeginThreads - 1) / kBeginThreads;
         const int b = block / per_row;
         const int piece = (block - b * per_row) * kBeginThreads + t;
+    uint32_t* fault;         // {token, position}, or nullptr
         const int64_t tok = a.tok[b];
         if (piece >= a.x_pieces) return;
         u32x4 v = u32x4{0u, 0u, 0u, 0u};  // a token outside the vocabulary
         if (tok >= 0 && tok < a.vocab) v = *reinterpret_cast<const u32x4*>(a.embed + tok * a.hidden + 8 * piece);
         *reinterpret_cast<u32x4*>(a.x + static_cast<int64_t>(b) * a.hidden + 8 * piece) = v;
         return;
+    if (a.fault != nullptr && block == 0 && t == 0) {  // the step's token needs a place after the position
+        const int64_t p = *a.pos;
+        if (p < 0 || p >= a.max_len - 1) __hip_atomic_store(a.fault + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
     }
     const int64_t p = *a.pos;
     if (a.table != nullptr && block == a.x_blocks) {
         for (int e = t; e < a.row; e += kBeginThreads)
             a.table_out[e] = p >= 0 && p < a.max_len ? a.table[p * a.row + e] : uint16_t{0};
+        if (a.fault != nullptr && piece == 0 && (tok < 0 || tok >= a.vocab))
+            __hip_atomic_store(a.fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         return;
     }
     // 8 elements of the mask a thread; scores row element e belongs to position e / groups
@@ -897,11 +904,19 @@ int nq_decode_begin(int dtype, const void* embed, int64_t vocab, int64_t hidden,
         (table && (row > INT32_MAX / 4 || max_len * row > ((int64_t)1 << 40))) ||
         (scores && (groups > 65535 || max_len * groups > INT32_MAX / 4 || scores_rows > INT32_MAX / 4 ||
                     scores_rows * max_len * groups > ((int64_t)1 << 38))))
+    return nq_decode_begin_checked(dtype, embed, vocab, hidden, tok, x, batch, position, max_len, table, row, table_out,
+                                   scores, scores_rows, groups, nullptr, stream);
+}
+
+int nq_decode_begin_checked(int dtype, const void* embed, int64_t vocab, int64_t hidden, const int64_t* tok, void* x,
+                            int64_t batch, const int64_t* position, int64_t max_len, const void* table, int64_t row,
+                            void* table_out, void* scores, int64_t scores_rows, int64_t groups, uint32_t* fault,
+                            nq_stream_t stream) {
         return fail(NQ_ERR_UNSUPPORTED, "%s: sizes too large", name);
     if (batch == 0) return NQ_OK;
     if (!position || (embed && (!tok || !x)) || (table && !table_out)) return fail(NQ_ERR_INVALID_ARGUMENT, "%s: null pointer", name);
     if (!aligned(embed, 16) || !aligned(x, 16) || !aligned(tok, 8) || !aligned(position, 8) || !aligned(table, 2) ||
-        !aligned(table_out, 2) || !aligned(scores, 16))
+        !aligned(table_out, 2) || !aligned(scores, 16) || !aligned(fault, 4))
         return fail(NQ_ERR_ALIGNMENT, "%s: misaligned operand (embed, x and scores need 16 bytes)", name);
     StepBegin a{};
     a.embed = static_cast<const uint16_t*>(embed);
@@ -920,7 +935,9 @@ int nq_decode_begin(int dtype, const void* embed, int64_t vocab, int64_t hidden,
     a.x_blocks = static_cast<int>(x_blocks);
     a.x_pieces = static_cast<int>(pieces);
     a.minus_inf = dtype == NQ_F16 ? 0xFC00u : 0xFF80u;
-    const int64_t blocks = x_blocks + (table ? 1 : 0) + ceil_div(a.scores_total, 8 * kBeginThreads);
+    a.fault = fault;
+    int64_t blocks = x_blocks + (table ? 1 : 0) + ceil_div(a.scores_total, 8 * kBeginThreads);
+    if (fault && blocks == 0) blocks = 1;  // to look at the position
     if (blocks == 0) return NQ_OK;
     if (blocks > INT32_MAX / 2) return fail(NQ_ERR_UNSUPPORTED, "%s: sizes too large", name);
     step_begin_kernel<<<static_cast<unsigned>(blocks), kBeginThreads, 0, as_stream(stream)>>>(a);

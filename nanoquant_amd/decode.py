@@ -22,6 +22,7 @@ from __future__ import annotations
 import math
 import time
 import warnings
+import weakref
 from dataclasses import dataclass
 
 import torch
@@ -569,6 +570,9 @@ class GraphDecoder:
         self.pos.fill_(T)
         return logits
 
+    def raise_faults(self):
+        """Raise what finished steps have reported."""
+
     def _prompt_logits(self, ids, positions):
         """The logits [B, vocab] of a prompt's last position."""
         return self.model(ids, positions, self.cache)[:, -1]
@@ -588,6 +592,23 @@ class GraphDecoder:
         for _ in range(steps):
             logits = self._step()
         return logits
+
+
+_FREE_FAULT_WORDS = []  # (words, device) of decoders that are gone
+
+
+def _fault_words(owner, device):
+    """Two words of pinned host memory (a numpy array) in which the step's launches leave {token, position} faults, for the
+    host to look at without waiting. A launch in flight may outlive ``owner``, so its words never go back to torch's
+    allocator: another decoder takes them, once the device that may still write them has been waited for."""
+    try:
+        words, used_on = _FREE_FAULT_WORDS.pop()
+        torch.cuda.synchronize(used_on)
+        words[:] = 0
+    except IndexError:
+        words = torch.zeros(2, dtype=torch.int32, pin_memory=True).numpy()
+    weakref.finalize(owner, _FREE_FAULT_WORDS.append, (words, device))
+    return words
 
 
 class FusedDecoder(GraphDecoder):
@@ -678,6 +699,8 @@ class FusedDecoder(GraphDecoder):
         if self.pair_order:
             j = torch.arange(D, device=dev)
             self.head_order = (j // 2) + (j % 2) * (D // 2)  # position i of a head holds feature head_order[i]
+        self.faults = _fault_words(self, dev)
+        self.room = max_len - 1  # steps left, if the program has not set the position itself
             self.q_order = (torch.arange(H, device=dev)[:, None] * D + self.head_order).reshape(-1)
             self.k_order = (torch.arange(KV, device=dev)[:, None] * D + self.head_order).reshape(-1)
             half = torch.stack((self.rope_cos[:, : D // 2], self.rope_sin[:, : D // 2]), dim=-1)
@@ -798,10 +821,11 @@ class FusedDecoder(GraphDecoder):
         if not plain:
             torch.index_select(embed, 0, self.tok, out=self.x)
         table, scores = (self.rope_table, self.scores_all) if self.attention == "torch" else (None, None)
-        self._check(lib.nq_decode_begin(
+        self._check(lib.nq_decode_begin_checked(
             dt, embed.data_ptr() if plain else None, embed.shape[0], s.hidden, self.tok.data_ptr(), self.x.data_ptr(), B, self.pos.data_ptr(),
             self.max_len, self._lib.ptr(table), 0 if table is None else table.shape[1], self.rope_row.data_ptr(),
-            self._lib.ptr(scores), 0 if scores is None else s.layers * B * KV, H // KV, st), "step begin")
+            self._lib.ptr(scores), 0 if scores is None else s.layers * B * KV, H // KV, self.faults.ctypes.data, st),
+            "step begin")
         if self.attention == "torch":
             if self.pair_order:
                 freqs = torch.view_as_complex(self.rope_row.view(1, D // 2, 2))  # cos + i sin of the position
@@ -883,9 +907,32 @@ def generate(model: NanoQuantLlama, prompt: torch.Tensor, max_new_tokens: int, s
                                    attention=attention)
         else:
             decoder = GraphDecoder(model, B, T + max_new_tokens, steps_per_graph, device=prompt.device)
+    def raise_faults(self):
+        if not (self.faults[0] or self.faults[1]):
+            return
+        torch.cuda.synchronize(self.device)  # no launch in flight sets them again
+        token, position = self.faults.tolist()
+        self.faults[:] = 0
+        what = ["a token outside the vocabulary"] * token + [f"a position outside max_len ({self.max_len})"] * position
+        raise RuntimeError(f"an earlier decode step had {' and '.join(what)}: prefill again")
+
+    @torch.no_grad()
+    def decode(self, steps: int, use_graph: bool = True):
+        self.raise_faults()
+        if steps > self.room:  # or the program has set the position back: ask the device
+            pos = int(self.pos)
+            self.room = self.max_len - 1 - pos
+            if steps > self.room:
+                raise ValueError(f"{steps} steps from position {pos} do not fit max_len {self.max_len}")
+        out = super().decode(steps, use_graph)
+        self.room -= max(steps, 0)
+        return out
+
         if use_graph:
             decoder.capture()
+        self.raise_faults()
     steps = max_new_tokens - 1
+        self.room = self.max_len - 1 - prompt.shape[1]
     torch.cuda.synchronize(prompt.device)
     t0 = time.perf_counter()
     decoder.prefill(prompt)
@@ -898,3 +945,4 @@ def generate(model: NanoQuantLlama, prompt: torch.Tensor, max_new_tokens: int, s
     prof = {"prefill_time_s_wall": t1 - t0, "decode_time_s_wall": t2 - t1, "decode_tokens_total": B * steps,
             "ms_per_token": 1e3 * (t2 - t1) / max(steps, 1)}
     return decoder.ids[:, :T + max_new_tokens].clone(), tps, prof
+    decoder.raise_faults()
