@@ -57,7 +57,6 @@ SIGNATURES = {
     "nq_last_error_message": (ctypes.c_char_p, []),
     "nq_version": (_int, []),
     "nq_pack_signs": (_int, [_vp, _vp, _i64, _i64, _int, _vp]),
-    "nq_header_digest": (ctypes.c_char_p, []),
     "nq_unpack_signs": (_int, [_vp, _vp, _i64, _i64, _int, _vp]),
     "nq_repack_signs": (_int, [_vp, _vp, _i64, _i64, _int, _int, _vp]),
     "nq_pack_marlin": (_int, [_vp, _vp, _i64, _i64, _vp]),
@@ -91,8 +90,6 @@ SIGNATURES = {
     "nq_decode_end": (_int, [_vp, _i64, _i64, _i64, _vp, _vp, _i64, _vp, _vp, _vp]),
     "nq_decode_begin": (_int, [_int, _vp, _i64, _i64, _vp, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i64, _i64, _vp]),
     "nq_gemm_onebit_workspace_bytes": (_size, [_i64, _i64, _i64]),
-    "nq_decode_begin_checked": (_int, [_int, _vp, _i64, _i64, _vp, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i64, _i64,
-                                       _vp, _vp]),
     "nq_gemm_onebit": (_int, [_int, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _size, _vp]),
     "nq_gemm_nanoquant_workspace_bytes": (_size, [_i64, _i64, _i64, _i64]),
     "nq_gemm_nanoquant": (_int, [_int, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _size,
@@ -114,20 +111,12 @@ ops = None  # the C++ operators' library, set by binary_kernels where it registe
 
 
 def _bind_ops(lib: ctypes.CDLL) -> None:
-    """Hand the C++ operators the library's functions. Built from another header they stay without, and pass every call
-    on to the operators in Python."""
+    """Hand the C++ operators the library's functions."""
     if ops is None:
         return
     table = (_vp * len(OPS_FUNCTIONS))(*(ctypes.cast(getattr(lib, name), _vp).value for name in OPS_FUNCTIONS))
     bind = ops.nq_ops_bind
     bind.restype, bind.argtypes = _int, [ctypes.POINTER(_vp), _int]
-    digest = getattr(ops, "nq_ops_header_digest", None)
-    if digest is not None:
-        digest.restype, digest.argtypes = ctypes.c_char_p, []
-    if digest is None or digest() != lib.nq_header_digest():
-        warnings.warn(f"{OPS_PATH} and {LIB_PATH} were built from different headers, so the operators run in Python; "
-                      "run `python -m nanoquant_amd.build`")
-        return
     if bind(table, len(OPS_FUNCTIONS)) != 0:
         raise ImportError(f"{OPS_PATH} and this package disagree; run `python -m nanoquant_amd.build`")
 

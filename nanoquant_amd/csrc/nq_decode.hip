@@ -22,7 +22,6 @@
 // chunks' sums are combined first). The cache layout is [batch, kv_heads, max_len, head_dim]
 // for K and V; head_dim 128.
 #include <algorithm>
-#include <type_traits>
 
 #include "nq_common.h"
 #include "nq_dense.h"
@@ -237,7 +236,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(
 }
 
 // Combine the chunks of one (sequence, query head): thread d takes output element d. What bounds it is latency:
-// the position, then one round of loads per 16 chunks. One block per (sequence, kv head) made its threads go
+// the position, then one round of loads per R chunks. One block per (sequence, kv head) made its threads go
 // through the G heads one after the other, a round each (16 sequences, 64 heads over 8, 500 positions: 8.2 -> 4.9 us).
 template <typename T, int G>
 __global__ __launch_bounds__(kHeadDim) void attn_combine_kernel(const float* __restrict__ parts,
@@ -255,10 +254,10 @@ __global__ __launch_bounds__(kHeadDim) void attn_combine_kernel(const float* __r
     const int kvh = bh - b * kv_heads;
     uint16_t* orow = out + (static_cast<size_t>(b) * kv_heads * G + static_cast<size_t>(kvh) * G) * D;
     const float* hp = parts + static_cast<size_t>(bh) * n_chunks * PF;
+    constexpr int R = 16;  // chunks whose partials are loaded together
     const int e = g * D + static_cast<int>(threadIdx.x);
     float M = -INFINITY, L = 0.0f, O = 0.0f;  // running combination
-    auto round = [&](auto chunks, int c0) {
-        constexpr int R = decltype(chunks)::value;  // chunks whose partials are loaded together
+    for (int c0 = 0; c0 < used; c0 += R) {
         float m[R], l[R], o[R];
 #pragma unroll
         for (int i = 0; i < R; ++i) {
@@ -273,21 +272,16 @@ __global__ __launch_bounds__(kHeadDim) void attn_combine_kernel(const float* __r
         const float scale = expf(M - bm);  // 0 on the first batch (M = -inf, bm finite)
         L *= scale;
         O *= scale;
-        // selects, not branches: into a branch the compiler moves the loads of l and o, which then come one after the
-        // other (both launches, one sequence of 32 heads, each with keys of its own: 500 / 1900 positions 8.6 / 16.3 us,
-        // so 7.4 / 11.7; 4 query heads per kv head 14.6 / 33.6, so 13.5 / 28.6)
 #pragma unroll
         for (int i = 0; i < R; ++i) {
-            const float f = expf(m[i] - bm);
-            const float Ln = fmaf(l[i], f, L), On = fmaf(o[i], f, O);
-            L = c0 + i < used ? Ln : L;
-            O = c0 + i < used ? On : O;
+            if (c0 + i < used) {
+                const float f = expf(m[i] - bm);
+                L = fmaf(l[i], f, L);
+                O = fmaf(o[i], f, O);
+            }
         }
         M = bm;
-    };
-    int c0 = 0;  // sixteen chunks a round, four where no more are left (128 positions: 16 took 0.65 us more)
-    for (; used - c0 > 4; c0 += 16) round(std::integral_constant<int, 16>{}, c0);
-    if (c0 < used) round(std::integral_constant<int, 4>{}, c0);
+    }
     orow[e] = T::from_float(O / L);
 }
 
@@ -588,19 +582,15 @@ __device__ inline int argmax_row(const float* __restrict__ row, int n, int vec) 
     if (vec) {
         constexpr int kAhead = 8;  // 16-byte loads of a thread in flight
         const rsrc_t rs = make_rsrc(row, static_cast<uint32_t>(n) * 4u);
-        for (int first = 0; first < n; first += 4 * kArgmaxThreads * kAhead) {
-            const int base = first + 4 * t;
+        for (int base = 4 * t; base < n; base += 4 * kArgmaxThreads * kAhead) {
             u32x4 d[kAhead];
 #pragma unroll
-            for (int u = 0; u < kAhead; ++u) {  // past the row: not read, not taken (4096 logits 4.9 -> 4.5 us)
-                d[u] = u32x4{0u, 0u, 0u, 0u};
-                if (first + 4 * kArgmaxThreads * u < n)  // uniform
-                    d[u] = load_b128(rs, 4u * static_cast<uint32_t>(base + 4 * kArgmaxThreads * u));
-            }
+            for (int u = 0; u < kAhead; ++u)  // past the row: not read (zeros), not taken
+                d[u] = load_b128(rs, 4u * static_cast<uint32_t>(base + 4 * kArgmaxThreads * u));
 #pragma unroll
             for (int u = 0; u < kAhead; ++u) {
                 const int i = base + 4 * kArgmaxThreads * u;
-                if (first + 4 * kArgmaxThreads * u < n && i < n) {
+                if (i < n) {
                     take(__uint_as_float(d[u].x), i);
                     take(__uint_as_float(d[u].y), i + 1);
                     take(__uint_as_float(d[u].z), i + 2);
@@ -678,24 +668,17 @@ struct StepBegin {
     int hidden, row, groups;
     int x_blocks, x_pieces;  // blocks over the embedding rows, 8-element pieces of a row
     uint32_t minus_inf;      // a pair
-    uint32_t* fault;         // {token, position}, or nullptr
 };
 constexpr int kBeginThreads = 256;
 
 __global__ __launch_bounds__(kBeginThreads) void step_begin_kernel(const StepBegin a) {
     const int t = static_cast<int>(threadIdx.x);
     const int block = static_cast<int>(blockIdx.x);
-    if (a.fault != nullptr && block == 0 && t == 0) {  // the step's token needs a place after the position
-        const int64_t p = *a.pos;
-        if (p < 0 || p >= a.max_len - 1) __hip_atomic_store(a.fault + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
     if (block < a.x_blocks) {
         const int per_row = (a.x_pieces + kBeginThreads - 1) / kBeginThreads;
         const int b = block / per_row;
         const int piece = (block - b * per_row) * kBeginThreads + t;
         const int64_t tok = a.tok[b];
-        if (a.fault != nullptr && piece == 0 && (tok < 0 || tok >= a.vocab))
-            __hip_atomic_store(a.fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         if (piece >= a.x_pieces) return;
         u32x4 v = u32x4{0u, 0u, 0u, 0u};  // a token outside the vocabulary
         if (tok >= 0 && tok < a.vocab) v = *reinterpret_cast<const u32x4*>(a.embed + tok * a.hidden + 8 * piece);
@@ -904,14 +887,6 @@ int nq_decode_end(const float* logits, int64_t rows, int64_t n, int64_t ldx, int
 int nq_decode_begin(int dtype, const void* embed, int64_t vocab, int64_t hidden, const int64_t* tok, void* x, int64_t batch,
                     const int64_t* position, int64_t max_len, const void* table, int64_t row, void* table_out, void* scores,
                     int64_t scores_rows, int64_t groups, nq_stream_t stream) {
-    return nq_decode_begin_checked(dtype, embed, vocab, hidden, tok, x, batch, position, max_len, table, row, table_out,
-                                   scores, scores_rows, groups, nullptr, stream);
-}
-
-int nq_decode_begin_checked(int dtype, const void* embed, int64_t vocab, int64_t hidden, const int64_t* tok, void* x,
-                            int64_t batch, const int64_t* position, int64_t max_len, const void* table, int64_t row,
-                            void* table_out, void* scores, int64_t scores_rows, int64_t groups, uint32_t* fault,
-                            nq_stream_t stream) {
     const char* name = "nq_decode_begin";
     if (dtype != NQ_F16 && dtype != NQ_BF16) return fail(NQ_ERR_DTYPE, "%s: unsupported dtype %d", name, dtype);
     if (batch < 0 || vocab <= 0 || hidden <= 0 || max_len <= 0 || (table && row <= 0) || (scores && (scores_rows < 0 || groups <= 0)))
@@ -926,7 +901,7 @@ int nq_decode_begin_checked(int dtype, const void* embed, int64_t vocab, int64_t
     if (batch == 0) return NQ_OK;
     if (!position || (embed && (!tok || !x)) || (table && !table_out)) return fail(NQ_ERR_INVALID_ARGUMENT, "%s: null pointer", name);
     if (!aligned(embed, 16) || !aligned(x, 16) || !aligned(tok, 8) || !aligned(position, 8) || !aligned(table, 2) ||
-        !aligned(table_out, 2) || !aligned(scores, 16) || !aligned(fault, 4))
+        !aligned(table_out, 2) || !aligned(scores, 16))
         return fail(NQ_ERR_ALIGNMENT, "%s: misaligned operand (embed, x and scores need 16 bytes)", name);
     StepBegin a{};
     a.embed = static_cast<const uint16_t*>(embed);
@@ -945,9 +920,7 @@ int nq_decode_begin_checked(int dtype, const void* embed, int64_t vocab, int64_t
     a.x_blocks = static_cast<int>(x_blocks);
     a.x_pieces = static_cast<int>(pieces);
     a.minus_inf = dtype == NQ_F16 ? 0xFC00u : 0xFF80u;
-    a.fault = fault;
-    int64_t blocks = x_blocks + (table ? 1 : 0) + ceil_div(a.scores_total, 8 * kBeginThreads);
-    if (fault && blocks == 0) blocks = 1;  // to look at the position
+    const int64_t blocks = x_blocks + (table ? 1 : 0) + ceil_div(a.scores_total, 8 * kBeginThreads);
     if (blocks == 0) return NQ_OK;
     if (blocks > INT32_MAX / 2) return fail(NQ_ERR_UNSUPPORTED, "%s: sizes too large", name);
     step_begin_kernel<<<static_cast<unsigned>(blocks), kBeginThreads, 0, as_stream(stream)>>>(a);

@@ -22,7 +22,6 @@ from __future__ import annotations
 import math
 import time
 import warnings
-import weakref
 from dataclasses import dataclass
 
 import torch
@@ -119,13 +118,6 @@ def _pointwise_kernel_takes(x, other) -> bool:
     return (x.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and other.dtype == x.dtype
             and other.device == x.device and x.numel() > 0 and x.shape[-1] % 8 == 0 and x.is_contiguous()
             and other.is_contiguous() and _only_eager(x, other) and x.data_ptr() % 16 == 0 and other.data_ptr() % 16 == 0)
-
-
-def _plain(module, cls) -> bool:
-    """Whether calling ``module`` runs ``cls.forward`` and nothing else: no subclass, no forward of the instance, no hooks."""
-    every = torch.nn.modules.module
-    return (type(module) is cls and "forward" not in vars(module) and not module._forward_hooks
-            and not module._forward_pre_hooks and not every._global_forward_hooks and not every._global_forward_pre_hooks)
 
 
 def silu_mul(gate, up):
@@ -577,9 +569,6 @@ class GraphDecoder:
         self.pos.fill_(T)
         return logits
 
-    def raise_faults(self):
-        """Raise what finished steps have reported."""
-
     def _prompt_logits(self, ids, positions):
         """The logits [B, vocab] of a prompt's last position."""
         return self.model(ids, positions, self.cache)[:, -1]
@@ -599,23 +588,6 @@ class GraphDecoder:
         for _ in range(steps):
             logits = self._step()
         return logits
-
-
-_FREE_FAULT_WORDS = []  # (words, device) of decoders that are gone
-
-
-def _fault_words(owner, device):
-    """Two words of pinned host memory (a numpy array) in which the step's launches leave {token, position} faults, for the
-    host to look at without waiting. A launch in flight may outlive ``owner``, so its words never go back to torch's
-    allocator: another decoder takes them, once the device that may still write them has been waited for."""
-    try:
-        words, used_on = _FREE_FAULT_WORDS.pop()
-        torch.cuda.synchronize(used_on)
-        words[:] = 0
-    except IndexError:
-        words = torch.zeros(2, dtype=torch.int32, pin_memory=True).numpy()
-    weakref.finalize(owner, _FREE_FAULT_WORDS.append, (words, device))
-    return words
 
 
 class FusedDecoder(GraphDecoder):
@@ -640,16 +612,8 @@ class FusedDecoder(GraphDecoder):
     its RMS-norm prologue: torch's linear reads the head's weights, cold after the layers, at a
     fraction of the bandwidth), which writes the float32 logits. One launch before the layers looks up
     the embeddings and prepares the position's rotary row and mask (``nq_decode_begin``), one after the
-    head takes the argmax and advances the position (``nq_decode_end``). The logits a step returns live in a buffer the
-    next step overwrites. Prefill runs the unfused model (it fills the same cache layout; ``attention`` is about the step, a
-    prompt runs ``nq_attention_prefill`` whatever it says), the logits of its last position through the step's norm and
-    head launch as long as those modules are the ones given here, without hooks.
-
-    ``decode`` raises ValueError for steps that do not fit ``max_len``. A step whose token or position a program has set
-    itself (``tok``, ``pos``) out of range reads zeros in their place and stores no token; the next ``decode`` or
-    ``prefill`` then raises RuntimeError, as does ``generate`` at its end.
-
-    Needs the model packed for the ``gemv`` kernel in float16 or bfloat16 and head_dim 128.
+    head takes the argmax and advances the position (``nq_decode_end``). The logits a step returns live in a buffer the next step overwrites. Prefill runs the unfused model (it fills the same cache
+    layout). Needs the model packed for the ``gemv`` kernel in float16 or bfloat16 and head_dim 128.
     """
 
     def __init__(self, model: NanoQuantLlama, batch: int, max_len: int, steps_per_graph: int = 1,
@@ -714,8 +678,6 @@ class FusedDecoder(GraphDecoder):
         if self.pair_order:
             j = torch.arange(D, device=dev)
             self.head_order = (j // 2) + (j % 2) * (D // 2)  # position i of a head holds feature head_order[i]
-        self.faults = _fault_words(self, dev)
-        self.room = max_len - 1  # steps left, if the program has not set the position itself
             self.q_order = (torch.arange(H, device=dev)[:, None] * D + self.head_order).reshape(-1)
             self.k_order = (torch.arange(KV, device=dev)[:, None] * D + self.head_order).reshape(-1)
             half = torch.stack((self.rope_cos[:, : D // 2], self.rope_sin[:, : D // 2]), dim=-1)
@@ -799,21 +761,6 @@ class FusedDecoder(GraphDecoder):
 
     def _head(self, x, out, stream):
         """The final RMS norm folded into the lm_head launch; float32 logits straight from it (with a bias, the
-    def _head_as_built(self) -> bool:
-        """Whether the model's norm and lm_head still are what the step's launch does, with nothing else to run: the modules
-        and weights of the construction, no forward of their own and no hooks."""
-        norm, lin = self.model.model.norm, self.model.lm_head
-
-        def same(weight, kept):  # the very memory (`kept` holds it, so no other tensor lies there)
-            if weight is None or kept is None:
-                return weight is kept
-            return (weight.dtype == kept.dtype and weight.device == kept.device and weight.shape == kept.shape
-                    and weight.stride() == kept.stride() and weight.data_ptr() == kept.data_ptr())
-
-        return (_plain(self.model, NanoQuantLlama) and _plain(norm, RMSNorm) and _plain(lin, nn.Linear)
-                and same(norm.weight, self.norm_weight) and same(lin.weight, self.head_weight)
-                and same(lin.bias, self.head_bias))
-
         dtype logits, the bias added in dtype, then widened, as the torch head rounds). x [batch, hidden]."""
         hw = self.head_weight
         self._check(self.lib.nq_dense_gemv(self.dcode, hw.data_ptr(), x.data_ptr(), self.norm_weight.data_ptr(),
@@ -822,11 +769,7 @@ class FusedDecoder(GraphDecoder):
         return out if self.head_bias is None else (out + self.head_bias).float()
 
     def _prompt_logits(self, ids, positions):
-        # the last position's logits only, through the step's norm and lm_head launch; a model that does more there (hooks,
-        # another norm or head, a forward of its own) runs whole
-        if not self._head_as_built():
-            return super()._prompt_logits(ids, positions)
-
+        # the last position's logits only, through the step's norm and lm_head launch
         def head(x):
             last = x[:, -1].contiguous()
             out = torch.empty_like(self.logits if self.head_bias is None else self.logits16)
@@ -855,11 +798,10 @@ class FusedDecoder(GraphDecoder):
         if not plain:
             torch.index_select(embed, 0, self.tok, out=self.x)
         table, scores = (self.rope_table, self.scores_all) if self.attention == "torch" else (None, None)
-        self._check(lib.nq_decode_begin_checked(
+        self._check(lib.nq_decode_begin(
             dt, embed.data_ptr() if plain else None, embed.shape[0], s.hidden, self.tok.data_ptr(), self.x.data_ptr(), B, self.pos.data_ptr(),
             self.max_len, self._lib.ptr(table), 0 if table is None else table.shape[1], self.rope_row.data_ptr(),
-            self._lib.ptr(scores), 0 if scores is None else s.layers * B * KV, H // KV, self.faults.ctypes.data, st),
-            "step begin")
+            self._lib.ptr(scores), 0 if scores is None else s.layers * B * KV, H // KV, st), "step begin")
         if self.attention == "torch":
             if self.pair_order:
                 freqs = torch.view_as_complex(self.rope_row.view(1, D // 2, 2))  # cos + i sin of the position
@@ -941,32 +883,9 @@ def generate(model: NanoQuantLlama, prompt: torch.Tensor, max_new_tokens: int, s
                                    attention=attention)
         else:
             decoder = GraphDecoder(model, B, T + max_new_tokens, steps_per_graph, device=prompt.device)
-    def raise_faults(self):
-        if not (self.faults[0] or self.faults[1]):
-            return
-        torch.cuda.synchronize(self.device)  # no launch in flight sets them again
-        token, position = self.faults.tolist()
-        self.faults[:] = 0
-        what = ["a token outside the vocabulary"] * token + [f"a position outside max_len ({self.max_len})"] * position
-        raise RuntimeError(f"an earlier decode step had {' and '.join(what)}: prefill again")
-
-    @torch.no_grad()
-    def decode(self, steps: int, use_graph: bool = True):
-        self.raise_faults()
-        if steps > self.room:  # or the program has set the position back: ask the device
-            pos = int(self.pos)
-            self.room = self.max_len - 1 - pos
-            if steps > self.room:
-                raise ValueError(f"{steps} steps from position {pos} do not fit max_len {self.max_len}")
-        out = super().decode(steps, use_graph)
-        self.room -= max(steps, 0)
-        return out
-
         if use_graph:
             decoder.capture()
-        self.raise_faults()
     steps = max_new_tokens - 1
-        self.room = self.max_len - 1 - prompt.shape[1]
     torch.cuda.synchronize(prompt.device)
     t0 = time.perf_counter()
     decoder.prefill(prompt)
@@ -979,4 +898,3 @@ def generate(model: NanoQuantLlama, prompt: torch.Tensor, max_new_tokens: int, s
     prof = {"prefill_time_s_wall": t1 - t0, "decode_time_s_wall": t2 - t1, "decode_tokens_total": B * steps,
             "ms_per_token": 1e3 * (t2 - t1) / max(steps, 1)}
     return decoder.ids[:, :T + max_new_tokens].clone(), tps, prof
-    decoder.raise_faults()
