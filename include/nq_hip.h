@@ -50,6 +50,8 @@ const char* nq_status_string(int status);
 const char* nq_last_error_message(void);
 /* Library version as 10000*major + 100*minor + patch. */
 int nq_version(void);
+/* Digest of this header as the library was built from it: a caller compiled apart from the library compares its own. */
+const char* nq_header_digest(void);
 
 /* ---------------------------------------------------------------- packing */
 

@@ -9,6 +9,7 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
+import warnings
 
 import torch  # noqa: F401  (must precede the CDLL load, see module docstring)
 
@@ -56,6 +57,7 @@ SIGNATURES = {
     "nq_status_string": (ctypes.c_char_p, [_int]),
     "nq_last_error_message": (ctypes.c_char_p, []),
     "nq_version": (_int, []),
+    "nq_header_digest": (ctypes.c_char_p, []),
     "nq_pack_signs": (_int, [_vp, _vp, _i64, _i64, _int, _vp]),
     "nq_unpack_signs": (_int, [_vp, _vp, _i64, _i64, _int, _vp]),
     "nq_repack_signs": (_int, [_vp, _vp, _i64, _i64, _int, _int, _vp]),
@@ -111,8 +113,16 @@ ops = None  # the C++ operators' library, set by binary_kernels where it registe
 
 
 def _bind_ops(lib: ctypes.CDLL) -> None:
-    """Hand the C++ operators the library's functions."""
+    """Hand the C++ operators the library's functions. Built from another header they stay without, and pass every call
+    on to the operators in Python."""
     if ops is None:
+        return
+    digest = getattr(ops, "nq_ops_header_digest", None)
+    if digest is not None:
+        digest.restype, digest.argtypes = ctypes.c_char_p, []
+    if digest is None or digest() != lib.nq_header_digest():
+        warnings.warn(f"{OPS_PATH} and {LIB_PATH} were built from different headers, so the operators run in Python; "
+                      "run `python -m nanoquant_amd.build`")
         return
     table = (_vp * len(OPS_FUNCTIONS))(*(ctypes.cast(getattr(lib, name), _vp).value for name in OPS_FUNCTIONS))
     bind = ops.nq_ops_bind

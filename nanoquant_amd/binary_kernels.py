@@ -12,7 +12,8 @@ sizes a call is bound by its host path, 24 us through the functions of this modu
 through those. They take every well-formed call; the functions here, registered as the same
 operators of the namespace ``nanoquant_amd``, take the rest: the first call (they load the
 HIP library), empty sizes, and every call to be refused, so that checks and messages stand
-here once. Without a built ``libnq_ops.so`` they serve ``binary_kernels`` directly.
+here once. Without a ``libnq_ops.so``, or with one that cannot be loaded (damaged, or built for
+another torch; a warning says so), they serve ``binary_kernels`` directly.
 
 Argument checks and their messages follow the reference: RuntimeError for
 device/contiguity/dtype/size problems (``cuda_utils.cuh:13-50``,
@@ -27,6 +28,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 
 import torch
 
@@ -264,22 +266,32 @@ def marlin_nanoquant_forward_fake(x, weight_u, weight_v, scale_g, scale_l, scale
 _GENERAL_NS = "nanoquant_amd"
 
 
+def _load_native():
+    """The library of the C++ operators, which registers them as it is loaded, or None."""
+    if not os.path.exists(_lib.OPS_PATH):
+        return None
+    try:
+        return ctypes.CDLL(_lib.OPS_PATH)
+    except OSError as e:
+        warnings.warn(f"{_lib.OPS_PATH} cannot be loaded, so the operators run in Python; run `python -m "
+                      f"nanoquant_amd.build` ({e})")
+        return None
+
+
 def _register():
     ops = ((GEMV_SCHEMA, nanoquant_dyn_forward_cuda, nanoquant_dyn_forward_fake),
            (ONEBIT_SCHEMA, marlin_onebit_forward_cuda, marlin_onebit_forward_fake),
            (NANOQUANT_SCHEMA, marlin_nanoquant_forward_cuda, marlin_nanoquant_forward_fake))
     lib, general = torch.library.Library(_NS, "DEF"), torch.library.Library(_GENERAL_NS, "DEF")
-    native = os.path.exists(_lib.OPS_PATH)
+    _lib.ops = _load_native()
     for schema, cuda, fake in ops:
         name = schema[:schema.index("(")]
         lib.define(schema)
         general.define(schema)
         general.impl(name, cuda, "CUDA")
-        if not native:
+        if _lib.ops is None:
             lib.impl(name, cuda, "CUDA")
         torch.library.register_fake(f"{_NS}::{name}", fake, lib=lib)
-    if native:
-        _lib.ops = ctypes.CDLL(_lib.OPS_PATH)  # registers its implementations as it is loaded
     return lib, general
 
 

@@ -9,6 +9,7 @@ Objects go to ``_build/`` (git-ignored).
 from __future__ import annotations
 
 import concurrent.futures
+import hashlib
 import os
 import shutil
 import subprocess
@@ -19,6 +20,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD_DIR = os.path.join(os.path.dirname(HERE), "_build")
 LIB_NAME = "libnq_hip.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
+HEADER = os.path.join(os.path.dirname(HERE), "include", "nq_hip.h")
 OPS_SOURCE = os.path.join(CSRC, "torch_ops", "nq_ops.cpp")
 OPS_PATH = os.path.join(HERE, "libnq_ops.so")
 ARCH = os.environ.get("NQ_OFFLOAD_ARCH", "gfx950")
@@ -48,13 +50,20 @@ def hipcc() -> str:
     return path
 
 
+def header_digest() -> str:
+    """Define of the C ABI's digest, by which the two libraries tell that they were built from the same header."""
+    with open(HEADER, "rb") as f:
+        return f'-DNQ_HEADER_DIGEST="{hashlib.sha256(f.read()).hexdigest()[:16]}"'
+
+
 def sources():
     return sorted(os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith((".hip", ".cpp")))
 
 
 def _compile(src: str) -> str:
     obj = os.path.join(BUILD_DIR, os.path.basename(src) + ".o")
-    cmd = [hipcc(), *COMMON_FLAGS, *FILE_FLAGS.get(os.path.basename(src), []), "-x", "hip", "-c", src, "-o", obj]
+    cmd = [hipcc(), *COMMON_FLAGS, *FILE_FLAGS.get(os.path.basename(src), []), header_digest(), "-x", "hip", "-c", src,
+           "-o", obj]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"compile failed: {' '.join(cmd)}\n{proc.stdout}\n{proc.stderr}")
@@ -73,7 +82,7 @@ def build_ops() -> str:
     lib_dir = os.path.join(os.path.dirname(torch.__file__), "lib")
     tmp = OPS_PATH + ".tmp"
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", header_digest()]
     for path in cpp_extension.include_paths("cuda"):
         cmd += ["-isystem", path]
     cmd += [OPS_SOURCE, "-o", tmp, f"-L{lib_dir}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip"]

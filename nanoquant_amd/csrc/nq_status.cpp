@@ -44,6 +44,8 @@ const char* nq_last_error_message(void) { return nq::g_last_error; }
 
 int nq_version(void) { return 100; }
 
+const char* nq_header_digest(void) { return NQ_HEADER_DIGEST; }  // of include/nq_hip.h, from the build
+
 }  // extern "C"
 
 // ----------------------------------------------------------------------------- measurement aid

@@ -169,6 +169,9 @@ extern "C" int nq_ops_bind(void* const* functions, int count) {
     return 0;
 }
 
+// Digest of the header that this library was built from, to be compared with nq_header_digest before binding.
+extern "C" const char* nq_ops_header_digest(void) { return NQ_HEADER_DIGEST; }
+
 TORCH_LIBRARY_IMPL(binary_kernels, CUDA, m) {
     m.impl("nanoquant_dyn_forward", &gemv);
     m.impl("marlin_onebit_forward", &onebit);

@@ -298,3 +298,49 @@ def test_repack_marlin_argument_errors_need_no_gpu():
         ku.repack_binary_marlin(torch.zeros(64, 1, dtype=torch.int32), (64, 16), (64, 8))
     with pytest.raises(ValueError, match="Expected"):
         ku.repack_binary_marlin(torch.zeros(64, 2, dtype=torch.int32), (64, 16))
+
+
+def test_an_operator_library_that_cannot_be_loaded_leaves_the_package_usable(tmp_path):
+    """A damaged or foreign libnq_ops.so: the package imports (its builder with it), warns and registers the operators
+    in Python."""
+    import shutil
+    import subprocess
+    import sys
+    shutil.copytree(os.path.join(ROOT, "nanoquant_amd"), tmp_path / "nanoquant_amd",
+                    ignore=shutil.ignore_patterns("*.so", "csrc", "__pycache__"))
+    (tmp_path / "nanoquant_amd" / "libnq_ops.so").write_bytes(b"not a library")
+    code = ("import torch, nanoquant_amd.build; from nanoquant_amd import _lib; assert _lib.ops is None; "
+            "has = torch._C._dispatch_has_kernel_for_dispatch_key; "
+            "assert all(has(f'binary_kernels::{n}', 'CUDA') for n in "
+            "('nanoquant_dyn_forward', 'marlin_onebit_forward', 'marlin_nanoquant_forward'))")
+    run = subprocess.run([sys.executable, "-W", "always", "-c", code], cwd=tmp_path, capture_output=True, text=True,
+                         env=dict(os.environ, PYTHONPATH=str(tmp_path)))
+    assert run.returncode == 0, run.stderr
+    assert "cannot be loaded" in run.stderr
+
+
+def test_an_operator_library_of_another_header_is_not_bound(monkeypatch):
+    class Ops:
+        def __init__(self, digest):
+            self.calls = []
+            if digest is not None:
+                self.nq_ops_header_digest = self._function(digest)
+            self.nq_ops_bind = self._function(0)
+
+        def _function(self, result):
+            def fn(*args):
+                self.calls.append(args)
+                return result
+            return fn
+
+    lib = _lib.load()
+    assert len(lib.nq_header_digest()) == 16
+    for digest, calls in ((b"0123456789abcdef", 1), (None, 0)):
+        ops = Ops(digest)
+        monkeypatch.setattr(_lib, "ops", ops)
+        with pytest.warns(UserWarning, match="different headers"):
+            _lib._bind_ops(lib)
+        assert len(ops.calls) == calls
+    monkeypatch.setattr(_lib, "ops", Ops(lib.nq_header_digest()))
+    _lib._bind_ops(lib)
+    assert len(_lib.ops.calls) == 2
