@@ -403,6 +403,15 @@ int nq_decode_begin(int dtype, const void* embed, int64_t vocab, int64_t hidden,
                     const int64_t* position, int64_t max_len, const void* table, int64_t row, void* table_out, void* scores,
                     int64_t scores_rows, int64_t groups, nq_stream_t stream);
 
+/* nq_decode_begin that reports what it cannot serve: a token outside [0, vocab) (of embed, when it is given) stores 1 at
+ * fault[0], a position outside [0, max_len - 1) 1 at fault[1] (the step's own token goes to the position after it).
+ * `fault`: two words that the device can write, pinned host memory among them, which the host then reads without waiting;
+ * the launch never clears them. */
+int nq_decode_begin_checked(int dtype, const void* embed, int64_t vocab, int64_t hidden, const int64_t* tok, void* x,
+                            int64_t batch, const int64_t* position, int64_t max_len, const void* table, int64_t row,
+                            void* table_out, void* scores, int64_t scores_rows, int64_t groups, uint32_t* fault,
+                            nq_stream_t stream);
+
 /* ---------------------------------------------------------------- measurement aid */
 
 /* Enqueue a one-thread kernel that writes the GPU's constant-rate wall clock to *dst (device

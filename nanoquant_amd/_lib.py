@@ -91,6 +91,8 @@ SIGNATURES = {
     "nq_argmax_rows": (_int, [_vp, _i64, _i64, _i64, _vp, _vp]),
     "nq_decode_end": (_int, [_vp, _i64, _i64, _i64, _vp, _vp, _i64, _vp, _vp, _vp]),
     "nq_decode_begin": (_int, [_int, _vp, _i64, _i64, _vp, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i64, _i64, _vp]),
+    "nq_decode_begin_checked": (_int, [_int, _vp, _i64, _i64, _vp, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i64, _i64,
+                                       _vp, _vp]),
     "nq_gemm_onebit_workspace_bytes": (_size, [_i64, _i64, _i64]),
     "nq_gemm_onebit": (_int, [_int, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _size, _vp]),
     "nq_gemm_nanoquant_workspace_bytes": (_size, [_i64, _i64, _i64, _i64]),

@@ -22,6 +22,7 @@ from __future__ import annotations
 import math
 import time
 import warnings
+import weakref
 from dataclasses import dataclass
 
 import torch
@@ -569,6 +570,9 @@ class GraphDecoder:
         self.pos.fill_(T)
         return logits
 
+    def raise_faults(self):
+        """Raise what finished steps have reported."""
+
     def _prompt_logits(self, ids, positions):
         """The logits [B, vocab] of a prompt's last position."""
         return self.model(ids, positions, self.cache)[:, -1]
@@ -588,6 +592,23 @@ class GraphDecoder:
         for _ in range(steps):
             logits = self._step()
         return logits
+
+
+_FREE_FAULT_WORDS = []  # (words, device) of decoders that are gone
+
+
+def _fault_words(owner, device):
+    """Two words of pinned host memory (a numpy array) in which the step's launches leave {token, position} faults, for the
+    host to look at without waiting. A launch in flight may outlive ``owner``, so its words never go back to torch's
+    allocator: another decoder takes them, once the device that may still write them has been waited for."""
+    try:
+        words, used_on = _FREE_FAULT_WORDS.pop()
+        torch.cuda.synchronize(used_on)
+        words[:] = 0
+    except IndexError:
+        words = torch.zeros(2, dtype=torch.int32, pin_memory=True).numpy()
+    weakref.finalize(owner, _FREE_FAULT_WORDS.append, (words, device))
+    return words
 
 
 class FusedDecoder(GraphDecoder):
@@ -670,6 +691,8 @@ class FusedDecoder(GraphDecoder):
         self.rope_table = torch.cat((self.rope_cos, self.rope_sin), dim=1).contiguous()  # [max_len, 2 D]
         self.tok = torch.zeros(batch, dtype=torch.long, device=dev)  # the step's input token ids
         self.counter = torch.zeros(1, dtype=torch.int32, device=dev)  # nq_decode_end's, zero between launches
+        self.faults = _fault_words(self, dev)
+        self.room = max_len - 1  # steps left, if the program has not set the position itself
         self.step_consts = step_constants(D, dt, dev)
         # the torch step in float16 rotates q and k as one complex product: their features in pair
         # order (feature j of a head, then j + D/2, ...), the cache's keys too (dot products do not
@@ -798,10 +821,11 @@ class FusedDecoder(GraphDecoder):
         if not plain:
             torch.index_select(embed, 0, self.tok, out=self.x)
         table, scores = (self.rope_table, self.scores_all) if self.attention == "torch" else (None, None)
-        self._check(lib.nq_decode_begin(
+        self._check(lib.nq_decode_begin_checked(
             dt, embed.data_ptr() if plain else None, embed.shape[0], s.hidden, self.tok.data_ptr(), self.x.data_ptr(), B, self.pos.data_ptr(),
             self.max_len, self._lib.ptr(table), 0 if table is None else table.shape[1], self.rope_row.data_ptr(),
-            self._lib.ptr(scores), 0 if scores is None else s.layers * B * KV, H // KV, st), "step begin")
+            self._lib.ptr(scores), 0 if scores is None else s.layers * B * KV, H // KV, self.faults.ctypes.data, st),
+            "step begin")
         if self.attention == "torch":
             if self.pair_order:
                 freqs = torch.view_as_complex(self.rope_row.view(1, D // 2, 2))  # cos + i sin of the position
@@ -856,9 +880,32 @@ class FusedDecoder(GraphDecoder):
                     "step end")
         return logits
 
+    def raise_faults(self):
+        if not (self.faults[0] or self.faults[1]):
+            return
+        torch.cuda.synchronize(self.device)  # no launch in flight sets them again
+        token, position = self.faults.tolist()
+        self.faults[:] = 0
+        what = ["a token outside the vocabulary"] * token + [f"a position outside max_len ({self.max_len})"] * position
+        raise RuntimeError(f"an earlier decode step had {' and '.join(what)}: prefill again")
+
+    @torch.no_grad()
+    def decode(self, steps: int, use_graph: bool = True):
+        self.raise_faults()
+        if steps > self.room:  # or the program has set the position back: ask the device
+            pos = int(self.pos)
+            self.room = self.max_len - 1 - pos
+            if steps > self.room:
+                raise ValueError(f"{steps} steps from position {pos} do not fit max_len {self.max_len}")
+        out = super().decode(steps, use_graph)
+        self.room -= max(steps, 0)
+        return out
+
     @torch.no_grad()
     def prefill(self, prompt: torch.Tensor) -> torch.Tensor:
+        self.raise_faults()
         logits = super().prefill(prompt)
+        self.room = self.max_len - 1 - prompt.shape[1]
         self.tok.copy_(self.ids[:, prompt.shape[1]])  # the step's input token, kept on the device
         if self.pair_order:  # the prompt's keys into the step's pair order
             for k_c in self.cache.k:
@@ -894,6 +941,7 @@ def generate(model: NanoQuantLlama, prompt: torch.Tensor, max_new_tokens: int, s
     decoder.decode(steps, use_graph=use_graph)
     torch.cuda.synchronize(prompt.device)
     t2 = time.perf_counter()
+    decoder.raise_faults()
     tps = B * steps / max(t2 - t1, 1e-9)
     prof = {"prefill_time_s_wall": t1 - t0, "decode_time_s_wall": t2 - t1, "decode_tokens_total": B * steps,
             "ms_per_token": 1e3 * (t2 - t1) / max(steps, 1)}

@@ -270,3 +270,75 @@ def test_rope_kv_write_against_torch(dtype, B, heads, kv_heads, D, pos):
     v0[:, :, pos] = v
     assert torch.equal(k_cache, k0)
     assert torch.equal(v_cache, v0)
+
+
+@pytest.fixture(scope="module")
+def fused_model():
+    from nanoquant_amd import _lib
+    _lib.load()
+    return kernel_model(random_llama(FUSED_SHAPES["gqa"], bpw=0.55, seed=19, device="cpu"), "gemv")
+
+
+@pytest.mark.parametrize("use_graph", [False, True], ids=["eager", "graph"])
+@pytest.mark.parametrize("attention", ["torch", "rope", "hip"])
+def test_fused_decode_past_the_end(fused_model, attention, use_graph):
+    """Steps that do not fit max_len are refused before anything runs, also once the program has moved the position; a
+    position set where the step's token has no place is reported by the next call."""
+    from nanoquant_amd.decode import FusedDecoder
+    announce("fused decode past the end", attention, use_graph)
+    dec = FusedDecoder(fused_model, 2, 12, attention=attention)
+    if use_graph:
+        dec.capture()
+    prompt = torch.randint(0, 1000, (2, 8), generator=torch.Generator().manual_seed(2)).cuda()
+    dec.prefill(prompt)
+    with pytest.raises(ValueError, match="max_len"):
+        dec.decode(4, use_graph)
+    assert int(dec.pos) == 8
+    dec.decode(3, use_graph)
+    with pytest.raises(ValueError, match="max_len"):
+        dec.decode(1, use_graph)
+    assert int(dec.pos) == 11
+    dec.pos.fill_(8)  # set back by the program: steps fit again
+    dec.tok.copy_(dec.ids[:, 8])
+    for _ in range(3):
+        dec.decode(1, use_graph)
+    dec.prefill(prompt[:, :4])
+    dec.pos.fill_(11)  # a cache row, but no place for the token after it
+    dec.decode(1, use_graph)
+    torch.cuda.synchronize()
+    with pytest.raises(RuntimeError, match="position"):
+        dec.decode(1, use_graph)
+    dec.prefill(prompt)
+    dec.decode(1, use_graph)
+    torch.cuda.synchronize()
+    dec.raise_faults()
+
+
+@pytest.mark.parametrize("use_graph", [False, True], ids=["eager", "graph"])
+def test_fused_decode_reports_tokens_outside_the_vocabulary(fused_model, use_graph):
+    from nanoquant_amd.decode import FusedDecoder
+    announce("fused decode tokens", use_graph)
+    dec = FusedDecoder(fused_model, 2, 16, attention="hip")
+    if use_graph:
+        dec.capture()
+    prompt = torch.randint(0, 1000, (2, 8), generator=torch.Generator().manual_seed(2)).cuda()
+    for token in (-1, 1000):
+        for call in (lambda: dec.decode(1, use_graph), lambda: dec.prefill(prompt)):
+            dec.prefill(prompt)
+            dec.tok[1] = token
+            dec.decode(1, use_graph)
+            torch.cuda.synchronize()
+            with pytest.raises(RuntimeError, match="token"):
+                call()
+    dec.prefill(prompt)
+    dec.tok.fill_(999)
+    dec.decode(1, use_graph)
+    torch.cuda.synchronize()
+    dec.raise_faults()
+    words = dec.faults
+    words[0] = 1
+    del dec
+    import gc
+    gc.collect()
+    again = FusedDecoder(fused_model, 2, 16, attention="hip")  # takes words that are clear, its own or a gone decoder's
+    again.raise_faults()

@@ -89,3 +89,28 @@ def test_step_begin(lib, batch, hidden, L, groups, rows, row, dtype):
         x.fill_(0)
         begin(True, True, True)
         assert torch.equal(x[:batch], embed[tok])
+
+
+@pytest.mark.parametrize("embed", [True, False], ids=["embed", "none"])
+@pytest.mark.parametrize("table", [True, False], ids=["table", "none"])
+def test_step_begin_reports(lib, embed, table):
+    """Tokens and positions outside their ranges into pinned host words, the first and last good values not."""
+    from nanoquant_amd import _lib
+    print("\n[case] step begin reports", embed, table, flush=True)
+    vocab, hidden, L, row, B = 50, 2056, 9, 16, 3
+    weights, rows = torch.randn(vocab, hidden, device="cuda").half(), torch.randn(L, row, device="cuda").half()
+    x, out = torch.zeros(B, hidden, device="cuda").half(), torch.zeros(row, device="cuda").half()
+    fault = torch.zeros(2, dtype=torch.int32, pin_memory=True)
+    for tokens, p, want in (([0, 49, 3], 0, (0, 0)), ([0, 49, 3], L - 2, (0, 0)), ([0, 50, 3], 1, (1, 0)),
+                            ([0, 1, -1], 1, (1, 0)), ([0, 1, 2], L - 1, (0, 1)), ([0, 1, 2], -1, (0, 1)),
+                            ([-5, 1, 2], 2 ** 40, (1, 1))):
+        tok, pos = torch.tensor(tokens, device="cuda"), torch.tensor([p], device="cuda")
+        fault.zero_()
+        _lib.check(lib.nq_decode_begin_checked(
+            _lib.NQ_F16, weights.data_ptr() if embed else None, vocab, hidden, tok.data_ptr(), x.data_ptr(), B,
+            pos.data_ptr(), L, rows.data_ptr() if table else None, row, out.data_ptr(), None, 0, 1, fault.data_ptr(),
+            _lib.stream_of(x.device)), "begin")
+        torch.cuda.synchronize()
+        assert fault.tolist() == [want[0] if embed else 0, want[1]], (tokens, p)
+    assert lib.nq_decode_begin_checked(_lib.NQ_F16, None, vocab, hidden, None, None, B, pos.data_ptr(), L, None, 0, None,
+                                       None, 0, 1, fault.data_ptr() + 1, None) == _lib.NQ_ERR_ALIGNMENT
