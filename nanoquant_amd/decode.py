@@ -121,6 +121,13 @@ def _pointwise_kernel_takes(x, other) -> bool:
             and other.is_contiguous() and _only_eager(x, other) and x.data_ptr() % 16 == 0 and other.data_ptr() % 16 == 0)
 
 
+def _plain(module, cls) -> bool:
+    """Whether calling ``module`` runs ``cls.forward`` and nothing else: no subclass, no forward of the instance, no hooks."""
+    every = torch.nn.modules.module
+    return (type(module) is cls and "forward" not in vars(module) and not module._forward_hooks
+            and not module._forward_pre_hooks and not every._global_forward_hooks and not every._global_forward_pre_hooks)
+
+
 def silu_mul(gate, up):
     """silu(gate) * up, rounded after the silu and after the product: one launch of the HIP library for
     contiguous float16 or bfloat16 tensors on the GPU, torch ops otherwise."""
@@ -633,8 +640,16 @@ class FusedDecoder(GraphDecoder):
     its RMS-norm prologue: torch's linear reads the head's weights, cold after the layers, at a
     fraction of the bandwidth), which writes the float32 logits. One launch before the layers looks up
     the embeddings and prepares the position's rotary row and mask (``nq_decode_begin``), one after the
-    head takes the argmax and advances the position (``nq_decode_end``). The logits a step returns live in a buffer the next step overwrites. Prefill runs the unfused model (it fills the same cache
-    layout). Needs the model packed for the ``gemv`` kernel in float16 or bfloat16 and head_dim 128.
+    head takes the argmax and advances the position (``nq_decode_end``). The logits a step returns live in a buffer the
+    next step overwrites. Prefill runs the unfused model (it fills the same cache layout; ``attention`` is about the step, a
+    prompt runs ``nq_attention_prefill`` whatever it says), the logits of its last position through the step's norm and
+    head launch as long as those modules are the ones given here, without hooks.
+
+    ``decode`` raises ValueError for steps that do not fit ``max_len``. A step whose token or position a program has set
+    itself (``tok``, ``pos``) out of range reads zeros in their place and stores no token; the next ``decode`` or
+    ``prefill`` then raises RuntimeError, as does ``generate`` at its end.
+
+    Needs the model packed for the ``gemv`` kernel in float16 or bfloat16 and head_dim 128.
     """
 
     def __init__(self, model: NanoQuantLlama, batch: int, max_len: int, steps_per_graph: int = 1,
@@ -791,8 +806,27 @@ class FusedDecoder(GraphDecoder):
                                            self.batch, hw.shape[1], hw.shape[0], out.shape[1], stream), "lm_head")
         return out if self.head_bias is None else (out + self.head_bias).float()
 
+    def _head_as_built(self) -> bool:
+        """Whether the model's norm and lm_head still are what the step's launch does, with nothing else to run: the modules
+        and weights of the construction, no forward of their own and no hooks."""
+        norm, lin = self.model.model.norm, self.model.lm_head
+
+        def same(weight, kept):  # the very memory (`kept` holds it, so no other tensor lies there)
+            if weight is None or kept is None:
+                return weight is kept
+            return (weight.dtype == kept.dtype and weight.device == kept.device and weight.shape == kept.shape
+                    and weight.stride() == kept.stride() and weight.data_ptr() == kept.data_ptr())
+
+        return (_plain(self.model, NanoQuantLlama) and _plain(norm, RMSNorm) and _plain(lin, nn.Linear)
+                and same(norm.weight, self.norm_weight) and same(lin.weight, self.head_weight)
+                and same(lin.bias, self.head_bias))
+
     def _prompt_logits(self, ids, positions):
-        # the last position's logits only, through the step's norm and lm_head launch
+        # the last position's logits only, through the step's norm and lm_head launch; a model that does more there (hooks,
+        # another norm or head, a forward of its own) runs whole
+        if not self._head_as_built():
+            return super()._prompt_logits(ids, positions)
+
         def head(x):
             last = x[:, -1].contiguous()
             out = torch.empty_like(self.logits if self.head_bias is None else self.logits16)

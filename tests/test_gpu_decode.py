@@ -342,3 +342,50 @@ def test_fused_decode_reports_tokens_outside_the_vocabulary(fused_model, use_gra
     gc.collect()
     again = FusedDecoder(fused_model, 2, 16, attention="hip")  # takes words that are clear, its own or a gone decoder's
     again.raise_faults()
+
+
+@torch.no_grad()
+def test_fused_prefill_runs_what_the_model_has_at_its_end(fused_model):
+    """Hooks on the norm, the head and the model, a head replaced after construction and a model with a forward of its own:
+    the prompt's logits are the model's."""
+    from nanoquant_amd.decode import FusedDecoder, NanoQuantLlama
+    announce("fused prefill ends")
+
+    class Own(NanoQuantLlama):
+        def forward(self, ids, positions, cache):
+            return super().forward(ids, positions, cache) + 1.0
+
+    model = copy.deepcopy(fused_model)
+    dec = FusedDecoder(model, 2, 16, attention="hip")
+    prompt = torch.randint(0, 1000, (2, 8), generator=torch.Generator().manual_seed(2)).cuda()
+
+    def both():
+        want = model(prompt, torch.arange(8, device="cuda"), dec.cache)[:, -1]
+        got = dec.prefill(prompt)
+        assert got.shape == want.shape and got.dtype == want.dtype
+        return got, want
+
+    def close(got, want):  # the head's launch sums in another order than torch's linear, both round to float16
+        return float((got - want).abs().max() / want.abs().max()) <= 2e-3
+
+    plain, want = both()
+    assert dec._head_as_built() and close(plain, want)
+    hooks = (lambda: model.model.norm.register_forward_hook(lambda m, a, y: y * 2),
+             lambda: model.lm_head.register_forward_pre_hook(lambda m, a: (a[0] * 2,)),
+             lambda: model.register_forward_hook(lambda m, a, y: y * 2))
+    for add in hooks:
+        handle = add()
+        got, want = both()
+        assert torch.equal(got, want) and close(got, 2 * plain)
+        handle.remove()
+    head = model.lm_head
+    model.lm_head = copy.deepcopy(head)
+    model.lm_head.weight.data.mul_(2)
+    got, want = both()
+    assert torch.equal(got, want) and close(got, 2 * plain)
+    model.lm_head = head
+    model.__class__ = Own
+    got, want = both()
+    assert torch.equal(got, want) and close(got, plain + 1)
+    model.__class__ = NanoQuantLlama
+    assert torch.equal(dec.prefill(prompt), plain)
