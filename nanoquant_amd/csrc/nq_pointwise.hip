@@ -21,10 +21,10 @@ __device__ inline uint32_t halves(uint32_t a, uint32_t b, F f) {
 }
 
 // One block per row of n = 8 c columns, CH 16-byte chunks a thread held in registers between the sum and the
-// scaling: y = T(g * T(x * rsqrt(mean(x^2) + eps))), mean and first product in fp32.
+// scaling: y = T(g * T(x * rsqrt(mean(x^2) + eps))), mean and first product in fp32. y may be x.
 template <typename T, int CH>
-__global__ __launch_bounds__(kThreads) void rms_norm_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ g,
-                                                            uint16_t* __restrict__ y, int n, float eps) {
+__global__ __launch_bounds__(kThreads) void rms_norm_kernel(const uint16_t* x, const uint16_t* __restrict__ g, uint16_t* y,
+                                                            int n, float eps) {
     __shared__ float part[kThreads / 64];
     const int t = threadIdx.x;
     const size_t row = static_cast<size_t>(blockIdx.x) * static_cast<size_t>(n);
@@ -67,10 +67,9 @@ __global__ __launch_bounds__(kThreads) void rms_norm_kernel(const uint16_t* __re
     }
 }
 
-// y = T(T(silu(gate)) * up), silu in fp32; eight elements a thread.
+// y = T(T(silu(gate)) * up), silu in fp32; eight elements a thread. y may be gate or up.
 template <typename T>
-__global__ __launch_bounds__(kThreads) void silu_mul_kernel(const uint16_t* __restrict__ gate,
-                                                            const uint16_t* __restrict__ up, uint16_t* __restrict__ y,
+__global__ __launch_bounds__(kThreads) void silu_mul_kernel(const uint16_t* gate, const uint16_t* up, uint16_t* y,
                                                             int64_t chunks) {
     const int64_t c = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     if (c >= chunks) return;

@@ -65,3 +65,25 @@ def test_other_forms_keep_torch_ops():
     out = torch.func.vmap(lambda a: silu_mul(a, a))(x)
     assert torch.equal(out, F.silu(x) * x)
     assert silu_mul(x[:, :1], x).shape == (4, 64)  # torch's broadcasting
+
+
+@DTYPES
+@pytest.mark.parametrize("shape", [(3, 2040), (300, 8192), (2, 16384)])
+def test_in_place(shape, dtype):
+    """The C functions with their output in an input's place: bit for bit what they give elsewhere."""
+    from nanoquant_amd import _lib
+    print("\n[case] pointwise in place", shape, dtype, flush=True)
+    lib, dt = _lib.load(), _lib.dtype_code(dtype)
+    a, b = (torch.randn(shape, device="cuda").to(dtype) for _ in range(2))
+    norm = RMSNorm(shape[-1], 1e-5, "cuda", dtype)
+    want = norm(a)
+    y = a.clone()
+    _lib.check(lib.nq_rms_norm(dt, y.data_ptr(), norm.weight.data_ptr(), y.data_ptr(), shape[0], shape[1], 1e-5,
+                               _lib.stream_of(y.device)), "rms_norm")
+    assert torch.equal(y, want)
+    want = silu_mul(a, b)
+    for k in range(2):
+        pair = [a.clone(), b.clone()]
+        _lib.check(lib.nq_silu_mul(dt, pair[0].data_ptr(), pair[1].data_ptr(), pair[k].data_ptr(), a.numel(),
+                                   _lib.stream_of(a.device)), "silu_mul")
+        assert torch.equal(pair[k], want)
