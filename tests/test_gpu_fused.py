@@ -520,3 +520,33 @@ def test_argmax_rows_argument_errors(lib):
     assert f(xp, 2, 64, 64, op + 4, None) == _lib.NQ_ERR_ALIGNMENT
     assert f(None, 2, 64, 64, op, None) == _lib.NQ_ERR_INVALID_ARGUMENT
     assert f(None, 0, 64, 64, None, None) == _lib.NQ_OK  # no rows
+
+
+@pytest.mark.parametrize("G", [1, 4])
+@pytest.mark.parametrize("pos", [1022, 1023, 1024, 2047])
+def test_attention_decode_long(lib, G, pos):
+    """One, just one and two rounds of sixteen chunks in the combine, against float64."""
+    from nanoquant_amd import _lib
+    announce("attention long", G, pos)
+    B, KV, D, L = 2, 2, 128, 2100
+    H = KV * G
+    W = (H + 2 * KV) * D
+    gen = torch.Generator(device="cuda").manual_seed(G + pos)
+    qkv = torch.randn(B, W, generator=gen, device="cuda").half()
+    kc, vc = (torch.randn(B, KV, L, D, generator=gen, device="cuda").half() for _ in range(2))
+    cos, sin = torch.ones(L, D, device="cuda").half(), torch.zeros(L, D, device="cuda").half()
+    out = torch.zeros(B, H * D, dtype=torch.float16, device="cuda")
+    at = torch.tensor([pos], device="cuda")
+    ws = torch.empty(lib.nq_attention_decode_workspace_bytes(B, H, KV, D, L), dtype=torch.uint8, device="cuda")
+    p0 = qkv.data_ptr()
+    _lib.check(lib.nq_attention_decode(_lib.NQ_F16, p0, p0 + 2 * H * D, p0 + 2 * (H + KV) * D, W, kc.data_ptr(),
+                                       vc.data_ptr(), cos.data_ptr(), sin.data_ptr(), at.data_ptr(), out.data_ptr(), B, H,
+                                       KV, D, L, D ** -0.5, ws.data_ptr(), ws.numel(),
+                                       torch.cuda.current_stream().cuda_stream), "attention")
+    torch.cuda.synchronize()
+    q = qkv[:, :H * D].cpu().double().view(B, KV, G, 1, D)
+    keys, vals = (c[:, :, :pos + 1].cpu().double().unsqueeze(2) for c in (kc, vc))
+    p = torch.softmax((q * keys).sum(-1) * D ** -0.5, dim=-1)
+    want = (p.unsqueeze(-1) * vals).sum(3).reshape(B, H * D).numpy()
+    err = rel(out, want)
+    assert err <= 2e-3, err
