@@ -348,15 +348,16 @@ void rows_kernel(const RowsArgs a, int q_tiles, int p_tiles, int split_steps, in
                             uint2{lo[0] | (uint32_t(lo[1]) << 16), lo[2] | (uint32_t(lo[3]) << 16)};
                     }
                 }
-        if (pt == 0) {  // the columns past kpad that stage 2 reads
-            const int width = a.zpitch - a.kpad;
-            for (int e = t; e < width * BQ; e += NT) {
-                const int q = e / width;
-                if (q0 + q < a.batch) {
-                    const size_t at = static_cast<size_t>(q0 + q) * a.zpitch + a.kpad + (e - q * width);
-                    a.z_hi[at] = 0;
-                    a.z_lo[at] = 0;
-                }
+        // the columns past kpad that stage 2 reads, in 16-byte pieces (kpad % 32 == 0, zpitch % 64 == 0), shared by the
+        // blocks of the batch rows (r = 544, which has 224 such columns, n = 1472, 513 rows: 15.0 us, 26.8 with 2-byte
+        // stores of the first block alone)
+        const int pieces = (a.zpitch - a.kpad) / 8;
+        for (int e = pt * NT + t; e < pieces * BQ; e += p_tiles * NT) {
+            const int q = e / pieces;
+            if (q0 + q < a.batch) {
+                const size_t at = static_cast<size_t>(q0 + q) * a.zpitch + a.kpad + 8 * (e - q * pieces);
+                *reinterpret_cast<u32x4*>(a.z_hi + at) = u32x4{0u, 0u, 0u, 0u};
+                *reinterpret_cast<u32x4*>(a.z_lo + at) = u32x4{0u, 0u, 0u, 0u};
             }
         }
         return;

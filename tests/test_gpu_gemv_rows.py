@@ -31,6 +31,7 @@ CASES = [
     (300, 40960, 300, 64, False),     # the same in several k ranges
     (64, 53248, 96, 100, True),
     (130, 33024, 65, 200, False),
+    (132, 1472, 544, 513, True),      # many columns past the rank, zeroed by the blocks of two row tiles
 ]
 
 
@@ -117,6 +118,48 @@ def test_rows_run_on_the_longest_inputs(lib, rows):
     print("\n[case] gemv rows, time", rows, flush=True)
     few, many = _stage1_us(lib, 32, 53248, 1632), _stage1_us(lib, rows, 53248, 1632)
     assert many < 8 * few, f"{rows} rows take {many:.0f} us, 32 rows {few:.0f}"
+
+
+def _graph_us(launch, count=16):
+    """Microseconds of one launch among `count` in a graph, the least of five replays."""
+    launch()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for _ in range(count):
+            launch()
+    times = []
+    for _ in range(6):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        graph.replay()
+        end.record()
+        torch.cuda.synchronize()
+        times.append(start.elapsed_time(end) * 1000 / count)
+    return min(times[1:])
+
+
+def _stage_us(lib, stage, rows, n, r, m):
+    from nanoquant_amd import _lib
+    half = lambda *s: torch.rand(*s, device="cuda").half()  # noqa: E731
+    words = lambda a, b: torch.randint(-2 ** 31, 2 ** 31 - 1, (a, (b + 31) // 32), dtype=torch.int32, device="cuda")  # noqa: E731
+    x, s_in, s_out, V, U, y = half(rows, n), half(n), half(m), words(r, n), words(m, r), half(rows, m)
+    nbytes = lib.nq_gemv_workspace_bytes(rows, n, r, m)
+    ws = torch.zeros(nbytes, dtype=torch.uint8, device="cuda")
+    if stage == 1:
+        return _graph_us(lambda: _lib.check(lib.nq_gemv_stage1(
+            _lib.NQ_F16, x.data_ptr(), s_in.data_ptr(), V.data_ptr(), None, rows, n, r, m, ws.data_ptr(), nbytes,
+            torch.cuda.current_stream().cuda_stream), "stage 1"))
+    return _graph_us(lambda: _lib.check(lib.nq_gemv_stage2(
+        _lib.NQ_F16, U.data_ptr(), s_out.data_ptr(), y.data_ptr(), rows, n, r, m, ws.data_ptr(), nbytes,
+        torch.cuda.current_stream().cuda_stream), "stage 2"))
+
+
+def test_rows_time_does_not_jump_with_the_sizes_beside(lib):
+    """Ranks with many columns to zero (r = 544; took twice the time of r = 512) cost little more than their neighbours."""
+    print("\n[case] gemv rows, neighbours", flush=True)
+    a, b = (_stage_us(lib, 1, 513, 1472, r, 64) for r in (512, 544))
+    assert b < 1.4 * a, (a, b)
 
 
 @pytest.mark.parametrize("offset", [1, 4])
