@@ -45,7 +45,7 @@ __device__ inline float of_bf16(uint16_t b) { return __uint_as_float(static_cast
 
 template <typename T, typename TO, bool kS2, int BP, int BQ, int CW, int KS>
 __global__ __launch_bounds__(BP * KS) __attribute__((amdgpu_waves_per_eu(2)))
-void rows_kernel(const RowsArgs a, int q_tiles, int p_tiles, int split_steps, int splits, int vec8) {
+void rows_kernel(const RowsArgs a, int q_tiles, int p_tiles, int split_steps, int splits, int vec) {
     constexpr int NX = kS2 ? 2 : 1;  // x, or z_hi and z_lo
     constexpr int NW = BP / 64;  // waves of a k group
     constexpr int NT = NW * 64;
@@ -388,8 +388,11 @@ void rows_kernel(const RowsArgs a, int q_tiles, int p_tiles, int split_steps, in
             const int o = f0 + 8 * (lane & 7);
             if (q < a.batch && o < a.rows) {
                 uint16_t* dst = a.y + static_cast<size_t>(q) * a.rows + o;
-                if (vec8) {
+                if (vec == 8) {
                     *reinterpret_cast<u32x4*>(dst) = d;
+                } else if (vec == 4) {
+                    *reinterpret_cast<uint2*>(dst) = uint2{d.x, d.y};
+                    if (o + 4 < a.rows) *reinterpret_cast<uint2*>(dst + 4) = uint2{d.z, d.w};
                 } else {
                     const uint32_t w[4] = {d.x, d.y, d.z, d.w};
 #pragma unroll
@@ -405,9 +408,11 @@ template <typename T, typename TO, bool kS2, int BP, int BQ, int CW, int KS>
 void launch_tile(const RowsArgs& a, const RowsPlan& p, hipStream_t st) {
     const int q_tiles = static_cast<int>(ceil_div(a.batch, BQ));
     const int p_tiles = static_cast<int>(ceil_div(a.rows, BP));
-    const int vec8 = kS2 && a.rows % 8 == 0 && aligned(a.y, 16);
+    // elements of y per store: its rows whole 16- or 8-byte pieces (m = 9804, r = 384 at 579 rows 12.2
+    // us, 21.8 in 2-byte stores)
+    const int vec = !kS2 ? 0 : a.rows % 8 == 0 && aligned(a.y, 16) ? 8 : a.rows % 4 == 0 && aligned(a.y, 8) ? 4 : 0;
     rows_kernel<T, TO, kS2, BP, BQ, CW, KS><<<dim3(static_cast<unsigned>(q_tiles * p_tiles * p.splits)), BP * KS, 0, st>>>(
-        a, q_tiles, p_tiles, p.split_steps, p.splits, vec8);
+        a, q_tiles, p_tiles, p.split_steps, p.splits, vec);
 }
 
 // Stage 1 runs these kernels on rows of 512 words or more from 33 batch rows, of 256-511 words from 64,

@@ -32,6 +32,7 @@ CASES = [
     (64, 53248, 96, 100, True),
     (130, 33024, 65, 200, False),
     (132, 1472, 544, 513, True),      # many columns past the rank, zeroed by the blocks of two row tiles
+    (9804, 256, 384, 579, False),     # outputs of whole 8-byte stores
 ]
 
 
@@ -156,10 +157,13 @@ def _stage_us(lib, stage, rows, n, r, m):
 
 
 def test_rows_time_does_not_jump_with_the_sizes_beside(lib):
-    """Ranks with many columns to zero (r = 544; took twice the time of r = 512) cost little more than their neighbours."""
+    """Ranks with many columns to zero (r = 544; took twice the time of r = 512) and outputs that are not whole 16-byte
+    stores (m = 9804; took 1.5 times the time of m = 9808) cost little more than their neighbours."""
     print("\n[case] gemv rows, neighbours", flush=True)
     a, b = (_stage_us(lib, 1, 513, 1472, r, 64) for r in (512, 544))
     assert b < 1.4 * a, (a, b)
+    a, b = (_stage_us(lib, 2, 579, 256, 384, m) for m in (9808, 9804))
+    assert b < 1.25 * a, (a, b)
 
 
 @pytest.mark.parametrize("offset", [1, 4])
