@@ -425,10 +425,12 @@ constexpr int64_t kWideWords = 512, kWideBatch = 33;
 constexpr int64_t kMidWords = 256, kMidBatch = 64;
 constexpr int64_t kNarrowBatch = 129;
 // On rows of up to 256 words the MFMA kernel also stays while its grid is one round of blocks (of 64
-// features x 16 batch rows up to 128 words, of 32 beyond), its time then being that of one block (n =
-// 4096, r = 1120 at 200 rows 13.2 against 13.9; at 300 rows, two rounds, 25.0 against 15.5; n = 8192, r =
-// 512 at 200 / 300 rows 12.7 / 13.3, 24.3 / 15.7).
-constexpr int64_t kMfmaRoundWords = 256, kMfmaRoundBlocks = 256;
+// features x 16 batch rows as long as 64 rows of words fit its LDS, of 32 beyond), its time then being that of
+// one block (n = 4096, r = 1120 at 200 rows 13.2 against 13.9; at 300 rows, two rounds, 25.0 against 15.5; n =
+// 4224, r = 1536 at 129 rows 11.7 / 15.5; n = 8192, r = 512 at 200 / 300 rows 12.7 / 13.3, 24.3 / 15.7), and on
+// somewhat longer ones where n % 64 columns would be a tail here (n = 8432, r = 768 at 140 rows 13.0 / 17.1; n =
+// 11560, r = 800 at 78 12.8 / 16.6; without a tail 14 / 12 on average there).
+constexpr int64_t kMfmaWords64 = 204, kMfmaRoundWords = 256, kMfmaTailWords = 376, kMfmaRoundBlocks = 256;
 constexpr int64_t kMinColumns = 512;               // shorter rows are not worth a pipeline
 constexpr int64_t kMaxSplits = 16, kMinSteps = 5;  // k ranges, and 64-k steps of the shortest
 
@@ -447,8 +449,8 @@ bool rows_stage1_plan(int64_t batch, int64_t n, int64_t r, int64_t kpad, size_t 
     const int64_t words = ceil_div(n, 32);
     const int64_t from = words >= kWideWords ? kWideBatch : (words >= kMidWords ? kMidBatch : kNarrowBatch);
     if (batch < from || n % 8 || n < kMinColumns || r <= 0) return false;
-    if (batch >= kNarrowBatch && words <= kMfmaRoundWords &&
-        ceil_div(r, words <= 128 ? 64 : 32) * ceil_div(batch, 16) <= kMfmaRoundBlocks)
+    const bool mfma_round = ceil_div(r, words <= kMfmaWords64 ? 64 : 32) * ceil_div(batch, 16) <= kMfmaRoundBlocks;
+    if (mfma_round && ((words <= kMfmaRoundWords && batch >= kNarrowBatch) || (words <= kMfmaTailWords && n % 64 != 0)))
         return false;
     const int64_t steps = n / 64;
     struct Shape {

@@ -13,13 +13,20 @@ pytestmark = pytest.mark.gpu
 # rounding is counted apart (half a unit in the last place).
 BAR = 2.0 ** -11 + 1e-4
 
-# (m, n, r, rows, s_mid): narrow inputs run from 129 rows (unless one round of the 16-row MFMA kernel
-# does), 256-511 words from 64, 512 words or more from 33
+# (m, n, r, rows, s_mid): narrow inputs run from 129 rows, 256-511 words from 64, 512 words or more from 33, but for
+# a small V (the k-split kernel, up to 96 rows) and where one round of the 16-row MFMA kernel does
 CASES = [
-    (300, 8192, 70, 64, True),        # the first batch on 256 words; ragged rank and outputs, k ranges
-    (64, 16384, 1, 33, True),         # the first batch on 512 words; a rank of 1
-    (1000, 8200, 130, 65, False),     # n % 64 == 8: the tail tile's first quarter; a second row tile of one row
-    (129, 8248, 257, 100, True),      # n % 64 == 56; outputs that are not whole 16-byte stores
+    (300, 8192, 3200, 64, True),      # the first batch on 256 words; ragged outputs, k ranges
+    (64, 16384, 2750, 33, True),      # the first batch on 512 words; a ragged rank
+    (64, 16392, 1, 33, True),         # a rank of 1
+    (1000, 12296, 130, 65, False),    # n % 64 == 8: the tail tile's first quarter; a second row tile of one row
+    (129, 12344, 257, 100, True),     # n % 64 == 56; outputs that are not whole 16-byte stores
+    (300, 8192, 70, 64, True),        # the sizes beside these that other kernels take
+    (64, 16384, 1, 33, True),
+    (1000, 8200, 130, 65, False),
+    (129, 8248, 257, 100, True),
+    (600, 4224, 1536, 129, True),     # 132 words, one round of the MFMA kernel
+    (600, 4224, 2080, 129, True),     # and more than one
     (72, 16416, 96, 127, False),      # n % 64 == 32
     (4096, 11008, 1632, 96, True),    # several k ranges over k groups
     (520, 4096, 1632, 630, False),    # four k groups, no k range
@@ -28,7 +35,8 @@ CASES = [
     (8100, 1024, 2000, 161, False),   # stage 2 in blocks of 32 rows, the last one of one row; a ragged last tile
     (2048, 1024, 2240, 2048, True),   # 256-feature tiles on every CU, one range
     (72, 33032, 130, 33, True),       # rows of more than 1024 words (n > 32768), n % 64 == 8
-    (300, 40960, 300, 64, False),     # the same in several k ranges
+    (300, 40960, 300, 64, False),     # (the k-split kernel keeps this one)
+    (300, 40960, 700, 64, False),     # several k ranges
     (64, 53248, 96, 100, True),
     (130, 33024, 65, 200, False),
     (132, 1472, 544, 513, True),      # many columns past the rank, zeroed by the blocks of two row tiles
