@@ -2649,17 +2649,20 @@ inline bool s2b_chosen(int batch, int m, const Plan& plan, int items = 1) {
 // at 4 9.5 / 9.9).
 // Pair, from three batch rows: s2t_kernel holds half as many batch rows a pass (m = 11008, r = 1632 at 2 / 3 rows 6.7 /
 // 8.1, 9.5 / 8.0; m = 4096, r = 1632 at 4 / 6 rows 5.2 / 5.4, 7.15 / 5.4), and beyond 16 but for the largest U (m =
-// 28672, r = 3520 at 32 rows 42.9 / 43.4; m = 11008, r = 2976 23.0 / 20.0); the largest U from two (24.4 / 20.9).
+// 28672, r = 3520 at 32 rows 42.9 / 43.4; m = 11008, r = 2976 23.0 / 20.0); the largest U from two (24.4 / 20.9). Beyond 16
+// batch rows not on fewer than 1200 rows either, whose few blocks run four column tiles each (m = 672, r = 1984 at 24 rows
+// 5.5 / 8.2, m = 1137, r = 1568 at 20 7.0 / 7.7).
 constexpr int64_t kSplitWork = 3500000, kSplitPairWork = 900000, kSplitPairOnePassWork = 1500000;
 constexpr int64_t kSplitLargeWords = 3000000;
 constexpr int kSplitTallRows = 16384, kSplitWideRows = 8192, kSplitWideWords = 64;
+constexpr int kSplitPairRows = 1200;
 inline bool split_chosen(int batch, int m, const Plan& plan, int items = 1) {
     if (batch < 2 || batch > kSplitMaxBatch || plan.s2_qw == 0 || plan.wr > kSplitMaxWords) return false;
     const int64_t words = static_cast<int64_t>(m) * plan.wr, work = words * batch;
     const int64_t passes = ceil_div(batch, s2t_rows_per_pass(batch, items * plan.s2_qw));
     if (items == 2) {
         if (batch <= 2) return words >= kSplitLargeWords;
-        if (batch > 16 && words >= kSplitLargeWords) return false;
+        if (batch > 16 && (words >= kSplitLargeWords || m < kSplitPairRows)) return false;
         return work >= (passes >= 2 ? kSplitPairWork : kSplitPairOnePassWork);
     }
     if (batch <= 8 && words >= kSplitLargeWords) return true;

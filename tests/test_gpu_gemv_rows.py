@@ -39,7 +39,7 @@ CASES = [
     (300, 40960, 700, 64, False),     # several k ranges
     (64, 53248, 96, 100, True),
     (130, 33024, 65, 200, False),
-    (132, 1472, 544, 513, True),      # many columns past the rank, zeroed by the blocks of two row tiles
+    (132, 1472, 544, 513, True),      # many columns past the rank, zeroed by the blocks of five feature tiles
     (9804, 256, 384, 579, False),     # outputs of whole 8-byte stores
 ]
 
