@@ -2629,12 +2629,21 @@ constexpr int64_t kS2bMinWordsFewRows = int64_t{1} << 21;
 // 32 rows 9.2 / 13, 15.1 / 12.9, 21.3 / 13, 25.6 / 12.9, 47.2 / 14.4; m = 4096, r = 1632 at 16 / 24 rows 10.9 /
 // 13, 15.5 / 13; m = 8192, r = 2240 at 8 rows 19.2 / 16; m = 28672, r = 3520 at 2 / 4 / 16 / 64 rows 21.4 / 25,
 // 39.6 / 25.4, 149 / 28.8, 588 / 67).
+// On ranks of a few words its second launch is most of a pair's time, and s2t_kernel keeps it below kS2bPairTallWork
+// words of U x batch rows (m = 10240, wr = 3 at 16 rows 5.7 / 6.1; m = 6131, wr = 8 at 35 7.45 / 8.7), and the largest U at
+// two rows (m = 16161, wr = 130 24.7 / 27.2).
+// `alone` false: one of several items that s2t_kernel would serve in one launch, so that a launch of its own has to be paid
+// for, from kS2bGroupWork on (us for two equal items, s2t against s2b: m = 3500, wr = 7 at 47 rows 4.4 / 6.4; m = 7266, wr
+// = 48 at 23 11.4 / 15.8; above 12 M on average 0.8 of the time, above 25 M half).
 constexpr int kS2bPairBatch = 8;
-constexpr int64_t kS2bPairWork = 4400000;
-inline bool s2b_chosen(int batch, int m, const Plan& plan, int items = 1) {
-    if (batch >= kS2bMinBatch && static_cast<int64_t>(m) * batch >= kS2bMinWork) return true;
-    if (items == 2 && batch >= kS2bPairBatch && static_cast<int64_t>(m) * plan.wr * batch >= kS2bPairWork) return true;
-    return static_cast<int64_t>(m) * plan.wr >= kS2bMinWordsFewRows &&
+constexpr int64_t kS2bPairWork = 4400000, kS2bPairTallWork = 2200000, kS2bGroupWork = 12000000;
+inline bool s2b_chosen(int batch, int m, const Plan& plan, int items = 1, bool alone = true) {
+    const int64_t words = static_cast<int64_t>(m) * plan.wr, work = words * batch;
+    if (!alone && work < kS2bGroupWork) return false;
+    if (batch >= kS2bMinBatch && static_cast<int64_t>(m) * batch >= kS2bMinWork && (items == 1 || work >= kS2bPairTallWork))
+        return true;
+    if (items == 2 && batch >= kS2bPairBatch && work >= kS2bPairWork) return true;
+    return words >= kS2bMinWordsFewRows && batch > (items == 2 ? 2 : 1) &&
            ceil_div(batch, s2t_rows_per_pass(batch, items * plan.s2_qw)) >= 2;
 }
 
@@ -3194,7 +3203,7 @@ int group_stage2(const char* name, int dtype, int64_t count, const nq_gemv_item*
             if (split_chosen(b, all[k].m, g.plan[k], pair) && (lead < 0 || all[k].m > all[lead].m)) lead = k;
         for (int64_t k = 0; k < count && lead >= 0; ++k) {
             if (!split_chosen(b, all[k].m, g.plan[k], pair) &&
-                (all[k].wr > kSplitMaxWords || all[k].m > all[lead].m || s2b_chosen(b, all[k].m, g.plan[k], pair)))
+                (all[k].wr > kSplitMaxWords || all[k].m > all[lead].m || s2b_chosen(b, all[k].m, g.plan[k], pair, count == pair)))
                 continue;
             tab.item[tab.count++] = SplitItem{all[k].u_bits, all[k].s_out, all[k].y, all[k].resid, all[k].z_hi, all[k].z_lo,
                                               all[k].m, all[k].wr, all[k].zpitch, all[k].ystride, 0, 0};
@@ -3210,7 +3219,7 @@ int group_stage2(const char* name, int dtype, int64_t count, const nq_gemv_item*
     if (rope == nullptr) {  // items whose batch the batched kernel serves better: a launch each
         const int pair = epilogue == NQ_EPI_GATED ? 2 : 1;
         for (int64_t k = 0; k < count; ++k) {
-            if (done[k] || !s2b_chosen(b, all[k].m, g.plan[k], pair)) continue;
+            if (done[k] || !s2b_chosen(b, all[k].m, g.plan[k], pair, count == pair)) continue;
             S2bCall c{all[k].u_bits, all[k].s_out, all[k].y, all[k].resid, all[k].z_hi, all[k].z_lo, all[k].m,
                       all[k].ystride, b, g.plan[k], st};
             if (pair == 2) {  // the gate into y of item 0, then up against it

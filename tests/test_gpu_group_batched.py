@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 # (m, r, rows, y_stride past the row): whole and ragged row tiles, 8-byte and 2-byte stores, each launch shape
 # (16 or 32 batch rows a block, 32- or 64-row tiles), and the smallest batch of a gated pair
 CASES = [(10240, 64, 16, 0), (5001, 333, 40, 3), (9000, 100, 65, 8), (4102, 200, 90, 2), (20000, 1000, 8, 4),
-         (4100, 1632, 24, 0), (16400, 4224, 2, 0), (1199, 640, 40, 1),
+         (4100, 1632, 24, 0), (16400, 4224, 2, 0), (8200, 1632, 32, 4), (4096, 64, 48, 0), (1199, 640, 40, 1),
          (1200, 640, 40, 0)]
 
 
