@@ -520,12 +520,9 @@ bool rows_stage2_plan(int64_t batch, int64_t m, int64_t wr, RowsPlan& p) {
 
 template <typename T>
 static void launch_stage1_tile(const RowsArgs& a, const RowsPlan& p, hipStream_t st) {
-    switch (p.tile) {
-        case kRows256: return launch_tile<T, T, false, 256, 64, 16, 1>(a, p, st);
-        case kRows128x2: return launch_tile<T, T, false, 128, 64, 8, 2>(a, p, st);
-        case kRows128x4: return launch_tile<T, T, false, 128, 64, 8, 4>(a, p, st);
-        case kRows256q32: return;  // a stage 2 tile
-    }
+    if (p.tile == kRows256) launch_tile<T, T, false, 256, 64, 16, 1>(a, p, st);
+    else if (p.tile == kRows128x2) launch_tile<T, T, false, 128, 64, 8, 2>(a, p, st);
+    else launch_tile<T, T, false, 128, 64, 8, 4>(a, p, st);  // kRows128x4
 }
 
 void launch_rows_stage1(int dtype, const RowsArgs& a, const RowsPlan& p, hipStream_t st) {

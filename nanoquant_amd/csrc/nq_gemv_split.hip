@@ -269,7 +269,11 @@ int launch_epi(const SplitTable& tab, int batch, SplitEpilogue epi, const SplitP
 
 template <typename T, int RT, int CT>
 int launch_waves(const SplitTable& tab, int batch, SplitEpilogue epi, const SplitPlan& p, hipStream_t st) {
-    return p.waves == 4 ? launch_epi<T, RT, CT, 4>(tab, batch, epi, p, st) : launch_epi<T, RT, CT, 8>(tab, batch, epi, p, st);
+    // the shapes of split_plan: four waves on four column tiles, eight on four row tiles by two column tiles
+    if constexpr (CT == 4) return launch_epi<T, RT, CT, 4>(tab, batch, epi, p, st);
+    else if constexpr (RT == 4 && CT == 2) return launch_epi<T, RT, CT, 8>(tab, batch, epi, p, st);
+    else if (p.waves == 4) return launch_epi<T, RT, CT, 4>(tab, batch, epi, p, st);
+    else return launch_epi<T, RT, CT, 8>(tab, batch, epi, p, st);
 }
 
 template <typename T, int RT>

@@ -268,18 +268,11 @@ def step_constants(head_dim: int, dtype, device):
     return eye, rot, values
 
 
-def step_mask(positions, cache: StaticKVCache, values, out=None):
+def step_mask(positions, cache: StaticKVCache, values):
     """The additive causal mask of a one-token step at ``positions`` (one position, on the device):
-    [1, L, 1], values[0] (0) for cache rows up to the position and values[1] (-inf) past it; written
-    into ``out`` (any shape that broadcasts [1, L, 1], e.g. every layer's scores at once) when it
-    is given."""
+    [1, L, 1], values[0] (0) for cache rows up to the position and values[1] (-inf) past it."""
     visible = cache.key_index.view(1, -1, 1) <= positions.view(1, 1, 1)
-    if out is None:
-        return torch.where(visible, values[0], values[1])
-    # the condition takes out's full shape, so that the result is written in place, not resized
-    L = visible.shape[1]
-    visible = visible.view([1] * (out.dim() - 2) + [L, 1]).expand(out.shape)
-    return torch.where(visible, values[0], values[1], out=out)
+    return torch.where(visible, values[0], values[1])
 
 
 def rotary_step_tables(cos, sin, positions, cache: StaticKVCache, dtype, with_mask: bool = True, consts=None):
