@@ -241,11 +241,12 @@ GEMV_CASES = [
     # the batched stage 1 (k split over blocks, then a finishing launch that adds the ranges in
     # order) runs on rows of 256 words or more: from 16 batch rows, from 8 on rows of 320 words or
     # more, from 3 on rows of 512, from 2 on rows of 513-1024 (whose one-row case runs the VALU
-    # kernel with four words per lane over four waves), from 1 on longer rows; a ragged rank and
-    # batch, one k range or several, 1, 2, 5 and 7 batch tiles. Narrower rows (64 words) at 64
+    # kernel with four words per lane over four waves), from 1 on longer rows, up to 48-96 rows by the
+    # size of V, where the kernels of many rows take over (the cases named rows_*); a ragged rank and
+    # batch, one k range or several, 1, 2, 3, 5 and 6 batch tiles. Narrower rows (64 words) at 64
     # and 100 rows, and each threshold's batch just below it, run the MFMA or VALU stage 1.
-    ("sb_b100", 2048, 2048, 512, 100, True),
-    ("sb_b64_r200", 1000, 2048, 200, 64, True),
+    ("s1m_b100", 2048, 2048, 512, 100, True),
+    ("s1m_b64_r200", 1000, 2048, 200, 64, True),
     ("sb_b70_wide", 600, 8192, 500, 70, True),
     ("sb_b20_wide_ragged", 700, 9216, 333, 20, False),
     ("sb_b96_wide", 300, 8192, 1000, 96, False),
@@ -287,10 +288,11 @@ GEMV_CASES = [
     # an even word count (padded) and an odd one (already odd)
     ("s1m_wide_even_b5", 300, 8192, 160, 5, True),
     ("s1m_wide_odd_b5", 300, 8224, 160, 5, True),
-    # 1024-word rows (n = 32737 .. 32768) where the k-split stage 1 does not run (more than 128
-    # batch rows; n % 32 != 0): the MFMA kernel with the unpadded stride (the padded one would not
-    # fit its staging buffer)
-    ("s1m_b130_n32768", 200, 32768, 96, 130, False),
+    # 1024-word rows (n = 32737 .. 32768) where the k-split stage 1 does not run (n % 32 != 0): the
+    # MFMA kernel with the unpadded stride (the padded one would not fit its staging buffer; the case
+    # s1m_b3_n32760 below), up to 32 rows, and the kernels of many rows at 130
+    ("rows_b130_n32768", 200, 32768, 96, 130, False),
+    ("s1m_b32_n32760", 200, 32760, 96, 32, False),
     # one batch row, whole words of up to 384 per row: the stage 1 with s_in and x in LDS, rows in
     # pairs per 64-bit shift, words split over 1-3 waves per row group; ragged ranks (rows past the
     # rank store zeros), s_mid, a rank of 1, each launch shape's width bucket (<= 64, 128, 256, 384)
@@ -300,12 +302,13 @@ GEMV_CASES = [
     ("s1l_b1_n12288_mid", 400, 12288, 130, 1, True),
     ("s1l_b1_n11008_r1", 64, 11008, 1, 1, True),
     ("s1m_b3_n32760", 300, 32760, 130, 3, True),
-    # the batched stage 1 where no plan fits one round of blocks (the x slice of 48+ batch rows
-    # leaves too little LDS for the rows' words): two rounds at 48 and 128 rows, three at 100, with
-    # ragged ranks and batch
-    ("sb_rounds_b48_n28672", 300, 28672, 3000, 48, True),
-    ("sb_rounds_b128_n11008", 500, 11008, 2976, 128, False),
-    ("sb_rounds_b100_n28672", 200, 28672, 2900, 100, True),
+    # the kernels of many rows on the sizes where no plan of the batched stage 1 fits one round of blocks
+    # (the x slice of 48+ batch rows leaves too little LDS for the rows' words), with ragged ranks and batch
+    ("rows_b48_n28672", 300, 28672, 3000, 48, True),
+    ("rows_b128_n11008", 500, 11008, 2976, 128, False),
+    ("rows_b100_n28672", 200, 28672, 2900, 100, True),
+    # ... and the batched stage 1 itself in two rounds of blocks
+    ("sb_rounds_b20_n65536", 64, 65536, 3300, 20, True),
     # the VALU stage 1 that decodes each sign word once for all batch rows: two to four rows on rows of
     # up to 128 words (each launch shape's width bucket), two rows on rows of 257-384 words; ragged
     # ranks and row ends, s_mid, a rank of 1; and the rows next to its bounds, which other kernels take
