@@ -121,8 +121,8 @@ int nq_permute_marlin_scales(const uint16_t* scale_in, uint16_t* scale_in_out, i
  * does on rows of 256 or more words (n >= 8161), n % 32 == 0, from a batch set by the words per row
  * w = n / 32: w > 1024 from 1 row; 513 <= w <= 1024 from 2; w = 512 from 3; 320 <= w <= 511 from 8;
  * 256 <= w <= 319 from 8 when V holds fewer than 256 K words (r * w), else from 16. The kernels of
- * many batch rows, which take over at 33 rows (w >= 512), 64 (256 <= w) or 129, do on grids that leave
- * CUs idle. This function is the authority: size workspaces from it, not from this list. A
+ * many batch rows, which take over at 33 rows (w >= 512), 64 (256 <= w) or 129 but for a small V, do on
+ * grids that leave CUs idle. This function is the authority: size workspaces from it, not from this list. A
  * workspace that holds the header and intermediate but not those sums is accepted and runs the
  * stage-1 kernels that keep none (results agree to rounding, not bit for bit). */
 size_t nq_gemv_workspace_bytes(int64_t batch, int64_t n, int64_t r, int64_t m);
