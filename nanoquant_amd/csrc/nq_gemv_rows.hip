@@ -43,9 +43,12 @@ constexpr int NBUF = 3;
 __device__ inline uint16_t bf16_of(float v) { return __builtin_bit_cast(uint16_t, static_cast<__bf16>(v)); }
 __device__ inline float of_bf16(uint16_t b) { return __uint_as_float(static_cast<uint32_t>(b) << 16); }
 
-template <typename T, typename TO, bool kS2, int BP, int BQ, int CW, int KS>
+// VEC: elements of y per store of stage 2, whose rows are whole pieces of that many (8 or 4; 1 any), apart so that the
+// widest does not pay for the others (m = 11008, r = 1632 at 300 rows 22.4 us, 22.55 with the choice in the kernel; m =
+// 9804, r = 384 at 579 11.5, 12.0).
+template <typename T, typename TO, bool kS2, int BP, int BQ, int CW, int KS, int VEC>
 __global__ __launch_bounds__(BP * KS) __attribute__((amdgpu_waves_per_eu(2)))
-void rows_kernel(const RowsArgs a, int q_tiles, int p_tiles, int split_steps, int splits, int vec) {
+void rows_kernel(const RowsArgs a, int q_tiles, int p_tiles, int split_steps, int splits) {
     constexpr int NX = kS2 ? 2 : 1;  // x, or z_hi and z_lo
     constexpr int NW = BP / 64;  // waves of a k group
     constexpr int NT = NW * 64;
@@ -388,9 +391,9 @@ void rows_kernel(const RowsArgs a, int q_tiles, int p_tiles, int split_steps, in
             const int o = f0 + 8 * (lane & 7);
             if (q < a.batch && o < a.rows) {
                 uint16_t* dst = a.y + static_cast<size_t>(q) * a.rows + o;
-                if (vec == 8) {
+                if constexpr (VEC == 8) {
                     *reinterpret_cast<u32x4*>(dst) = d;
-                } else if (vec == 4) {
+                } else if constexpr (VEC == 4) {
                     *reinterpret_cast<uint2*>(dst) = uint2{d.x, d.y};
                     if (o + 4 < a.rows) *reinterpret_cast<uint2*>(dst + 4) = uint2{d.z, d.w};
                 } else {
@@ -404,15 +407,12 @@ void rows_kernel(const RowsArgs a, int q_tiles, int p_tiles, int split_steps, in
     }
 }
 
-template <typename T, typename TO, bool kS2, int BP, int BQ, int CW, int KS>
+template <typename T, typename TO, bool kS2, int BP, int BQ, int CW, int KS, int VEC>
 void launch_tile(const RowsArgs& a, const RowsPlan& p, hipStream_t st) {
     const int q_tiles = static_cast<int>(ceil_div(a.batch, BQ));
     const int p_tiles = static_cast<int>(ceil_div(a.rows, BP));
-    // elements of y per store: its rows whole 16- or 8-byte pieces (m = 9804, r = 384 at 579 rows 12.2
-    // us, 21.8 in 2-byte stores)
-    const int vec = !kS2 ? 0 : a.rows % 8 == 0 && aligned(a.y, 16) ? 8 : a.rows % 4 == 0 && aligned(a.y, 8) ? 4 : 0;
-    rows_kernel<T, TO, kS2, BP, BQ, CW, KS><<<dim3(static_cast<unsigned>(q_tiles * p_tiles * p.splits)), BP * KS, 0, st>>>(
-        a, q_tiles, p_tiles, p.split_steps, p.splits, vec);
+    rows_kernel<T, TO, kS2, BP, BQ, CW, KS, VEC><<<dim3(static_cast<unsigned>(q_tiles * p_tiles * p.splits)), BP * KS, 0, st>>>(
+        a, q_tiles, p_tiles, p.split_steps, p.splits);
 }
 
 // Stage 1 runs these kernels on rows of 512 words or more from 33 batch rows, of 256-511 words from 64,
@@ -520,9 +520,9 @@ bool rows_stage2_plan(int64_t batch, int64_t m, int64_t wr, RowsPlan& p) {
 
 template <typename T>
 static void launch_stage1_tile(const RowsArgs& a, const RowsPlan& p, hipStream_t st) {
-    if (p.tile == kRows256) launch_tile<T, T, false, 256, 64, 16, 1>(a, p, st);
-    else if (p.tile == kRows128x2) launch_tile<T, T, false, 128, 64, 8, 2>(a, p, st);
-    else launch_tile<T, T, false, 128, 64, 8, 4>(a, p, st);  // kRows128x4
+    if (p.tile == kRows256) launch_tile<T, T, false, 256, 64, 16, 1, 8>(a, p, st);
+    else if (p.tile == kRows128x2) launch_tile<T, T, false, 128, 64, 8, 2, 8>(a, p, st);
+    else launch_tile<T, T, false, 128, 64, 8, 4, 8>(a, p, st);  // kRows128x4
 }
 
 void launch_rows_stage1(int dtype, const RowsArgs& a, const RowsPlan& p, hipStream_t st) {
@@ -530,10 +530,18 @@ void launch_rows_stage1(int dtype, const RowsArgs& a, const RowsPlan& p, hipStre
     else launch_stage1_tile<BF16>(a, p, st);
 }
 
+template <typename TO, int VEC>
+static void launch_stage2_vec(const RowsArgs& a, const RowsPlan& p, hipStream_t st) {
+    if (p.tile == kRows256q32) launch_tile<BF16, TO, true, 256, 32, 8, 1, VEC>(a, p, st);
+    else launch_tile<BF16, TO, true, 256, 64, 8, 1, VEC>(a, p, st);
+}
+
+// 8-byte stores: m = 9804, r = 384 at 579 rows 11.5 us, 21.0 in 2-byte ones.
 template <typename TO>
 static void launch_stage2_tile(const RowsArgs& a, const RowsPlan& p, hipStream_t st) {
-    if (p.tile == kRows256q32) launch_tile<BF16, TO, true, 256, 32, 8, 1>(a, p, st);
-    else launch_tile<BF16, TO, true, 256, 64, 8, 1>(a, p, st);
+    if (a.rows % 8 == 0 && aligned(a.y, 16)) launch_stage2_vec<TO, 8>(a, p, st);
+    else if (a.rows % 4 == 0 && aligned(a.y, 8)) launch_stage2_vec<TO, 4>(a, p, st);
+    else launch_stage2_vec<TO, 1>(a, p, st);
 }
 
 void launch_rows_stage2(int dtype, const RowsArgs& a, const RowsPlan& p, hipStream_t st) {
