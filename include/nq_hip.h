@@ -332,6 +332,16 @@ int nq_attention_prefill(int dtype, const void* q, int64_t q_stride, const void*
                          const int64_t* positions, void* out, int64_t batch, int64_t tokens, int64_t heads,
                          int64_t kv_heads, int64_t head_dim, int64_t max_len, float scaling, nq_stream_t stream);
 
+/* nq_attention_prefill with device memory (16-byte aligned) of nq_attention_prefill_workspace_bytes, with which a few tokens
+ * on a long cache share their keys over the grid (0 bytes where they do not; NULL or less memory runs as above). */
+size_t nq_attention_prefill_workspace_bytes(int64_t batch, int64_t tokens, int64_t heads, int64_t kv_heads, int64_t head_dim,
+                                            int64_t max_len);
+int nq_attention_prefill_ws(int dtype, const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
+                            int64_t v_stride, void* k_cache, void* v_cache, const void* rope_cos, const void* rope_sin,
+                            const int64_t* positions, void* out, int64_t batch, int64_t tokens, int64_t heads,
+                            int64_t kv_heads, int64_t head_dim, int64_t max_len, float scaling, void* workspace,
+                            size_t workspace_bytes, nq_stream_t stream);
+
 /* Rotary embedding and KV-cache write of one new token per sequence, with the attention products
  * left to the caller: the first part of nq_attention_decode on its own. qkv [batch, qkv_stride]
  * holds heads query heads, kv_heads key heads and kv_heads value heads of head_dim (even) each;

@@ -83,6 +83,9 @@ SIGNATURES = {
                                    _i64, ctypes.c_float, _vp, _size, _vp]),
     "nq_attention_prefill": (_int, [_int, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64,
                                     _i64, _i64, _i64, _i64, ctypes.c_float, _vp]),
+    "nq_attention_prefill_workspace_bytes": (_size, [_i64, _i64, _i64, _i64, _i64, _i64]),
+    "nq_attention_prefill_ws": (_int, [_int, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64,
+                                       _i64, _i64, _i64, _i64, ctypes.c_float, _vp, _size, _vp]),
     "nq_rope_kv_write": (_int, [_int, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64,
                                  _vp]),
     "nq_rms_norm": (_int, [_int, _vp, _vp, _vp, _i64, _i64, ctypes.c_float, _vp]),

@@ -14,6 +14,7 @@
 //    exchange with lane ^ 32, and P^T's accumulator layout is already a B operand: lane group kg holds
 //    keys 4 kg .. +3 and 8 + 4 kg .. +3 of each 16, the key order in which V^T is laid out in LDS. Scores
 //    and sums stay in fp32 (the torch path rounds the scores to T).
+// 3. A few tokens on a long cache share their keys over the grid in 2, and attn_join_kernel adds the shares.
 //
 // The scores never reach memory: at 2048 tokens and 32 heads the torch path writes and reads them (256 MB
 // in T, 512 MB in fp32) eight times over. What bounds this kernel is issue: per tile and wave 32 MFMAs
@@ -34,6 +35,7 @@ constexpr int D = 128;
 constexpr int kRowsPerBlock = 128;
 constexpr int kKeys = 64;
 constexpr float kSlack = 8.0f;
+constexpr int kWholeTiles = 6;  // up to so many key tiles are not shared: the sums' way costs as much
 
 struct AttnArgs {
     const uint16_t* q;
@@ -48,6 +50,9 @@ struct AttnArgs {
     uint16_t* out;  // [batch][tokens][heads * 128]
     int batch, tokens, kv_heads, groups, max_len;
     float scale;  // times log2(e)
+    float* part_o;  // [splits][batch * kv_heads * tokens * groups][128], where the keys are split
+    float* part_ml;  // the same rows' {maximum, sum}
+    int splits;
 };
 
 // Eight elements of a head and their rotary partners (d and d + 64): T(T(x cos) + T(rotate_half(x) sin)).
@@ -120,9 +125,10 @@ __device__ inline uint32_t pack2(float a, float b) {
     return static_cast<uint32_t>(T::from_float(a)) | (static_cast<uint32_t>(T::from_float(b)) << 16);
 }
 
-template <typename T, int KS>
+// kPart: a block takes one of a.splits shares of its rows' key tiles and leaves sums for attn_join_kernel.
+template <typename T, int KS, bool kPart>
 __global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(2))) void prefill_attn_kernel(const AttnArgs a) {
-    static_assert(KS == 1 || KS == 2, "one or two groups of waves");
+    static_assert(KS == 1 || (KS == 2 && !kPart), "one or two groups of waves");
     __shared__ __attribute__((aligned(16))) uint16_t ksall[KS][2][kKeys * D];
     __shared__ __attribute__((aligned(16))) uint16_t vtall[KS][2][D * kKeys];
     __shared__ int lims[4];
@@ -138,7 +144,7 @@ __global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(2))) v
     // Row tiles in order of falling length, the longest blocks first. A grid that is resident at once (two
     // blocks a CU) has no later blocks to fill in behind the short ones: its second half goes the other
     // way round, so that a CU gets a long block and a short one.
-    const int n_tiles = static_cast<int>(gridDim.x) / heads;
+    const int n_tiles = static_cast<int>(gridDim.x) / heads;  // (blockIdx.y: the share of the keys)
     const int order = static_cast<int>(blockIdx.x) / heads;
     const int tile = KS == 1 && gridDim.x <= 512u && 2 * order >= n_tiles ? order - (n_tiles + 1) / 2 : n_tiles - 1 - order;
     const int bh = static_cast<int>(blockIdx.x) % heads;
@@ -186,7 +192,16 @@ __global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(2))) v
     if (grp == 0 && lane == 0) lims[wave] = wmax;
     __syncthreads();
     const int last = __builtin_amdgcn_readfirstlane(max(max(lims[0], lims[1]), max(lims[2], lims[3])));
-    const int tiles = last / kKeys + 1;  // one (all masked) where every position is below 0
+    int tiles = last / kKeys + 1;  // one (all masked) where every position is below 0
+    int it0 = 0;
+    bool whole = !kPart;  // this block takes all of its rows' keys
+    if (kPart) {
+        whole = tiles <= kWholeTiles;
+        if (whole && blockIdx.y > 0) return;
+        const int share = whole ? tiles : (tiles + a.splits - 1) / a.splits;
+        it0 = min(static_cast<int>(blockIdx.y) * share, tiles);
+        tiles = min(share, tiles - it0);  // none in some last shares
+    }
 
     const size_t head = static_cast<size_t>(bh) * a.max_len * D;
     const uint16_t* kbase = a.k_cache + head;
@@ -236,13 +251,15 @@ __global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(2))) v
     // group g takes tiles g, g + KS, ...; all groups run the rounds of the longest (the barriers are the
     // block's), a tile past the last one being loaded (keys clamped, values zero) and not computed
     const int rounds = (tiles + KS - 1) / KS;
-    load_v(grp);
-    issue_k(grp, 0);
-    wait_vmcnt<0>();
-    store_v(0);
+    if (!kPart || rounds > 0) {
+        load_v(it0 + grp);
+        issue_k(it0 + grp, 0);
+        wait_vmcnt<0>();
+        store_v(0);
+    }
     barrier_keep_dma();
     for (int round = 0; round < rounds; ++round) {
-        const int it = round * KS + grp;
+        const int it = it0 + round * KS + grp;
         const int buf = round & 1;
         const bool more = round + 1 < rounds;
         if (more) {
@@ -367,6 +384,22 @@ __global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(2))) v
             for (int i = 0; i < 16; ++i) o[dt][i] = o[dt][i] * a0 + red[(16 * dt + i) * 256 + t] * a1;
     }
     l += __shfl_xor(l, 32, 64);
+    if constexpr (kPart) {  // the sums as they are, 16 bytes a lane
+        if (R0 + c < rows) {
+            const size_t row = (static_cast<size_t>(blockIdx.y) * heads + bh) * static_cast<size_t>(rows) + (R0 + c);
+            // a sum of -1: the row is done
+            if (kg == 0) *reinterpret_cast<float2*>(a.part_ml + 2 * row) = whole ? float2{0.0f, -1.0f} : float2{m, l};
+            if (tiles > 0 && !whole) {
+#pragma unroll
+                for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+                    for (int g4 = 0; g4 < 4; ++g4)
+                        *reinterpret_cast<f32x4*>(a.part_o + row * D + 32 * dt + 8 * g4 + 4 * kg) =
+                            f32x4{o[dt][4 * g4], o[dt][4 * g4 + 1], o[dt][4 * g4 + 2], o[dt][4 * g4 + 3]};
+            }
+        }
+        if (!whole) return;
+    }
     const float inv = 1.0f / l;
 
     // the wave's rows through LDS (its 8 KB of the V buffers, 16-byte chunk ch of row r at ch ^ (r % 16)),
@@ -392,6 +425,54 @@ __global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(2))) v
     }
 }
 
+// out = T(sum_s o_s 2^(m_s - M) / sum_s l_s 2^(m_s - M)), M the largest m_s: 32 threads a row, four dimensions each.
+// Bound by latency: eight shares' sums are loaded together. A share without keys has m = -inf and l = 0, and no o.
+template <typename T>
+__global__ __launch_bounds__(256) void attn_join_kernel(const AttnArgs a) {
+    const int rows = a.tokens * a.groups;
+    const int64_t total = static_cast<int64_t>(a.batch) * a.kv_heads * rows;
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * 8 + (threadIdx.x >> 5);
+    const int d = 4 * static_cast<int>(threadIdx.x & 31);
+    if (row >= total) return;
+    if (a.part_ml[2 * row + 1] == -1.0f) return;  // (of share 0)
+    float M = -__builtin_huge_valf(), L = 0.0f;
+    f32x4 O = f32x4{0.f, 0.f, 0.f, 0.f};
+    constexpr int kAhead = 8;
+    for (int s0 = 0; s0 < a.splits; s0 += kAhead) {
+        float2 ml[kAhead];
+        f32x4 o[kAhead];
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+            const int64_t at = min(s0 + i, a.splits - 1) * total + row;
+            ml[i] = *reinterpret_cast<const float2*>(a.part_ml + 2 * at);
+            o[i] = *reinterpret_cast<const f32x4*>(a.part_o + at * D + d);
+        }
+        float bm = M;
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) bm = fmaxf(bm, ml[i].x);  // a share taken twice changes nothing here
+        const float mu = bm == -__builtin_huge_valf() ? 0.0f : bm;
+        const float keep = __builtin_amdgcn_exp2f(M - mu);
+        L *= keep;
+        O = f32x4{O.x * keep, O.y * keep, O.z * keep, O.w * keep};
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+            const bool none = s0 + i >= a.splits || (ml[i].x == -__builtin_huge_valf() && ml[i].y == 0.0f);
+            const float f = __builtin_amdgcn_exp2f(ml[i].x - mu);
+            L = none ? L : fmaf(ml[i].y, f, L);
+            O = none ? O : f32x4{fmaf(o[i].x, f, O.x), fmaf(o[i].y, f, O.y), fmaf(o[i].z, f, O.z), fmaf(o[i].w, f, O.w)};
+        }
+        M = bm;
+    }
+    const float inv = 1.0f / L;
+    const int64_t bh = row / rows;
+    const int R = static_cast<int>(row - bh * rows);
+    const int64_t b = bh / a.kv_heads;
+    const int kvh = static_cast<int>(bh - b * a.kv_heads);
+    const int tok = R / a.groups;
+    const size_t at = ((static_cast<size_t>(b) * a.tokens + tok) * (a.kv_heads * a.groups) + kvh * a.groups + (R - tok * a.groups)) * D;
+    *reinterpret_cast<uint2*>(a.out + at + d) = uint2{pack2<T>(O.x * inv, O.y * inv), pack2<T>(O.z * inv, O.w * inv)};
+}
+
 // Two groups of waves share a block's keys where the grid leaves a CU one block at most and its longest block
 // walks over twelve tiles or more (the host does not know the positions, only that the last token sees at
 // least the others): both launches, fp16, us, one group / two: 32 heads at 1000 tokens 43.1 / 40.4, 16 at 2000
@@ -401,16 +482,35 @@ __global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(2))) v
 // grouped heads 20.2 / 27.3).
 constexpr int64_t kSplitBlocks = 256, kSplitTokens = 768;
 
+// A few tokens on a long context are a few blocks with a long walk each, 1.2 us a tile, where the torch ops, slower
+// otherwise, have the whole chip: their keys are shared over the grid, up to two blocks a CU, from caches of 4096 positions
+// on (the host does not know how much of one is filled) and at least 512 positions a share. All launches, us, torch
+// ops, whole, shared: 4 tokens of 8 heads over 2 after 29625 178, 567, 36; 2 tokens of 32 heads after 19239 236, 380, 66.
+// A short context pays the join's launch: 2 to 64 tokens alone in such a cache 13-14 whole, 15 shared, torch ops 100-500.
+// More tokens were never slower than the torch ops, and keep one launch.
+constexpr int64_t kPartTokens = 64, kPartBlocks = 512, kPartKeys = 4096, kPartShare = 512, kPartMax = 32;
+int prefill_splits(int64_t batch, int64_t tokens, int64_t kv_heads, int64_t groups, int64_t max_len) {
+    const int64_t blocks = ceil_div(tokens * groups, kRowsPerBlock) * batch * kv_heads;
+    if (blocks <= 0 || tokens > kPartTokens || max_len < kPartKeys) return 1;
+    return static_cast<int>(std::max<int64_t>(1, std::min({kPartBlocks / blocks, max_len / kPartShare, kPartMax})));
+}
+
 template <typename T>
 void launch_prefill(const AttnArgs& a, hipStream_t st) {
     const int64_t kv_threads = static_cast<int64_t>(a.batch) * a.tokens * a.kv_heads * 16;
     kv_rows_kernel<T><<<dim3(static_cast<unsigned>(ceil_div(kv_threads, 256))), 256, 0, st>>>(a);
     const int64_t tiles = ceil_div(static_cast<int64_t>(a.tokens) * a.groups, kRowsPerBlock);
     const int64_t blocks = tiles * a.batch * a.kv_heads;
-    if (blocks <= kSplitBlocks && a.tokens >= kSplitTokens)
-        prefill_attn_kernel<T, 2><<<dim3(static_cast<unsigned>(blocks)), 512, 0, st>>>(a);
-    else
-        prefill_attn_kernel<T, 1><<<dim3(static_cast<unsigned>(blocks)), 256, 0, st>>>(a);
+    if (a.splits > 1) {
+        prefill_attn_kernel<T, 1, true>
+            <<<dim3(static_cast<unsigned>(blocks), static_cast<unsigned>(a.splits)), 256, 0, st>>>(a);
+        const int64_t rows = static_cast<int64_t>(a.batch) * a.kv_heads * a.tokens * a.groups;
+        attn_join_kernel<T><<<dim3(static_cast<unsigned>(ceil_div(rows, 8))), 256, 0, st>>>(a);
+    } else if (blocks <= kSplitBlocks && a.tokens >= kSplitTokens) {
+        prefill_attn_kernel<T, 2, false><<<dim3(static_cast<unsigned>(blocks)), 512, 0, st>>>(a);
+    } else {
+        prefill_attn_kernel<T, 1, false><<<dim3(static_cast<unsigned>(blocks)), 256, 0, st>>>(a);
+    }
 }
 
 }  // namespace
@@ -420,10 +520,28 @@ using namespace nq;
 
 extern "C" {
 
+size_t nq_attention_prefill_workspace_bytes(int64_t batch, int64_t tokens, int64_t heads, int64_t kv_heads, int64_t head_dim,
+                                            int64_t max_len) {
+    if (batch <= 0 || tokens <= 0 || heads <= 0 || kv_heads <= 0 || head_dim != D || heads % kv_heads || tokens > kPartTokens ||
+        batch > INT32_MAX || heads > INT32_MAX || max_len > (int64_t{1} << 22))
+        return 0;
+    const int splits = prefill_splits(batch, tokens, kv_heads, heads / kv_heads, max_len);
+    return splits > 1 ? static_cast<size_t>(splits) * batch * tokens * heads * (D + 2) * sizeof(float) : 0;
+}
+
 int nq_attention_prefill(int dtype, const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
                          int64_t v_stride, void* k_cache, void* v_cache, const void* rope_cos, const void* rope_sin,
                          const int64_t* positions, void* out, int64_t batch, int64_t tokens, int64_t heads,
                          int64_t kv_heads, int64_t head_dim, int64_t max_len, float scaling, nq_stream_t stream) {
+    return nq_attention_prefill_ws(dtype, q, q_stride, k, k_stride, v, v_stride, k_cache, v_cache, rope_cos, rope_sin, positions,
+                                   out, batch, tokens, heads, kv_heads, head_dim, max_len, scaling, nullptr, 0, stream);
+}
+
+int nq_attention_prefill_ws(int dtype, const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
+                            int64_t v_stride, void* k_cache, void* v_cache, const void* rope_cos, const void* rope_sin,
+                            const int64_t* positions, void* out, int64_t batch, int64_t tokens, int64_t heads,
+                            int64_t kv_heads, int64_t head_dim, int64_t max_len, float scaling, void* workspace,
+                            size_t workspace_bytes, nq_stream_t stream) {
     const char* name = "nq_attention_prefill";
     if (dtype != NQ_F16 && dtype != NQ_BF16) return fail(NQ_ERR_DTYPE, "%s: unsupported dtype %d", name, dtype);
     if (batch < 0 || tokens < 0 || heads <= 0 || kv_heads <= 0 || max_len <= 0)
@@ -444,7 +562,8 @@ int nq_attention_prefill(int dtype, const void* q, int64_t q_stride, const void*
                           rope_sin, static_cast<const void*>(out)})
         if (!aligned(p, 16)) return fail(NQ_ERR_ALIGNMENT, "%s: tensors must be 16-byte aligned", name);
     if (!aligned(positions, 8)) return fail(NQ_ERR_ALIGNMENT, "%s: positions must be 8-byte aligned", name);
-    AttnArgs a;
+    if (!aligned(workspace, 16)) return fail(NQ_ERR_ALIGNMENT, "%s: workspace must be 16-byte aligned", name);
+    AttnArgs a{};
     a.q = static_cast<const uint16_t*>(q);
     a.k = static_cast<const uint16_t*>(k);
     a.v = static_cast<const uint16_t*>(v);
@@ -463,6 +582,13 @@ int nq_attention_prefill(int dtype, const void* q, int64_t q_stride, const void*
     a.groups = static_cast<int>(heads / kv_heads);
     a.max_len = static_cast<int>(max_len);
     a.scale = scaling * 1.44269504088896340736f;  // exp(x) = exp2(x log2(e))
+    const size_t need = nq_attention_prefill_workspace_bytes(batch, tokens, heads, kv_heads, head_dim, max_len);
+    a.splits = 1;
+    if (workspace && need > 0 && workspace_bytes >= need) {
+        a.splits = prefill_splits(batch, tokens, kv_heads, a.groups, max_len);
+        a.part_o = static_cast<float*>(workspace);
+        a.part_ml = a.part_o + static_cast<size_t>(a.splits) * batch * tokens * heads * D;
+    }
     if (dtype == NQ_F16) launch_prefill<F16>(a, as_stream(stream));
     else launch_prefill<BF16>(a, as_stream(stream));
     return check_launch(name);

@@ -226,11 +226,14 @@ def rotary_attention(shape: LlamaShape, layer: int, q, k, v, cos, sin, positions
         out = torch.empty_like(q, memory_format=torch.contiguous_format)
         lib = _lib.load()
         with torch.cuda.device(q.device):
-            _lib.check(lib.nq_attention_prefill(
+            L = cache.k[layer].shape[2]
+            nbytes = lib.nq_attention_prefill_workspace_bytes(q.shape[0], q.shape[1], H, KV, D, L)
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
+            _lib.check(lib.nq_attention_prefill_ws(
                 _lib.dtype_code(q.dtype), q.data_ptr(), q.stride(1), k.data_ptr(), k.stride(1), v.data_ptr(), v.stride(1),
                 cache.k[layer].data_ptr(), cache.v[layer].data_ptr(), cos.data_ptr(), sin.data_ptr(),
-                positions.data_ptr(), out.data_ptr(), q.shape[0], q.shape[1], H, KV, D, cache.k[layer].shape[2],
-                D ** -0.5, _lib.stream_of(q.device)), "rotary_attention")
+                positions.data_ptr(), out.data_ptr(), q.shape[0], q.shape[1], H, KV, D, L, D ** -0.5, _lib.ptr(ws), nbytes,
+                _lib.stream_of(q.device)), "rotary_attention")
         return out
     B, T = q.shape[0], q.shape[1]
     G = H // KV

@@ -160,3 +160,80 @@ def test_prefill_attention_argument_errors():
     assert call(stride=504) == _lib.NQ_ERR_SHAPE
     assert call(p=None) == _lib.NQ_ERR_INVALID_ARGUMENT
     assert call(p=24) == _lib.NQ_ERR_ALIGNMENT
+
+
+# (heads, kv_heads, batch, tokens, past, gap): the shortest cache that is split, one tile a share and a short last one, a
+# context of two tiles in a long cache (not shared), of six and seven tiles, a share that ends inside the tokens' own keys,
+# groups, a second block of one row beside a full one, the last count of tokens, prompts
+LONG_CASES = [(2, 2, 1, 2, 4094, 0), (2, 1, 2, 33, 5000, 99), (4, 4, 1, 2, 70, 5000), (4, 4, 1, 2, 382, 5000), (4, 4, 1, 2, 383, 5000),
+              (4, 2, 1, 64, 4031, 1), (8, 1, 1, 5, 9001, 1), (43, 1, 1, 3, 5000, 0), (3, 3, 1, 64, 0, 5000), (6, 2, 1, 50, 350, 4000),
+              (16, 16, 2, 2, 4500, 0)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("case", LONG_CASES, ids=lambda c: "x".join(map(str, c)))
+def test_prefill_attention_long_caches(case, dtype, torch_ops):
+    """Keys shared over the grid: the same bars as above, the same value again and in a graph's replays."""
+    from nanoquant_amd import _lib
+    print("\n[case] prefill attention, long", case, dtype, flush=True)
+    heads, kv, batch, tokens, past, gap = case
+    shape, q, k, v, cos, sin, pos, cache = args = _inputs(case[:5], dtype, gap)
+    assert _lib.load().nq_attention_prefill_workspace_bytes(batch, tokens, heads, kv, 128, past + tokens + gap) > 0
+    ref = _exact(*args)
+    run = lambda: rotary_attention(shape, 0, q, k, v, cos, sin, pos, cache)  # noqa: E731
+    y = run()
+    want = torch_ops(shape, 0, q, k, v, cos, sin, pos, cache)
+    assert y.shape == want.shape and y.dtype == want.dtype and y.is_contiguous()
+    assert _error(y, ref) <= 1.1 * _error(want, ref)
+    assert torch.equal(run(), y)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        replayed = run()
+    for _ in range(3):
+        replayed.zero_()
+        graph.replay()
+        assert torch.equal(run(), y)
+        torch.cuda.synchronize()
+        assert torch.equal(replayed, y)
+
+
+def test_prefill_attention_long_cache_edges():
+    """With and without the shares: positions below 0 (NaN rows, no cache row), keys of NaN and infinity in one share, NaN
+    past the last position, and a workspace that is too small."""
+    from nanoquant_amd import _lib
+    lib = _lib.load()
+    shape, q, k, v, cos, sin, pos, cache = _inputs((4, 2, 1, 40, 4200), torch.float16, 60)
+    L = cache.k[0].shape[2]
+    need = lib.nq_attention_prefill_workspace_bytes(1, 40, 4, 2, 128, L)
+    assert need > 0 and need % 16 == 0
+
+    def call(nbytes):
+        out = torch.empty_like(q)
+        ws = torch.randint(0, 256, (max(nbytes, 16),), dtype=torch.uint8, device="cuda")
+        _lib.check(lib.nq_attention_prefill_ws(
+            _lib.NQ_F16, q.data_ptr(), 512, k.data_ptr(), 256, v.data_ptr(), 256, cache.k[0].data_ptr(), cache.v[0].data_ptr(),
+            cos.data_ptr(), sin.data_ptr(), pos.data_ptr(), out.data_ptr(), 1, 40, 4, 2, 128, L, 0.088, ws.data_ptr(), nbytes,
+            _lib.stream_of(q.device)), "prefill")
+        return out
+
+    def close(a, b):  # rounded once to float16, sums of another order: one unit of the row's largest value
+        assert torch.equal(a.isnan(), b.isnan())
+        torch.testing.assert_close(a, b, rtol=2e-3, atol=2e-4, equal_nan=True)
+
+    cache.k[0][:, :, 4240:] = float("nan")
+    cache.v[0][:, :, 4240:] = float("nan")
+    plain = call(0)
+    assert not plain.isnan().any() and torch.equal(call(need - 16), plain)
+    close(call(need), plain)
+    pos[3:5] = -1
+    close(call(need), call(0))
+    cache.k[0][0, 1, 700] = float("nan")
+    close(call(need), call(0))
+    cache.k[0][0, 1, 700] = 0
+    cache.v[0][0, 0, 2000, 5] = float("inf")
+    close(call(need), call(0))
+    pos.fill_(-1)
+    assert call(need).isnan().all()
+    assert lib.nq_attention_prefill_workspace_bytes(1, 65, 4, 2, 128, L) == 0
+    assert lib.nq_attention_prefill_workspace_bytes(1, 40, 4, 2, 128, 4095) == 0
