@@ -174,6 +174,13 @@ def test_rows_time_does_not_jump_with_the_sizes_beside(lib):
     assert b < 1.25 * a, (a, b)
 
 
+def test_rows_leave_one_round_to_the_mfma_kernel(lib):
+    """n = 4224 at 129 rows, one round of blocks of 64 features, takes about the time of 128 (it took 1.35 times that)."""
+    print("\n[case] gemv rows, one round", flush=True)
+    a, b = (_stage_us(lib, 1, rows, 4224, 1536, 64) for rows in (128, 129))
+    assert b < 1.2 * a, (a, b)
+
+
 @pytest.mark.parametrize("offset", [1, 4])
 def test_rows_without_range_sums_and_unaligned_output(lib, offset):
     """No room for the k ranges' sums (one range runs), and outputs off their 16-byte alignment."""

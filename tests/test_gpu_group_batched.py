@@ -88,3 +88,40 @@ def test_batched_epilogues(case, dtype):
     gate["y"].fill_(7.0)
     _group(lib, [gate, up], x, _lib.NQ_EPI_GATED, dtype)
     close(gate["y"], torch.nn.functional.silu(single[0].float()).to(dtype) * single[1], 4)
+
+
+def test_small_items_share_a_launch():
+    """Two stored items of a small rank take less than two launches of one (they took as much)."""
+    from nanoquant_amd import _lib
+    lib = _lib.load()
+    m, r, batch, dtype = 3500, 224, 47, torch.float16
+    print("\n[case] group batched, small items", flush=True)
+    entries = [_entry(i, m, 64, r, dtype, 0, batch) for i in (1, 2)]
+    arr = (_lib.GemvItem * 2)()
+    for it, e in zip(arr, entries):
+        it.v_bits, it.s_in, it.s_mid, it.u_bits, it.s_out = (e[k].data_ptr() for k in ("V", "s_in", "s_mid", "U", "s_out"))
+        it.y, it.y_stride, it.r, it.m = e["y"].data_ptr(), m, r, m
+    ws = torch.zeros(lib.nq_gemv_group_workspace_bytes(2, arr, batch), dtype=torch.uint8, device="cuda")
+
+    def us(count):
+        def launch():
+            _lib.check(lib.nq_gemv_group_stage2(_lib.NQ_F16, count, arr, batch, _lib.NQ_EPI_STORE, ws.data_ptr(), ws.numel(),
+                                                torch.cuda.current_stream().cuda_stream), "stage 2")
+        launch()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(16):
+                launch()
+        times = []
+        for _ in range(6):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            graph.replay()
+            end.record()
+            torch.cuda.synchronize()
+            times.append(start.elapsed_time(end) * 1000 / 16)
+        return min(times[1:])
+
+    one, two = us(1), us(2)
+    assert two < 1.7 * one, (one, two)
